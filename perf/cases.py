@@ -1,0 +1,562 @@
+"""The work this library is used for, as cases that can be timed and checked.
+
+Every case goes through the public Python entry points (Solver, Batch, Server,
+SceneImage) the way a program that uses them does, from the scene in hand to
+the state it reads back:
+
+  frames   a Solver stepped and read back each frame (an interactive program)
+  cloth    a Solver holding one cloth, advanced some updates between readings
+  gas      a clone of a saved world of free circles, rolled out and read
+  image    a soft body dropped on the floor, rolled out from a stored scene
+           image in device memory the caller owns (an environment's reset)
+  batch    many soft bodies of mixed size in flight, advanced together
+  pile     a Batch made of many small piles in contact, rolled out and read
+  served   soft bodies resident in a Server, advanced by requests
+
+Scenes are drawn from the seed with numpy alone and handed over through the
+bulk adders; exact() steps the same scenes in 64-bit arithmetic with torch and
+plain Python.
+"""
+import math
+
+import numpy as np
+import torch
+
+from bendy2d_amd import Batch, SceneImage, Server, Solver
+
+DT = 1.0 / 60.0
+HUGE = ((-1.0e5, -1.0e5), (2.0e5, 2.0e5))
+
+
+def listed():
+    return [
+        # the smallest call: a handful of soft polygons with the solver's
+        # default gravity, bounds and substep, read every frame
+        {"name": "frame polygons", "kind": "frames", "scene": "polygons", "count": 5, "points": 12},
+        # the pinned 32x32 cloth over a static circle, read every frame
+        {"name": "frame cloth 32", "kind": "frames", "scene": "cloth", "nx": 32, "ny": 32, "sub_steps": 8,
+         "link_iters": 8, "colliders": 1},
+        # a ragged cloth over several colliders, some frames between readings
+        {"name": "cloth 211x317", "kind": "cloth", "nx": 211, "ny": 317, "sub_steps": 3, "link_iters": 5,
+         "colliders": 6, "updates": 20, "readback": True},
+        # the throughput-scale cloth
+        {"name": "cloth 1024", "kind": "cloth", "nx": 1024, "ny": 1024, "sub_steps": 4, "link_iters": 8,
+         "colliders": 0, "updates": 20, "readback": False},
+        # worlds of free circles in a walled box: past one workgroup's size,
+        # and the full-size box
+        {"name": "gas 20011", "kind": "gas", "n": 20011, "updates": 8},
+        {"name": "gas 262144", "kind": "gas", "n": 262144, "updates": 8},
+        # one soft body from flight into a pile: an ordinary one and a large one
+        {"name": "drop 31x31", "kind": "image", "side": 31, "updates": 24},
+        {"name": "drop 100x100", "kind": "image", "side": 100, "updates": 24},
+        # mixed soft bodies in flight: a few, and enough to fill the device
+        {"name": "batch 48", "kind": "batch", "scenes": 48, "max_side": 40, "updates": 32},
+        {"name": "batch 640", "kind": "batch", "scenes": 640, "max_side": 128, "updates": 64},
+        # many piles in dense contact
+        {"name": "piles 96", "kind": "pile", "scenes": 96, "max_n": 2000, "updates": 8},
+        # scenes resident in a server, each asked for some updates
+        {"name": "served 64", "kind": "served", "scenes": 64, "max_side": 48, "updates": 16},
+    ]
+
+
+def draw(rng):
+    def log(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    kind = rng.choice(("frames", "frames", "cloth", "gas", "image", "batch", "pile", "served"))
+    if kind == "frames" and rng.random() < 0.5:
+        return {"kind": kind, "scene": "polygons", "count": rng.randint(3, 8), "points": rng.randint(6, 20)}
+    if kind == "frames":
+        return {"kind": kind, "scene": "cloth", "nx": log(8, 120), "ny": log(8, 120), "sub_steps": rng.randint(1, 8),
+                "link_iters": rng.randint(1, 8), "colliders": rng.randint(0, 4)}
+    if kind == "cloth":
+        return {"kind": kind, "nx": log(140, 800), "ny": log(140, 800), "sub_steps": rng.randint(1, 4),
+                "link_iters": rng.randint(1, 8), "colliders": rng.randint(0, 8), "updates": rng.randint(10, 20),
+                "readback": rng.random() < 0.5}
+    if kind == "gas":
+        return {"kind": kind, "n": log(2000, 200000), "updates": rng.randint(4, 8)}
+    if kind == "image":
+        return {"kind": kind, "side": log(12, 100), "updates": rng.randint(12, 24)}
+    if kind == "pile":
+        return {"kind": kind, "scenes": log(24, 96), "max_n": log(300, 2000), "updates": rng.randint(4, 8)}
+    return {"kind": kind, "scenes": log(24, 128), "max_side": log(16, 64), "updates": rng.randint(8, 32)}
+
+
+# ---- scenes ------------------------------------------------------------------
+
+
+class Scene:
+    """One scene's arrays as a program holds them (float32)."""
+
+    def __init__(self, gravity=(0.0, -9.81), bounds=HUGE, sub_steps=1, link_iters=1):
+        self.gravity, self.bounds, self.sub_steps, self.link_iters = gravity, bounds, sub_steps, link_iters
+        self.circles = False        # the bodies are circles of radius r (else particles)
+        self.r = 0.0
+        self.pos = self.prev = np.zeros((0, 2), np.float32)
+        self.pin = None             # particles: pinned flags
+        self.links = []             # (a, b, target) arrays, in order; links of one entry share no end
+        self.colliders = []         # ("circle", centre, radius) or ("polygon", vertices)
+        self.polygons = []          # (points, (a, b, t), is_static)
+
+    def solver(self):
+        s = Solver()
+        s.gravity, s.bounds = self.gravity, self.bounds
+        s.set_sub_steps(self.sub_steps)
+        s.set_link_iterations(self.link_iters)
+        n = len(self.pos)
+        if n and self.circles:
+            c = np.zeros((n, 7), np.float32)
+            c[:, 0:2], c[:, 2:4], c[:, 6] = self.pos, self.prev, self.r
+            s.add_circles(c)
+        elif n:
+            s.add_particles(self.pos, self.prev)
+        if self.links:
+            a, b, t = (np.concatenate(v) for v in zip(*self.links))
+            (s.add_circle_links if self.circles else s.add_particle_links)(a, b, t)
+        if self.pin is not None:
+            s.set_pinned_range(0, self.pin)
+        for c in self.colliders:
+            if c[0] == "circle":
+                s.add_static_circle(c[1], c[2])
+            else:
+                s.add_static_polygon(c[1])
+        for pts, (a, b, t), static in self.polygons:
+            p = np.zeros((len(pts), 6), np.float32)
+            p[:, 0:2] = p[:, 2:4] = pts
+            s.add_polygon(p, (a, b, t), static)
+        return s
+
+
+def grid_links(nx, ny, first=0):
+    """Structural and shear links of an ny x nx grid, spacing 1, in eight groups whose links share no end."""
+    i = first + np.arange(nx * ny, dtype=np.uint32).reshape(ny, nx)
+    diag = np.float32(math.sqrt(2.0))
+    groups = [(i[:, p:-1:2], i[:, p + 1::2], np.float32(1)) for p in (0, 1)]
+    groups += [(i[p:-1:2], i[p + 1::2], np.float32(1)) for p in (0, 1)]
+    groups += [(i[p:-1:2, :-1], i[p + 1::2, 1:], diag) for p in (0, 1)]
+    groups += [(i[p:-1:2, 1:], i[p + 1::2, :-1], diag) for p in (0, 1)]
+    return [(a.ravel(), b.ravel(), np.full(a.size, t, np.float32)) for a, b, t in groups if a.size]
+
+
+def grid(nx, ny, x0, y0, spacing=1.0):
+    """Points of an ny x nx grid whose first row is the top one."""
+    y, x = np.mgrid[0:ny, 0:nx]
+    return np.stack([x0 + spacing * x, y0 - spacing * y], -1).reshape(-1, 2)
+
+
+def moving(sc, rng, pos, jitter, drift, spread):
+    """Jittered positions with a common and a thermal velocity, carried as previous positions."""
+    p = pos + rng.uniform(-jitter, jitter, pos.shape)
+    v = np.asarray(drift) + spread * rng.standard_normal(pos.shape)
+    sc.pos = p.astype(np.float32)
+    sc.prev = (p - v * (DT / sc.sub_steps)).astype(np.float32)
+
+
+def random_collider(rng, centre, radius, polygon):
+    centre = (float(np.float32(centre[0])), float(np.float32(centre[1])))
+    if not polygon:
+        return ("circle", centre, float(np.float32(radius)))
+    m = int(rng.integers(3, 9))
+    a = (2 * math.pi * np.arange(m) + 0.9 * rng.uniform(-1, 1, m)) / m
+    return ("polygon", (np.array(centre) + radius * np.stack([np.cos(a), np.sin(a)], -1)).astype(np.float32))
+
+
+def cloth_scene(case, rng):
+    nx, ny = case["nx"], case["ny"]
+    sc = Scene(sub_steps=case["sub_steps"], link_iters=case["link_iters"])
+    moving(sc, rng, grid(nx, ny, 0.0, 0.0), 0.01, (0.0, 0.0), 0.0)
+    sc.links = grid_links(nx, ny)
+    sc.pin = np.zeros(nx * ny, np.uint8)
+    sc.pin[:nx] = 1
+    for k in range(case["colliders"]):
+        at = (nx * (k + rng.uniform(0.2, 0.8)) / case["colliders"], -ny - rng.uniform(-2.0, 6.0))
+        sc.colliders.append(random_collider(rng, at, rng.uniform(2.0, 8.0), k % 2 == 1))
+    return sc
+
+
+def polygon_scene(case, rng):
+    sc = Scene(gravity=(0.0, 98.2), bounds=((0.0, 0.0), (100.0, 100.0)))
+    n = case["points"]
+    for k in range(case["count"]):
+        c = np.array([12.0 + 19.0 * (k % 4), 12.0 + 24.0 * (k // 4)]) + rng.uniform(-2.0, 2.0, 2)
+        a = 2 * math.pi * (np.arange(n) + rng.uniform()) / n
+        pts = (c + rng.uniform(5.0, 8.0) * np.stack([np.cos(a), np.sin(a)], -1)).astype(np.float32)
+        ends = [(i, (i + 1) % n) for i in range(n)] + [(i, (i + n // 3) % n) for i in range(n)]
+        lo = np.array([min(e) for e in ends], np.uint64)
+        hi = np.array([max(e) for e in ends], np.uint64)
+        t = np.hypot(*(pts[lo.astype(int)] - pts[hi.astype(int)]).T).astype(np.float32)
+        sc.polygons.append((pts, (lo, hi, t), False))
+    ramp = np.array([[20, 70], [80, 78], [80, 82], [20, 82]], np.float32)
+    sc.polygons.append((ramp, (np.zeros(0, np.uint64), np.zeros(0, np.uint64), np.zeros(0, np.float32)), True))
+    return sc
+
+
+def gas_scene(case, rng):
+    n = case["n"]
+    box = 2.0 * math.sqrt(n)
+    sc = Scene(bounds=((0.0, 0.0), (box, box)), sub_steps=4)
+    sc.circles, sc.r = True, 0.5
+    moving(sc, rng, rng.uniform(0.5, box - 0.5, (n, 2)), 0.0, (0.0, 0.0), 1.0)
+    for _ in range(max(4, n // 4096)):
+        sc.colliders.append(random_collider(rng, rng.uniform(0.0, box, 2), rng.uniform(4.0, 16.0), False))
+    w = 64.0
+    for x0, y0, x1, y1 in ((-w, -w, 0, box + w), (box, -w, box + w, box + w), (-w, -w, box + w, 0),
+                           (-w, box, box + w, box + w)):
+        sc.colliders.append(("polygon", np.array([[x0, y0], [x1, y0], [x1, y1], [x0, y1]], np.float32)))
+    return sc
+
+
+def body_scene(rng, side, falling):
+    """A soft body of side x side linked circles: in flight without gravity, or falling onto the floor."""
+    w = 3.0 * side + 40.0
+    sc = Scene(gravity=(0.0, -9.81 if falling else 0.0), bounds=((0.0, 0.0), (w, w)), sub_steps=8)
+    sc.circles, sc.r = True, float(np.float32(0.35))
+    top = side + 0.5 if falling else w - 6.0
+    drift = (rng.uniform(-1, 1), -8.0) if falling else rng.uniform(-0.1, 0.1, 2)
+    moving(sc, rng, grid(side, side, 0.5 * (w - side + 1), top), 0.01, drift, 0.05 if falling else 0.0)
+    sc.links = grid_links(side, side)
+    polygon = bool(rng.integers(0, 2))
+    for _ in range(int(rng.integers(1, 9))):
+        at = (rng.uniform(0.1, 0.9) * w, -4.0 if falling else rng.uniform(0.1, 0.6) * w)
+        sc.colliders.append(random_collider(rng, at, rng.uniform(4.5, 7.0) if falling else rng.uniform(2.0, 10.0),
+                                            polygon))
+        polygon = not polygon
+    return sc
+
+
+def spread_sizes(lo, hi, count):
+    """count sizes spread log-uniformly over [lo, hi], the largest first, in no order of size."""
+    return [int(round(lo * (hi / lo) ** ((1.0 + 0.6180339887498949 * k) % 1.0 if k else 1.0))) for k in range(count)]
+
+
+def pile_scene(rng, n):
+    """n circles just out of touch, stacked over the floor of a narrow box, about to settle."""
+    cols = max(4, int(math.sqrt(n)))
+    sc = Scene(bounds=((0.0, 0.0), (0.75 * cols + 1.0, 200.0)), sub_steps=8)
+    sc.circles, sc.r = True, float(np.float32(0.35))
+    rows = -(-n // cols)
+    moving(sc, rng, grid(cols, rows, 0.7, 0.4 + 0.75 * (rows - 1), 0.75)[:n], 0.02, (0.0, -1.0), 0.5)
+    sc.colliders.append(random_collider(rng, (0.375 * cols, 0.0), 1.0, False))
+    return sc
+
+
+def scenes_of(case, seed):
+    rng = np.random.default_rng(seed)
+    kind = case["kind"]
+    if kind == "frames":
+        return [(polygon_scene if case["scene"] == "polygons" else cloth_scene)(case, rng)]
+    if kind == "cloth":
+        return [cloth_scene(case, rng)]
+    if kind == "gas":
+        return [gas_scene(case, rng)]
+    if kind == "image":
+        return [body_scene(rng, case["side"], True)]
+    if kind == "pile":
+        return [pile_scene(rng, n) for n in spread_sizes(64.0, case["max_n"], case["scenes"])]
+    return [body_scene(rng, side, False) for side in spread_sizes(4.0, case["max_side"], case["scenes"])]
+
+
+# ---- the calls ---------------------------------------------------------------
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    st = {"case": case, "solvers": [sc.solver() for sc in scenes_of(case, seed)]}
+    first = st["solvers"][0]
+    if kind in ("frames", "cloth"):
+        # the running program: its first update has planned the scene
+        first.set_readback(bool(case.get("readback", False)))
+        first.update(DT)
+        first.sync()
+    elif kind == "image":
+        img = SceneImage(first)
+        st["image"] = img
+        st["stored"] = torch.from_numpy(img.host).cuda()
+        st["live"] = torch.empty_like(st["stored"])
+        st["work"] = torch.empty(img.workspace_bytes, dtype=torch.uint8, device="cuda")
+        st["host"] = torch.empty(img.host.nbytes, dtype=torch.uint8, pin_memory=True)
+    elif kind == "batch":
+        st["batch"] = Batch()
+        for s in st["solvers"]:
+            st["batch"].add_scene(s)
+        st["batch"].update(DT, 1)
+        st["batch"].sync()
+    elif kind == "served":
+        st["server"] = Server(memory_budget=1 << 30, steps_per_launch=case["updates"])
+        st["ids"] = [st["server"].create(s, 1, DT)[1] for s in st["solvers"]]
+        if not st["server"].wait_idle():
+            raise RuntimeError("the server did not finish its first requests")
+        st["server"].poll()
+    return st
+
+
+def run(st):
+    case, solvers = st["case"], st["solvers"]
+    kind, first = case["kind"], solvers[0]
+    if kind == "frames":
+        first.update(DT)
+        if case["scene"] == "cloth":
+            return first.get_particles()
+        return np.concatenate([first.get_polygon(i)["particles"] for i in range(first.get_polygons_len())])
+    if kind == "cloth":
+        for _ in range(case["updates"]):
+            first.update(DT)
+        return first.get_particles()
+    if kind == "gas":
+        world = first.clone()
+        for _ in range(case["updates"]):
+            world.update(DT)
+        return world.get_circles()
+    if kind == "image":
+        st["live"].copy_(st["stored"])
+        stream = torch.cuda.current_stream()
+        st["image"].update(st["live"].data_ptr(), st["work"].data_ptr(), st["work"].numel(), DT, case["updates"],
+                           stream.cuda_stream)
+        st["host"].copy_(st["live"], non_blocking=True)
+        stream.synchronize()
+        SceneImage.read(first, st["host"].numpy())
+        return first.get_circles()
+    if kind == "pile":
+        batch = Batch()
+        for s in solvers:
+            batch.add_scene(s)
+        batch.update(DT, case["updates"])
+        if "out" not in st:  # solvers that receive the results; `solvers` keep the start
+            st["out"] = [s.clone() for s in solvers]
+        for i, s in enumerate(st["out"]):
+            batch.read_scene(i, s)
+        return np.concatenate([s.get_circles() for s in st["out"]])
+    if kind == "batch":
+        st["batch"].update(DT, case["updates"])
+        for i, s in enumerate(solvers):
+            st["batch"].read_scene(i, s)
+        return np.concatenate([s.get_circles() for s in solvers])
+    server = st["server"]
+    for sid in st["ids"]:
+        server.advance(sid, case["updates"], DT)
+    if not server.wait_idle() or any(d["status"] for d in server.poll()):
+        raise RuntimeError("a request failed")
+    for sid, s in zip(st["ids"], solvers):
+        server.read_scene(sid, s)
+    return np.concatenate([s.get_circles() for s in solvers])
+
+
+def work(case):
+    """Bytes: each body's position and previous position read and written once, each link record read once.
+    Flops: the link, pair, collider and integration laws, once for each substep (and link sweep)."""
+    total_bytes = flops = 0.0
+    for sc in scenes_of(case, 0):
+        n = len(sc.pos) + sum(len(p[0]) for p in sc.polygons)
+        links = sum(len(l[0]) for l in sc.links) + sum(len(p[1][0]) for p in sc.polygons)
+        steps = case.get("updates", 1) * sc.sub_steps
+        total_bytes += 32.0 * n + 12.0 * links
+        flops += steps * (22.0 * links * sc.link_iters + n * (20.0 + 4.0 * len(sc.colliders)) +
+                          (20.0 * n if sc.circles else 0.0))
+    return {"bytes": total_bytes, "flops": flops}
+
+
+# ---- the same scenes in 64 bits ----------------------------------------------
+
+
+def exact(case, seed):
+    scenes = scenes_of(case, seed)
+    kind = case["kind"]
+    updates = case.get("updates", 1) + (0 if kind in ("gas", "image", "pile") else 1)
+    # pair sweeps in plain Python take about 5 us a circle and substep
+    rows = sum(len(sc.pos) * sc.sub_steps * updates for sc in scenes if sc.circles)
+    if kind in ("gas", "image", "pile") and rows > 2.0e6:
+        return None
+    # and link groups about 100 us each in torch
+    groups = sum(len(sc.links) * sc.link_iters * sc.sub_steps * updates for sc in scenes)
+    if groups > 1.2e5:
+        return None
+    out = []
+    for sc in scenes:
+        v = exact_polygons(sc, updates) if sc.polygons else exact_bodies(sc, updates, kind in ("batch", "served"))
+        if v is None:
+            return None
+        out.append(v)
+    return np.concatenate(out)
+
+
+def planes_of(vertices):
+    v = np.asarray(vertices, np.float64)
+    nxt = np.roll(v, -1, 0)
+    if float(np.sum(v[:, 0] * nxt[:, 1] - nxt[:, 0] * v[:, 1])) < 0.0:
+        v = v[::-1]
+        nxt = np.roll(v, -1, 0)
+    e = nxt - v
+    n = np.stack([e[:, 1], -e[:, 0]], -1) / np.hypot(e[:, 0], e[:, 1])[:, None]
+    return n, np.sum(n * v, -1)
+
+
+def bodies_phase(p, q, sc, delta, free):
+    """Colliders, bounds and Verlet of the bodies `free` marks (torch, 64 bits)."""
+    r = sc.r
+    p0, q0 = p.clone(), q.clone()
+    for c in sc.colliders:
+        if c[0] == "circle":
+            d = p - torch.tensor(c[1], dtype=p.dtype, device=p.device)
+            dist = d.norm(dim=1, keepdim=True)
+            hit = (dist < r + c[2]) & (dist > 0)
+            p = torch.where(hit, p + d / dist * (r + c[2] - dist), p)
+        else:
+            n, off = (torch.tensor(x, dtype=p.dtype, device=p.device) for x in planes_of(c[1]))
+            smax, arg = (p @ n.T - off).max(dim=1, keepdim=True)
+            p = torch.where(smax < r, p + n[arg[:, 0]] * (r - smax), p)
+    (lx, ly), (sx, sy) = sc.bounds
+    lo = torch.tensor([lx, ly], dtype=p.dtype, device=p.device) + r
+    hi = torch.tensor([lx + sx, ly + sy], dtype=p.dtype, device=p.device) - r
+    for lim, out in ((lo, p < lo), (hi, p > hi)):
+        q, p = torch.where(out, lim - (q - p), q), torch.where(out, lim.expand_as(p), p)
+    g = torch.tensor([float(np.float32(x)) for x in sc.gravity], dtype=p.dtype, device=p.device)
+    p, q = p + (p - q) + g * delta * delta, p
+    return torch.where(free, p, p0), torch.where(free, q, q0)
+
+
+def circle_pairs(p, r):
+    """The circle pairs (i, j), i < j, in order, each against the positions the pairs before it left."""
+    pos = p.tolist()
+    margin = r
+    h = 2.0 * r + margin
+    cells = {}
+    cell = [(math.floor(x / h), math.floor(y / h)) if x == x and y == y else None for x, y in pos]
+    for i, c in enumerate(cell):
+        if c:
+            cells.setdefault(c, set()).add(i)
+    touch = 4.0 * r * r
+
+    def move(i, x, y):
+        pos[i] = [x, y]
+        if x != x:  # takes part in no further pair
+            cells[cell[i]].discard(i)
+            return
+        c = (math.floor(x / h), math.floor(y / h))
+        if c != cell[i]:
+            cells[cell[i]].discard(i)
+            cells.setdefault(c, set()).add(i)
+            cell[i] = c
+
+    for i in range(len(pos)):
+        last = i
+        while True:
+            # every j > last near circle i, until i has moved out of the margin
+            x0, y0 = pos[i]
+            if cell[i] is None or x0 != x0:
+                break
+            cx, cy = cell[i]
+            near = sorted(j for dx in (-1, 0, 1) for dy in (-1, 0, 1) for j in cells.get((cx + dx, cy + dy), ())
+                          if j > last and (pos[j][0] - x0) ** 2 + (pos[j][1] - y0) ** 2 < h * h)
+            for j in near:
+                last = j
+                xi, yi = pos[i]
+                xj, yj = pos[j]
+                dx, dy = xi - xj, yi - yj
+                d2 = dx * dx + dy * dy
+                if d2 < touch:
+                    d = math.sqrt(d2)
+                    k = 0.5 * (2.0 * r - d) / d if d else math.nan  # two at one place lose their positions
+                    move(i, xi + dx * k, yi + dy * k)
+                    move(j, xj - dx * k, yj - dy * k)
+                    if not math.hypot(pos[i][0] - x0, pos[i][1] - y0) <= 0.99 * margin:
+                        break
+            else:
+                break
+    return torch.tensor(pos, dtype=torch.float64)
+
+
+def exact_bodies(sc, updates, in_flight):
+    device = "cuda" if len(sc.pos) > 20000 and not sc.circles else "cpu"
+    p, q = (torch.tensor(x, dtype=torch.float64, device=device) for x in (sc.pos, sc.prev))
+    free = torch.ones(len(p), 1, dtype=torch.bool, device=device)
+    if sc.pin is not None:
+        free = torch.tensor(sc.pin == 0, device=device)[:, None]
+    links = [(torch.tensor(a.astype(np.int64), device=device), torch.tensor(b.astype(np.int64), device=device),
+              float(t[0])) for a, b, t in sc.links]
+    delta = float(np.float32(DT)) / sc.sub_steps
+    for _ in range(updates * sc.sub_steps):
+        for _ in range(sc.link_iters):
+            for a, b, t in links:
+                pa, pb, fa, fb = p[a], p[b], free[a], free[b]
+                d = pa - pb
+                dist = d.norm(dim=1, keepdim=True)
+                c = d / dist * (dist - t)
+                p[a] = torch.where(fa, pa - torch.where(fb, 0.5 * c, c), pa)
+                p[b] = torch.where(fb, pb + torch.where(fa, 0.5 * c, c), pb)
+        if in_flight:
+            # a body in flight keeps its circles apart: no pair acts
+            if links and min(float((p[a] - p[b]).norm(dim=1).min()) for a, b, _ in links) <= 2.0 * sc.r:
+                return None
+        elif sc.circles:
+            p = circle_pairs(p, sc.r)
+        p, q = bodies_phase(p, q, sc, delta, free)
+    out = np.zeros((len(p), 7 if sc.circles else 6))
+    out[:, 0:2], out[:, 2:4] = p.cpu().numpy(), q.cpu().numpy()
+    if sc.circles:
+        out[:, 6] = sc.r
+    return out
+
+
+def crossing(p1, p2, p3, p4):
+    s1, s2 = p2 - p1, p4 - p3
+    den = -s2[0] * s1[1] + s1[0] * s2[1]
+    if den == 0.0:
+        return None
+    d = p1 - p3
+    s, t = (-s1[1] * d[0] + s1[0] * d[1]) / den, (s2[0] * d[1] - s2[1] * d[0]) / den
+    return p1 + t * s1 if 0.0 <= s <= 1.0 and 0.0 <= t <= 1.0 else None
+
+
+def push_out(pts, centre, other, other_centre):
+    """Every edge of one polygon against the points of another; the last point that hits moves the edge."""
+    n = len(pts)
+    for e in range(n):
+        a, b = pts[e].copy(), pts[(e + 1) % n].copy()
+        for k in range(len(other)):
+            o = other[k].copy()
+            at = crossing(a, b, o, other_centre)
+            if at is None:
+                continue
+            along = (b - a) / np.hypot(*(b - a))
+            inward = centre - (at + along * float(along @ (centre - at)))
+            inward = inward / np.hypot(*inward)
+            to_a, to_b = np.hypot(*(at - a)), np.hypot(*(at - b))
+            shift = 2.0 / 3.0 * inward * float(inward @ (at - o))
+            new = crossing(a, b, o, o - 10000.0 * inward)
+            if new is None:
+                continue
+            pts[e], pts[(e + 1) % n] = a - shift * to_b / (to_a + to_b), b - shift * to_a / (to_a + to_b)
+            other[k] = new
+
+
+def exact_polygons(sc, updates):
+    polys = [np.array(p[0], np.float64) for p in sc.polygons]
+    prevs = [p.copy() for p in polys]
+    g = np.array([float(np.float32(x)) for x in sc.gravity])
+    lo = np.array(sc.bounds[0])
+    hi = lo + np.array(sc.bounds[1])
+    delta = float(np.float32(DT)) / sc.sub_steps
+    accs = [np.zeros_like(p) for p in polys]
+    for _ in range(updates * sc.sub_steps):
+        for acc in accs:
+            acc += g
+        centres = [p.mean(0) for p in polys]
+        for p, (_, (la, lb, lt), _) in zip(polys, sc.polygons):
+            for a, b, t in zip(la.astype(int), lb.astype(int), lt.astype(np.float64)):
+                d = p[a] - p[b]
+                dist = np.hypot(*d)
+                c = 0.5 * d / dist * (dist - t)
+                p[a] -= c
+                p[b] += c
+        for i in range(len(polys)):
+            for j in range(i + 1, len(polys)):
+                push_out(polys[i], centres[i], polys[j], centres[j])
+                push_out(polys[j], centres[j], polys[i], centres[i])
+        for k, (p, q) in enumerate(zip(polys, prevs)):
+            for lim, out in ((lo, p < lo), (hi, p > hi)):
+                q[out] = (lim - (q - p))[out]
+                p[out] = np.broadcast_to(lim, p.shape)[out]
+            if not sc.polygons[k][2]:
+                polys[k], prevs[k] = p + (p - q) + accs[k] * delta * delta, p.copy()
+                accs[k][:] = 0.0
+    return np.concatenate([np.concatenate(v, 1) for v in zip(polys, prevs, accs)])
