@@ -212,7 +212,7 @@ def body_scene(rng, side, falling):
     sc = Scene(gravity=(0.0, -9.81 if falling else 0.0), bounds=((0.0, 0.0), (w, w)), sub_steps=8)
     sc.circles, sc.r = True, float(np.float32(0.35))
     top = side + 0.5 if falling else w - 6.0
-    drift = (rng.uniform(-1, 1), -8.0) if falling else rng.uniform(-0.1, 0.1, 2)
+    drift = (rng.uniform(-1, 1), -20.0) if falling else rng.uniform(-0.1, 0.1, 2)
     moving(sc, rng, grid(side, side, 0.5 * (w - side + 1), top), 0.01, drift, 0.05 if falling else 0.0)
     sc.links = grid_links(side, side)
     polygon = bool(rng.integers(0, 2))
