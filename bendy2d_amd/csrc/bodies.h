@@ -19,6 +19,32 @@ struct BodyParams {
     uint32_t ncol, nplanes;
 };
 
+// A convex polygon's planes (nx, ny, c) against a body of radius r.  The push
+// uses the plane of largest signed distance, and only when that distance is
+// below r; a plane at r or beyond already rules the push out, so the scan stops
+// once it has for every lane (a NaN distance, first or later, never pushes
+// either way).  plane(e): the e-th plane, e uniform; own(e): the same at a
+// lane's own e.
+template <typename F, typename G>
+__device__ __forceinline__ void static_planes(float2 &p, float r, uint32_t n, F &&plane, G &&own) {
+    float smax = 0.0f;
+    uint32_t arg = 0xffffffffu;
+    bool out = n == 0u;
+#pragma unroll 1
+    for (uint32_t e = 0; e < n; e++) {
+        const auto w = plane(e);
+        const float sd = (w.x * p.x + w.y * p.y) - w.z;
+        out = out || sd >= r;
+        if (arg == 0xffffffffu || sd > smax) { smax = sd; arg = e; }
+        if (__ballot(!out) == 0ull) return;
+    }
+    if (!out && smax < r) {
+        const auto w = own(arg);
+        const float push = r - smax;
+        p.x = p.x + w.x * push; p.y = p.y + w.y * push;
+    }
+}
+
 // Static colliders in insertion order against a body of radius r (0 for
 // particles and polygon points).  hdr: (kind, plane offset, planes, -);
 // geo: circle (cx, cy, R, -); pl: polygon edge planes (nx, ny, c, -).

@@ -44,23 +44,67 @@ __global__ void __launch_bounds__(WG) k_tiled_pass(const float2 *__restrict__ sr
     const uint32_t t = xcd_tile(blockIdx.x, ntiles);
     const TileInfo ti = tiles[t];
     const int tid = threadIdx.x;
+    const uint32_t *lo = loff + ti.loff_off;
+    const LinkS *lk = links + ti.link_off;
+    // Layer bounds: each lane holds one, read back by lane (a load before every
+    // layer would put its latency there); past 63 layers they are loaded.
+    const uint32_t lane = tid & 63u;
+    const uint32_t held = lo[min(lane, nlayers)];
+    auto bound = [&](uint32_t L) { return L < 64u ? (uint32_t)__builtin_amdgcn_readlane(held, L) : lo[L]; };
+    // A thread's first two records of the next layer load while it solves the
+    // current one (and stay in flight across the barrier): nothing is left
+    // behind a barrier but LDS and arithmetic.  Loads past a layer's end read
+    // its tile's first record instead, unused.  (1024 x 1024 cloth: 0.515 ->
+    // 0.475 ms an update.)
+    auto load = [&](uint32_t l, uint32_t e) { return lk[l < e ? l : 0u]; };
+    uint32_t b0 = bound(0), b1 = bound(1);
+    LinkS n0 = load(b0 + tid, b1), n1 = load(b0 + WG + tid, b1);
     for (uint32_t r = tid; r < ti.int_count; r += WG) s_reg[region_slot(r)] = src[ti.int_start + r];
     for (uint32_t h = tid; h < ti.halo_count; h += WG)
         s_reg[region_slot(ti.int_count + h)] = src[halo[ti.halo_off + h]];
-    __syncthreads();
-    const uint32_t *lo = loff + ti.loff_off;
-    const LinkS *lk = links + ti.link_off;
-    for (uint32_t L = 0; L < nlayers; L++) {
-        const uint32_t e = lo[L + 1];
-        for (uint32_t l = lo[L] + tid; l < e; l += WG) {
-            LinkS rec = lk[l];
-            const uint32_t a = rec.a & 0x7fffu, b = rec.b & 0x7fffu;
-            float2 A = s_reg[a], B = s_reg[b];
-            solve_particle_link(A.x, A.y, B.x, B.y, rec.t, (rec.a & kScenePinBit) != 0, (rec.b & kScenePinBit) != 0);
-            s_reg[a] = A;
-            s_reg[b] = B;
+    lds_barrier();
+    auto solve = [&](const LinkS &rec) {
+        const uint32_t a = rec.a & 0x7fffu, b = rec.b & 0x7fffu;
+        float2 A = s_reg[a], B = s_reg[b];
+        const float dx = A.x - B.x, dy = A.y - B.y;
+        float dist, nx, ny;
+        length_and_unit(dx, dy, dx * dx + dy * dy, dist, nx, ny);
+        const float e = dist - rec.t;
+        nx = nx * e;
+        ny = ny * e;
+        float cx = nx * 0.5f, cy = ny * 0.5f;
+        // a free end beside a pinned one takes the whole correction (a
+        // wavefront without pinned ends passes this by)
+        const bool pa = (rec.a & kScenePinBit) != 0, pb = (rec.b & kScenePinBit) != 0;
+        if (__builtin_expect(__ballot(((rec.a | rec.b) & kScenePinBit) != 0) != 0ull, 0)) {
+            const float2 a0 = A, b0 = B;
+            if (pa || pb) { cx = nx; cy = ny; }
+            A.x = A.x - cx; A.y = A.y - cy;
+            B.x = B.x + cx; B.y = B.y + cy;
+            if (pa) A = a0;
+            if (pb) B = b0;
+        } else {
+            A.x = A.x - cx; A.y = A.y - cy;
+            B.x = B.x + cx; B.y = B.y + cy;
         }
-        __syncthreads();
+        s_reg[a] = A;
+        s_reg[b] = B;
+    };
+    for (uint32_t L = 0; L < nlayers; L++) {
+        const LinkS r0 = n0, r1 = n1;
+        const uint32_t l = b0 + tid, lo0 = b0, e = b1;
+        if (L + 1 < nlayers) {
+            b0 = b1;
+            b1 = bound(L + 2);
+            n0 = load(b0 + tid, b1);
+            n1 = load(b0 + WG + tid, b1);
+        }
+        if (l < e) solve(r0);
+        if (lo0 + WG < e) {
+            if (l + WG < e) solve(r1);
+            for (uint32_t k = l + 2 * WG; k < e; k += WG) solve(lk[k]);
+        }
+        lds_barrier();
     }
     if (fuse) {
         for (uint32_t r = tid; r < ti.int_count; r += WG) {
