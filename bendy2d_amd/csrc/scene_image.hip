@@ -53,17 +53,6 @@ int fail(int code, const std::string &msg) {
     return code;
 }
 
-// Launch shape of a single scene on an otherwise idle device, as the SCENE
-// engine picks it: about two bodies per lane; positions, previous positions
-// and (when they fit) link records in LDS.
-void launch_shape(const SceneDesc &d, uint32_t &wg, uint32_t &lds) {
-    uint32_t want = 64;
-    while (want < 1024 && want * 2 < d.N) want <<= 1;
-    wg = want;
-    const size_t with_links = 16ull * d.N + 8ull * d.L;
-    lds = (uint32_t)(with_links <= scene_max_lds() ? with_links : std::min<size_t>(16ull * d.N, scene_max_lds()));
-}
-
 int image_of(const bd_solver *s, SceneImage &img, std::string &err) {
     HostScene h;
     int rc = solver_export(s, h, err);
@@ -209,7 +198,7 @@ int32_t bd_scene_image_describe(const bd_solver *s, bd_scene_image_info *info) {
     info->workspace_bytes = img.desc.Nc >= 2 ? img.desc.ws_bytes : 0u;
     info->n_bodies = img.desc.N;
     info->n_circles = img.desc.Nc;
-    launch_shape(img.desc, info->workgroup, info->lds_bytes);
+    scene_launch_shape(img.desc, info->workgroup, info->lds_bytes);
     return BD_OK;
 }
 

@@ -1,0 +1,67 @@
+"""Circle-pair sweeps over active lists against the f32 oracle bit for bit:
+piles whose round state and lists sit in LDS, in place of parked positions or
+in the workspace, of one radius or several, slow and fast enough that circles
+leave their margins (so sweeps are checked pair by pair, or run again wider)."""
+import numpy as np
+import pytest
+
+from helpers import bits_equal, first_diff, state, to_oracle
+from bendy2d_amd import Batch, Solver
+
+pytestmark = pytest.mark.gpu
+
+DT = 1.0 / 60.0
+# bytes of LDS: none; a few circles' state; positions without previous ones;
+# state in place of previous positions and lists in the workspace; all of it
+BUDGETS = [0, 2048, 9 * 1024, 28 * 1024, 144 * 1024]
+
+
+def pile(n, seed, mixed, speed):
+    rng = np.random.default_rng(seed)
+    cols = max(2, int(np.sqrt(n)))
+    k = np.arange(n)
+    c = np.zeros((n, 7), np.float32)
+    c[:, 0] = 1.0 + 0.72 * (k % cols) + rng.uniform(-0.03, 0.03, n)
+    c[:, 1] = 0.6 + 0.72 * (k // cols) + rng.uniform(-0.03, 0.03, n)
+    c[:, 2:4] = c[:, 0:2] - speed * rng.standard_normal((n, 2)) * (DT / 4)
+    c[:, 6] = rng.uniform(0.2, 0.5, n) if mixed else 0.35
+    s = Solver()
+    s.gravity, s.bounds = (0.0, -9.81), ((0.0, 0.0), (0.75 * cols + 2.0, 200.0))
+    s.set_sub_steps(4)
+    s.add_circles(c)
+    return s
+
+
+@pytest.mark.parametrize("lds", BUDGETS)
+@pytest.mark.parametrize("mixed,speed", [(False, 0.5), (True, 2.0), (False, 60.0), (True, 200.0)])
+def test_piles(lds, mixed, speed):
+    scenes = [pile(n, 10 * n + int(speed), mixed, speed) for n in (2, 33, 65, 300, 1500)]
+    oracles = [to_oracle(s, 32, candidate_mode=True) for s in scenes]
+    b = Batch()
+    for s in scenes:
+        b.add_scene(s)
+    b.config = dict(wg_small=128, wg_large=1024, split_points=1024, lds_small=lds, lds_large=lds,
+                    steps_per_launch=2, use_graph=0, split_tiny=64, wg_tiny=64, lds_tiny=lds)
+    b.update(DT, 4)
+    b.sync()
+    assert b.cc_stats()["err_scenes"] == 0
+    for i, (s, o) in enumerate(zip(scenes, oracles)):
+        for _ in range(4):
+            assert o.update(DT) == 0
+        b.read_scene(i, s)
+        assert bits_equal(state(s), state(o)), f"scene {i}: {first_diff(state(s), state(o))}"
+
+
+@pytest.mark.parametrize("n", [31, 32, 33, 34, 300])
+def test_clump(n):
+    # every circle touches every other: lists as long as the scene
+    rng = np.random.default_rng(n)
+    s = Solver()
+    for _ in range(n):
+        s.add_circle(rng.uniform(-0.3, 0.3, 2).astype(np.float32), 1.0)
+    s.gravity, s.bounds = (0.0, 0.0), ((-1000.0, -1000.0), (2000.0, 2000.0))
+    o = to_oracle(s, 32)
+    for _ in range(3):
+        s.update(DT)
+        assert o.update(DT) == 0
+    assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
