@@ -93,6 +93,42 @@ void BatchCore::build_order(const std::vector<uint32_t> &active) {
     n_large = (uint32_t)large.size();
     order_dirty = true;
     invalidate_graph();
+    choose_shapes();
+}
+
+// The classes' workgroups and LDS.  The configured ones suit a full device: few
+// lanes to a small scene, so that many scenes share a CU.  While every scene of
+// the launch can have lanes of its own, the launch takes as long as its slowest
+// scene, and the classes run on what their largest scene would run on alone:
+// about two bodies to a lane, everything in LDS.  The line is where all
+// scenes' own workgroups and LDS are resident at once (3 wavefronts to a SIMD
+// at the kernels' register counts, 144 KiB of LDS to a CU): 48 flying bodies of
+// up to 40 x 40 (12,000 lanes) ran 375 us an update on 64 and 128 lanes and run
+// 116 on 256 and 1,024; 640 bodies of up to 128 x 128 (400,000 lanes) stay as
+// configured.
+void BatchCore::choose_shapes() {
+    tiny = Shape{cfg.wg_tiny, cfg.lds_tiny};
+    small = Shape{cfg.wg_small, cfg.lds_small};
+    large = Shape{cfg.wg_large, cfg.lds_large};
+    if (!adapt) return;
+    Shape own[3];
+    const uint32_t count[3] = {n_tiny, n_small, n_large};
+    uint64_t lanes = 0, lds = 0;
+    for (size_t k = 0; k < order.size(); k++) {
+        const int c = k < n_tiny ? 0 : k < n_tiny + n_small ? 1 : 2;
+        uint32_t wg, bytes;
+        scene_launch_shape(descs[order[k]], wg, bytes);
+        own[c].wg = std::max(own[c].wg, wg);
+        own[c].lds = std::max(own[c].lds, bytes);
+    }
+    for (int c = 0; c < 3; c++) {
+        lanes += (uint64_t)count[c] * own[c].wg;
+        lds += (uint64_t)count[c] * own[c].lds;
+    }
+    if (lanes > (uint64_t)num_cu * 768u || lds > (uint64_t)num_cu * scene_max_lds()) return;
+    tiny = Shape{std::max(tiny.wg, own[0].wg), std::max(tiny.lds, own[0].lds)};
+    small = Shape{std::max(small.wg, own[1].wg), std::max(small.lds, own[1].lds)};
+    large = Shape{std::max(large.wg, own[2].wg), std::max(large.lds, own[2].lds)};
 }
 
 void BatchCore::order_by(const std::vector<uint64_t> &cost) {
@@ -137,8 +173,8 @@ int BatchCore::upload_tables(std::string &err) {
 // streams.
 int BatchCore::enqueue_launch(uint32_t steps, std::string &err) {
     launch_fill_u32((uint32_t *)d_queue.p, 3, 0u, stream);
-    int vs = variant_for_wg((int)cfg.wg_small), vl = variant_for_wg((int)cfg.wg_large);
-    int vt = n_tiny ? variant_for_wg((int)cfg.wg_tiny) : 0;
+    int vs = variant_for_wg((int)small.wg), vl = variant_for_wg((int)large.wg);
+    int vt = n_tiny ? variant_for_wg((int)tiny.wg) : 0;
     if (vs < 0 || vl < 0 || vt < 0) { err = "no kernel variant for the configured workgroup size"; return BD_ERR_ARG; }
     const SceneDesc *dd = (const SceneDesc *)d_desc.p;
     const uint32_t *od = (const uint32_t *)d_order.p;
@@ -147,22 +183,22 @@ int BatchCore::enqueue_launch(uint32_t steps, std::string &err) {
     BD_HIP(hipStreamWaitEvent(side, ev_fork, 0));
     if (n_tiny) {
         BD_HIP(hipStreamWaitEvent(side2, ev_fork, 0));
-        uint32_t blocks = std::min<uint32_t>(n_tiny, (uint32_t)(num_cu * scene_blocks_per_cu(vt, cfg.lds_tiny)));
-        int rc = launch_scene_variant(vt, std::max<uint32_t>(blocks, 1), cfg.lds_tiny, side2, dd, states_dev(), od,
+        uint32_t blocks = std::min<uint32_t>(n_tiny, (uint32_t)(num_cu * scene_blocks_per_cu(vt, tiny.lds)));
+        int rc = launch_scene_variant(vt, std::max<uint32_t>(blocks, 1), tiny.lds, side2, dd, states_dev(), od,
                                       n_tiny, q + 2, steps, err);
         if (rc) return rc;
         BD_HIP(hipEventRecord(ev_join2, side2));
     }
     od += n_tiny;
     if (n_large) {
-        uint32_t blocks = std::min<uint32_t>(n_large, (uint32_t)(num_cu * scene_blocks_per_cu(vl, cfg.lds_large)));
-        int rc = launch_scene_variant(vl, std::max<uint32_t>(blocks, 1), cfg.lds_large, side, dd, states_dev(), od + n_small,
+        uint32_t blocks = std::min<uint32_t>(n_large, (uint32_t)(num_cu * scene_blocks_per_cu(vl, large.lds)));
+        int rc = launch_scene_variant(vl, std::max<uint32_t>(blocks, 1), large.lds, side, dd, states_dev(), od + n_small,
                                       n_large, q + 1, steps, err);
         if (rc) return rc;
     }
     if (n_small) {
-        uint32_t blocks = std::min<uint32_t>(n_small, (uint32_t)(num_cu * scene_blocks_per_cu(vs, cfg.lds_small)));
-        int rc = launch_scene_variant(vs, std::max<uint32_t>(blocks, 1), cfg.lds_small, stream, dd, states_dev(), od,
+        uint32_t blocks = std::min<uint32_t>(n_small, (uint32_t)(num_cu * scene_blocks_per_cu(vs, small.lds)));
+        int rc = launch_scene_variant(vs, std::max<uint32_t>(blocks, 1), small.lds, stream, dd, states_dev(), od,
                                       n_small, q, steps, err);
         if (rc) return rc;
     }
@@ -292,6 +328,7 @@ bd_batch *bd_batch_new(void) {
     try {
         bd_batch *b = new bd_batch();
         b->core.cfg = bd_batch_config{128, 1024, 2048, 32 * 1024, 144 * 1024, 1, 1, 400, 64, 8 * 1024};
+        b->core.adapt = true;
         return b;
     } catch (...) {
         set_last_error("allocation failed");
@@ -465,6 +502,8 @@ int32_t bd_batch_set_config(bd_batch *b, const bd_batch_config *cfg) {
     if (b->core.cfg.lds_tiny > scene_max_lds()) b->core.cfg.lds_tiny = (uint32_t)scene_max_lds();
     if (b->core.cfg.steps_per_launch < 1) b->core.cfg.steps_per_launch = 1;
     b->core.invalidate_graph();
+    b->core.adapt = false;  // as asked from now on
+    b->core.choose_shapes();
     if (reorder && b->uploaded) {
         std::vector<uint32_t> all(b->images.size());
         std::iota(all.begin(), all.end(), 0u);

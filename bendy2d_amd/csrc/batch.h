@@ -23,6 +23,11 @@ struct BatchCore {
     std::vector<uint64_t> order_ticks;   // per scene slot: its device ticks at the last ordering
     std::vector<uint32_t> order_rounds;  // per scene slot: its pair rounds at the last ordering
     uint32_t n_tiny = 0, n_small = 0, n_large = 0;
+    // the configuration is the default one: launches that leave CUs idle take
+    // wider workgroups and more LDS than it says (see choose_shapes)
+    bool adapt = false;
+    struct Shape { uint32_t wg = 0, lds = 0; };
+    Shape tiny, small, large;         // what the classes run on
     bool descs_dirty = true, order_dirty = true;
     DevBuf<uint8_t> d_desc, d_order, d_queue;
     size_t d_desc_cap = 0;
@@ -42,6 +47,7 @@ struct BatchCore {
     int init_device(std::string &err);
     void invalidate_graph();
     void build_order(const std::vector<uint32_t> &active);
+    void choose_shapes();
     // the same classes, each ordered by cost[slot] (largest first, ties by
     // bodies plus links); the launch graph stays valid
     void order_by(const std::vector<uint64_t> &cost);

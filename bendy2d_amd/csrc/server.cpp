@@ -420,6 +420,7 @@ bd_server *bd_server_new(const bd_server_config *cfg) {
     std::unique_ptr<bd_server> S(new bd_server());
     S->cfg = *cfg;
     S->core.cfg = cfg->launch;
+    S->core.adapt = S->heavy.adapt = !S->core.cfg.wg_small;
     if (!S->core.cfg.wg_small) S->core.cfg = bd_batch_config{128, 1024, 2048, 32 * 1024, 144 * 1024, 1, 0, 400, 64, 8 * 1024};
     S->core.cfg.use_graph = 0;
     S->core.cfg.steps_per_launch = std::max<uint32_t>(cfg->steps_per_launch, 1);

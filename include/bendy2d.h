@@ -302,7 +302,10 @@ typedef struct bd_batch bd_batch;
  * steps_per_launch updates run per kernel launch; use_graph replays the launch
  * sequence as a captured hipGraph.  A third class takes the smallest scenes:
  * those of at most split_tiny bodies run on workgroups of wg_tiny threads with
- * lds_tiny bytes of LDS (split_tiny = 0: no third class). */
+ * lds_tiny bytes of LDS (split_tiny = 0: no third class).  Until a
+ * configuration is set (bd_batch_set_config, bd_batch_autotune, a server's
+ * launch), launches whose scenes leave CUs idle take wider workgroups and more
+ * LDS than the default one says. */
 typedef struct bd_batch_config {
     uint32_t wg_small, wg_large;
     uint32_t split_points;

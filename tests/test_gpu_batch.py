@@ -229,3 +229,27 @@ def test_round_state_placements(lds_small, placement):
     st = [b.scene_status(i) for i in range(len(scenes))]
     assert all(x["err"] == 0 for x in st), st
     assert sum(x["rounds"] for x in st) > 0
+
+
+@pytest.mark.parametrize("count", [1, 5, 300, 800])
+def test_default_shapes_match_oracle(count):
+    # the default configuration widens workgroups while CUs would be idle and
+    # not beyond; every class is present, scenes repeat every five
+    sides = (2, 5, 19, 33, 47)
+    kinds = []
+    for k, side in enumerate(sides):
+        s = Solver()
+        workloads.softbody(s, 7000 + k, max_side=side)
+        o = to_oracle(s, 32, candidate_mode=True)
+        for _ in range(3):
+            assert o.update(1.0 / 60.0) == 0
+        kinds.append((s, state(o)))
+    b = Batch()
+    for k in range(count):
+        b.add_scene(kinds[k % 5][0])
+    b.update(1.0 / 60.0, 3)
+    b.sync()
+    for k in (*range(min(count, 5)), count - 1):
+        out = kinds[k % 5][0].clone()
+        b.read_scene(k, out)
+        assert bits_equal(state(out), kinds[k % 5][1]), f"scene {k}: {first_diff(state(out), kinds[k % 5][1])}"
