@@ -103,9 +103,10 @@ __device__ __forceinline__ float wg_max(float v, float *s_red) {
 // (ROCm's device library: a row-shift and row-broadcast sequence)
 extern "C" __device__ uint32_t __ockl_wfscan_add_u32(uint32_t, bool);
 
-// Exclusive scan in place over a[0..n) in global memory by one workgroup.
+// Exclusive scan of a[0..n) into out[0..n] (out[n] the total) in global memory by
+// one workgroup; out may be a.
 template <int WG>
-__device__ void wg_scan_global(uint32_t *a, uint32_t n, uint32_t *s_wave) {
+__device__ void wg_scan_global(const uint32_t *a, uint32_t *out, uint32_t n, uint32_t *s_wave) {
     uint32_t carry = 0;
     // The wave index is uniform and the lane scan takes no lane masks: the
     // loops over the waves below are scalar loops, and no per-lane compare
@@ -128,11 +129,12 @@ __device__ void wg_scan_global(uint32_t *a, uint32_t n, uint32_t *s_wave) {
         for (uint32_t w = wave; w < WG / 64; w++) total += s_wave[w];
         uint32_t run = carry + woff + inc - local;
         for (int k = 0; k < 4; k++) {
-            if (i0 + k < n) a[i0 + k] = run;
+            if (i0 + k < n) out[i0 + k] = run;
             run += v[k];
         }
         carry += total;
     }
+    if (threadIdx.x == 0) out[n] = carry;
     __syncthreads();
 }
 
@@ -188,11 +190,16 @@ constexpr uint32_t kParkPairs = 32;
 constexpr int kFallbackAttempt = 4;
 // Sweeps after such a fallback that run sequentially without trying lists.
 constexpr uint32_t kFallbackStreak = 16;
-// A list is rebuilt before a sweep once some circle drifted this fraction of
-// its skin from its list-build position (relative to a common shift of the scene):
-// the fraction that a valid sweep may use, so a sweep that pushes nothing
-// needs no check.
+// A circle has drifted once it is further than this fraction of its skin from
+// its list-build position (relative to a common shift of the scene): the
+// fraction that a valid sweep may use.  A list is rebuilt before a sweep when
+// more than kDriftedBase + Nc / kDriftedShare circles have, or one of those has
+// come into reach of a circle it does not list; else the sweep's check looks at
+// each of them on its own.  A few circles shot out of a
+// collider or a pile move by more than any skin every substep, and brought a new
+// list each time (20 to 320 us, against about 1 us a circle for the check).
 constexpr float kDriftRebuild = 0.8f;
+constexpr uint32_t kDriftedBase = 8u, kDriftedShare = 64u;
 
 // FbGrid: bucket heads (u16, tmask + 1 of them, 0xffff for an empty bucket),
 // per-circle next links (u16) and a candidate buffer of cap entries (u16): in
@@ -214,7 +221,7 @@ struct CCShared {
     uint32_t nnear, stalled; // circles beyond their active margins; a list left unfinished
     const uint16_t *act;     // the sweep's active lists (LDS or workspace)
     uint32_t halt;           // the scene's time budget for this launch is spent
-    float4 red4[16];         // the wavefronts' drift boxes (see drift_box)
+    float4 red4[32];         // the wavefronts' drift boxes and sums (see drift_box)
     uint32_t cnt3[3];        // worklist lengths, rotating (see the round loop)
     uint32_t poly_last[2];   // polygon pairs: 1 + the last point of the other polygon that
                              // hit the current edge, two slots used alternately
@@ -238,6 +245,8 @@ struct CCShared {
         float skin;
         uint32_t list_valid, pairs, since_build;
         float s_cell, smin;
+        uint32_t level;   // of the active margins' base (see kActiveBase)
+        uint32_t clean;   // sweeps since a margin was too small
     } cs;
     // statistics of the scene during a launch, written by lane 0 only (in LDS
     // rather than in every lane's registers)
@@ -248,27 +257,31 @@ struct CCShared {
     } cnt;
 };
 
-// minimum over the active lanes of the wavefront (ROCm's device library)
+// minimum and sum over the active lanes of the wavefront (ROCm's device library)
 extern "C" __device__ float __ockl_wfred_min_f32(float);
+extern "C" __device__ float __ockl_wfred_add_f32(float);
 
-// Drift of the circles from their list-build positions: the centre u of the
-// finite displacements' bounding box, and half the box's diagonal, which no
-// displacement is further from u than (infinite when some circle has a finite
-// position but a non-finite list-build one).  Every thread gets the
-// workgroup's result.  Run every substep: the box takes four lane reductions
-// (minima of the bounds and the negated bounds) and one barrier; a mean in
-// place of the centre took nine values through LDS-routed shuffles (640 flying
-// bodies: the sweep phase 2.1 times shorter).  The slots are free again by the
-// next call: barriers lie between.
+// Drift of the circles from their list-build positions: a common shift u of the
+// scene, and a bound no finite displacement is further from u than (infinite
+// when some circle has a finite position but a non-finite list-build one).
+// Every thread gets the workgroup's result.  With MEAN u is the mean
+// displacement: one circle shot out of a pile must not shift all others.
+// Without, u is the centre of the displacements' box, which is enough to see
+// that nobody drifted far, and is asked every substep of a body in flight: the
+// box takes four lane reductions (minima of the bounds and the negated bounds)
+// and one barrier (640 flying bodies: the sweep phase 2.1 times shorter than
+// with nine values through LDS-routed shuffles).  The slots are free again by
+// the next call: barriers lie between.
 struct Drift {
     float ux, uy, box;
 };
 
-template <int WG>
+template <int WG, bool MEAN>
 __device__ __forceinline__ Drift drift_box(const float2 *P, uint32_t Np, uint32_t Nc, const float2 *ref_,
                                            float4 *red4) {
     BD_GLOBAL const uint64_t *const ref = to_global((const uint64_t *)ref_);
     float4 v = make_float4(INFINITY, INFINITY, INFINITY, INFINITY);
+    float sx = 0.0f, sy = 0.0f, n = 0.0f;
 #pragma unroll 2
     for (uint32_t c = threadIdx.x; c < Nc; c += WG) {
         const float2 p = P[Np + c];
@@ -281,6 +294,7 @@ __device__ __forceinline__ Drift drift_box(const float2 *P, uint32_t Np, uint32_
             v.y = fminf(v.y, ok ? -dx : -INFINITY);
             v.z = fminf(v.z, dy);
             v.w = fminf(v.w, -dy);
+            if (MEAN && ok) { sx += dx; sy += dy; n += 1.0f; }
         }
     }
     auto reduce = [&]() {
@@ -288,77 +302,164 @@ __device__ __forceinline__ Drift drift_box(const float2 *P, uint32_t Np, uint32_
         v.y = __ockl_wfred_min_f32(v.y);
         v.z = __ockl_wfred_min_f32(v.z);
         v.w = __ockl_wfred_min_f32(v.w);
+        if constexpr (MEAN) {
+            sx = __ockl_wfred_add_f32(sx);
+            sy = __ockl_wfred_add_f32(sy);
+            n = __ockl_wfred_add_f32(n);
+        }
     };
     reduce();
     if constexpr (WG > 64) {
-        if ((threadIdx.x & 63u) == 0u) red4[threadIdx.x >> 6] = v;
+        const uint32_t lane = threadIdx.x & 63u;
+        if (lane == 0u) {
+            red4[threadIdx.x >> 6] = v;
+            if constexpr (MEAN) red4[16u + (threadIdx.x >> 6)] = make_float4(sx, sy, n, 0.0f);
+        }
         __syncthreads();
-        v = red4[threadIdx.x & (WG / 64u - 1u)];
+        v = red4[lane & (WG / 64u - 1u)];
+        if constexpr (MEAN) {
+            const float4 t = red4[16u + (lane & (WG / 64u - 1u))];
+            const bool once = lane < WG / 64u;  // each wavefront's sums once
+            sx = once ? t.x : 0.0f;
+            sy = once ? t.y : 0.0f;
+            n = once ? t.z : 0.0f;
+        }
         reduce();
     }
     const float x0 = uni(v.x), x1 = -uni(v.y), y0 = uni(v.z), y1 = -uni(v.w);
     if (!(x0 <= x1)) return Drift{0.0f, 0.0f, x0 == INFINITY ? 0.0f : INFINITY};  // no finite circle, or not ok
-    const float bx = 0.5f * (x1 - x0), by = 0.5f * (y1 - y0);
+    float ux = 0.5f * (x0 + x1), uy = 0.5f * (y0 + y1), bx = 0.5f * (x1 - x0), by = 0.5f * (y1 - y0);
+    if constexpr (MEAN) {
+        if (uni(n) > 0.0f) {
+            ux = uni(sx) / uni(n);
+            uy = uni(sy) / uni(n);
+            bx = fmaxf(fabsf(x0 - ux), fabsf(x1 - ux));
+            by = fmaxf(fabsf(y0 - uy), fabsf(y1 - uy));
+        }
+    }
     const float box = sqrtf(bx * bx + by * by);
-    return Drift{0.5f * (x0 + x1), 0.5f * (y0 + y1), box == box ? box : INFINITY};
+    return Drift{ux, uy, box == box ? box : INFINITY};
 }
 
 // An upper bound of the drift as a fraction of the smallest skin, with a margin
 // for the rounding of the box.
 __device__ __forceinline__ float drift_share(float box, float smin) { return (box * 1.0001f) / (smin * 0.9999f); }
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// The candidate grid's buckets.  Cell (x, y) goes to bucket (x + y stride) mod T
+// with stride about 0.618 T: the cells of a row are consecutive buckets, so a row
+// of neighbouring cells is one run of records, and the rows start evenly spread
+// over the table.  Three neighbouring rows of three cells share no bucket
+// (T >= 32: the starts of rows 1 and 2 apart are at least 3 buckets away).  With
+// a hash per cell each of the 9 cells cost two loads and its records a cache line
+// of their own, also where neighbours in space are neighbours in memory.  A list
+// build, in all: 10,000 circles of a soft body 213 -> 91 us, a gas of 16,000
+// 660 -> 318, one of 2,000 with 319 outliers 384 -> 110.
+// T is the power of two at or above the circle count where the counters of that
+// many buckets fit the LDS beside the positions (grid_buckets), else half of it:
+// circles per bucket hardly change the time (its records are one run), counters
+// in LDS do.
+struct CCGrid {
+    uint32_t T, stride, Nc;
+    double inv_h;
+    const uint32_t *start;  // first record of each bucket, start[T] = Nc (workspace)
+};
+
+__device__ __forceinline__ uint32_t grid_buckets(uint32_t Np, uint32_t Nc, uint32_t T) {
+    const uint32_t half = T >> 1;
+    return half >= 32u && 8u * (Np + Nc) + 2u * half > 136u * 1024u ? half >> 1 : half;
+}
+
+__device__ __forceinline__ CCGrid cc_grid(uint32_t Np, uint32_t Nc, uint32_t table, double h, const uint32_t *start) {
+    const uint32_t T = grid_buckets(Np, Nc, table);
+    return CCGrid{T, (uint32_t)((float)T * 0.618034f) | 1u, Nc, 1.0 / h, start};
+}
+
+__device__ __forceinline__ uint32_t grid_bucket(const CCGrid &g, uint32_t cx, uint32_t cy) {
+    return (cx + cy * g.stride) & (g.T - 1u);
+}
+
+// The records of the n cells from (cx, cy) on along its row: first record and
+// count; the run goes on at record 0 after the last one.  start(k) is the first
+// record of bucket k, k <= T.  (Records of other cells in these buckets are among
+// them; with n >= T they are all records.)
+template <typename F>
+__device__ __forceinline__ uint32_t grid_row(const CCGrid &g, uint32_t cx, uint32_t cy, uint32_t n, F start,
+                                             uint32_t &first) {
+    if (n >= g.T) { first = 0u; return g.Nc; }
+    const uint32_t b = grid_bucket(g, cx, cy), e = b + n;
+    const bool wrap = e > g.T;
+    const uint32_t s0 = start(b), s1 = start(wrap ? e - g.T : e);
+    first = s0;
+    return wrap ? g.Nc - s0 + s1 : s1 - s0;
+}
+
+// The buckets' first records: 16-bit in LDS while a list is built (when they
+// fit), and 32-bit in the workspace.
+template <bool LDS>
+struct GridStart;
+template <>
+struct GridStart<true> {
+    BD_LDS const uint16_t *p;
+    __device__ __forceinline__ uint32_t operator()(uint32_t k) const { return p[k]; }
+};
+template <>
+struct GridStart<false> {
+    BD_GLOBAL const uint32_t *p;
+    __device__ __forceinline__ uint32_t operator()(uint32_t k) const { return p[k]; }
+};
+template <bool LDS>
+__device__ __forceinline__ GridStart<LDS> grid_start(const uint32_t *global, uint32_t lds_off) {
+    extern __shared__ float2 s_dyn[];
+    if constexpr (LDS) return {to_lds((const uint16_t *)((const uint8_t *)s_dyn + lds_off))};
+    else return {to_global(global)};
+}
+
 // Candidate pairs are the pairs closer than (r_c + skin_c) + (r_o + skin_o)
 // when the list is built.  A normal circle (skin <= s_cell) finds its normal
-// partners in the 3x3 cells of size h = 2 (r_max + s_cell) around it: the
-// circles sit in hash buckets as 16-byte records, and each distinct bucket of
-// the 9 is scanned once (a record from another cell that hashes there is
-// still a true partner when it passes the distance test, and it is in no
-// other scanned bucket).  An outlier (larger skin) finds all its partners
-// itself and writes itself into its normal partners' lists too, so normal
-// circles never search far.  The first `cap` partners go to out; the count
-// is returned in full.
-__device__ __noinline__ uint32_t gather_normal(uint32_t c, const CCWork &w, float2 p, float ec, double inv_h,
-                                               uint32_t tmask, uint16_t *out, uint32_t cap) {
-    const int cx0 = scell(p.x, inv_h), cy0 = scell(p.y, inv_h);
-    uint32_t kk[9];
-    bool dup[9];
-#pragma unroll
-    for (int i = 0; i < 9; i++) kk[i] = cell_hash(cx0 + (i % 3) - 1, cy0 + (i / 3) - 1) & tmask;
-#pragma unroll
-    for (int i = 0; i < 9; i++) {
-        dup[i] = false;
-#pragma unroll
-        for (int j = 0; j < i; j++) dup[i] = dup[i] || kk[j] == kk[i];
+// partners in the 3x3 cells of size h = 2 (r_max + s_cell) around it: three runs
+// of records (a record from another cell in those buckets is still a true
+// partner when it passes the distance test, and it is in one run only).  An
+// outlier (larger skin) finds all its partners itself and writes itself into its
+// normal partners' lists too, so normal circles never search far.  The first
+// `cap` partners go to out; the count is returned in full.
+template <bool LDS>
+__device__ __noinline__ uint32_t gather_normal(uint32_t c, const CCWork &w, CCGrid g, uint32_t lds_off,
+                                               float2 p, float ec, uint16_t *out_, uint32_t cap) {
+    const GridStart<LDS> start = grid_start<LDS>(w.start, lds_off);
+    BD_GLOBAL const f32x4 *const rec = to_global((const f32x4 *)w.rec);
+    BD_GLOBAL uint16_t *const out = (BD_GLOBAL uint16_t *)(uint64_t)out_;  // (each lane its own)
+    const uint32_t Nc = uni(g.Nc);
+    const uint32_t cx = (uint32_t)scell(p.x, g.inv_h) - 1u, cy = (uint32_t)scell(p.y, g.inv_h);
+    uint32_t s0[3], pre1, pre2, total;
+    if (g.T < 32u) {
+        s0[0] = s0[1] = s0[2] = 0u;
+        pre1 = pre2 = total = Nc;  // a table too small for separate rows: every record
+    } else {
+        pre1 = grid_row(g, cx, cy - 1u, 3u, start, s0[0]);
+        pre2 = pre1 + grid_row(g, cx, cy, 3u, start, s0[1]);
+        total = pre2 + grid_row(g, cx, cy + 1u, 3u, start, s0[2]);
     }
-    // the buckets' record ranges, loaded together, then their records as one
-    // run, kU at a time (a record sits at start + rank in its bucket's range)
-    uint32_t s0[9], pre[10];
-    pre[0] = 0u;
-#pragma unroll
-    for (int i = 0; i < 9; i++) {
-        const uint32_t a = w.start[kk[i]], b = w.start[kk[i] + 1];
-        s0[i] = a;
-        pre[i + 1] = pre[i] + (dup[i] ? 0u : b - a);
-    }
-    const uint32_t total = pre[9];
     constexpr uint32_t kU = 4;
     uint32_t n = 0;
 #pragma unroll 1
     for (uint32_t t0 = 0; t0 < total; t0 += kU) {
-        float4 r[kU];
+        f32x4 r[kU];
 #pragma unroll
         for (uint32_t u = 0; u < kU; u++) {
-            const uint32_t t = t0 + u;
-            uint32_t s = 0;
-#pragma unroll
-            for (int i = 0; i < 9; i++)
-                if (t >= pre[i]) s = s0[i] + (t - pre[i]);
-            r[u] = t < total ? w.rec[s] : make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(c));
+            const uint32_t t = min(t0 + u, total - 1u);
+            uint32_t s = t < pre1 ? s0[0] + t : t < pre2 ? s0[1] + (t - pre1) : s0[2] + (t - pre2);
+            if (s >= Nc) s -= Nc;
+            r[u] = rec[s];
         }
 #pragma unroll
         for (uint32_t u = 0; u < kU; u++) {
             const uint32_t o = __float_as_uint(r[u].w);
-            if (o == c || (o & kOutlierBit)) continue;  // an outlier lists its pairs itself; padding is c
+            // an outlier lists its pairs itself
+            if (t0 + u >= total || o == c || (o & kOutlierBit)) continue;
             float ex = p.x - r[u].x, ey = p.y - r[u].y;
             float lim = ec + r[u].z;
             if (ex * ex + ey * ey < lim * lim) {
@@ -371,19 +472,23 @@ __device__ __noinline__ uint32_t gather_normal(uint32_t c, const CCWork &w, floa
 }
 
 // Outliers' partners.  A near outlier (its normal partners lie within 8
-// cells) has those cells scanned: the (outlier, cell) items of all near
+// cells) has those cells scanned: the (outlier, row of cells) items of all near
 // outliers are spread over the workgroup's threads when the outliers fit one
-// stage, else a wavefront takes one outlier at a time.  A far one is searched
+// stage, else 16 lanes take one outlier at a time.  A far one is searched
 // by the whole workgroup over every circle, and pairs of two outliers by all pairs among
 // the outliers.  An outlier-normal pair is found once, by the outlier, and
 // goes into both lists; an outlier-outlier pair is found once per direction
 // (the test is symmetric) and goes into the first one's list.  MODE 0 counts
 // into cnt, MODE 1 appends at the lists' cursors.  stage: WG / 2 entries of
 // LDS scratch.  Returns the far outliers.
-template <int WG, int MODE>
-__device__ __noinline__ uint32_t gather_outliers(uint32_t Nc, const CCWork &w, const float *crad, const uint16_t *outs,
-                                    uint32_t n_out, float rmax, float s_cell, double h, double inv_h,
-                                    uint32_t tmask, uint32_t *cursor, float4 *stage, uint32_t *s_wave) {
+template <int WG, int MODE, bool LDS>
+__device__ __noinline__ uint32_t gather_outliers(const CCWork &w, CCGrid g, uint32_t lds_off, const float *crad,
+                                    const uint16_t *outs, uint32_t n_out_, float rmax, float s_cell, double h,
+                                    uint32_t *cursor, float4 *stage, uint32_t *s_wave) {
+    const uint32_t n_out = uni(n_out_), Nc = uni(g.Nc);
+    const GridStart<LDS> start = grid_start<LDS>(w.start, lds_off);
+    BD_GLOBAL const f32x4 *const rec = to_global((const f32x4 *)w.rec);
+    const double inv_h = g.inv_h;
     auto add = [&](uint32_t c, uint32_t o) {
         if (MODE == 0) atomicAdd(&w.cnt[c], 1u);
         else w.cand[atomicAdd(&cursor[c], 1u)] = (uint16_t)o;
@@ -402,37 +507,48 @@ __device__ __noinline__ uint32_t gather_outliers(uint32_t Nc, const CCWork &w, c
         __syncthreads();
     };
     const bool one_tile = n_out <= kStage;
-    // the cells a near outlier scans: (2R + 1)^2 around its own, R = ceil(reach)
-    auto near_side = [&](float ec) -> int {
+    // the rows a near outlier scans: 2R + 1 of as many cells, R = ceil(reach)
+    auto near_side = [&](float ec) -> uint32_t {
         const double reach = reach_of(ec);
-        return reach <= 8.0 ? 2 * (int)ceil(reach) + 1 : 0;
+        return reach <= 8.0 ? 2u * (uint32_t)(int)ceil(reach) + 1u : 0u;
     };
-    auto scan_cell = [&](uint32_t c, float2 p, float ec, int cx, int cy) {
-        const uint32_t kk = cell_hash(cx, cy) & tmask;
-#pragma unroll 4
-        for (uint32_t s = w.start[kk], s1 = w.start[kk + 1]; s < s1; s++) {
-            const float4 r = w.rec[s];
-            const uint32_t o = __float_as_uint(r.w);
-            if (o & kOutlierBit) continue;  // outliers: below
-            if (scell(r.x, inv_h) != cx || scell(r.y, inv_h) != cy) continue;  // another cell, same bucket
-            float ex = p.x - r.x, ey = p.y - r.y;
-            float lim = ec + r.z;
-            if (ex * ex + ey * ey < lim * lim) { add(c, o); add(o, c); }
+    // row q of the outlier's cells
+    auto scan_row = [&](uint32_t c, float2 p, float ec, uint32_t side, uint32_t q) {
+        const uint32_t cx = (uint32_t)scell(p.x, inv_h) - (side >> 1), cy = (uint32_t)scell(p.y, inv_h) - (side >> 1) + q;
+        uint32_t s0;
+        const uint32_t len = grid_row(g, cx, cy, side, start, s0);
+        constexpr uint32_t kU = 4;
+#pragma unroll 1
+        for (uint32_t t0 = 0; t0 < len; t0 += kU) {
+            f32x4 r[kU];
+#pragma unroll
+            for (uint32_t u = 0; u < kU; u++) {
+                uint32_t s = s0 + min(t0 + u, len - 1u);
+                if (s >= Nc) s -= Nc;
+                r[u] = rec[s];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kU; u++) {
+                const uint32_t o = __float_as_uint(r[u].w);
+                float ex = p.x - r[u].x, ey = p.y - r[u].y;
+                float lim = ec + r[u].z;
+                if (t0 + u >= len || (o & kOutlierBit) || !(ex * ex + ey * ey < lim * lim)) continue;  // outliers: below
+                // found in the row of its own cell only (other rows may hold the same buckets)
+                if ((uint32_t)scell(r[u].y, inv_h) != cy || (uint32_t)scell(r[u].x, inv_h) - cx >= side) continue;
+                add(c, o);
+                add(o, c);
+            }
         }
     };
     if (one_tile && n_out) {
         stage_tile(0u, n_out);
-        // every (near outlier, cell) item across the workgroup: each outlier's
-        // first item (an exclusive prefix over the outliers' cell counts) goes
+        // every (near outlier, row) item across the workgroup: each outlier's
+        // first item (an exclusive prefix over the outliers' row counts) goes
         // in its stage entry's w, and a thread takes a contiguous run of items,
         // finding its first outlier by bisection
         const uint32_t t = threadIdx.x;
-        uint32_t cells = 0;
-        if (t < n_out) {
-            const int side = near_side(stage[t].z);
-            cells = (uint32_t)(side * side);
-        }
-        const uint32_t inc = __ockl_wfscan_add_u32(cells, true);
+        const uint32_t rows = t < n_out ? near_side(stage[t].z) : 0u;
+        const uint32_t inc = __ockl_wfscan_add_u32(rows, true);
         if (lane == 63u) s_wave[wave] = inc;
         __syncthreads();
         const uint32_t uw = uni(wave);
@@ -442,14 +558,14 @@ __device__ __noinline__ uint32_t gather_outliers(uint32_t Nc, const CCWork &w, c
         items = below;
 #pragma unroll 1
         for (uint32_t v = uw; v < WG / 64; v++) items += s_wave[v];
-        if (t < n_out) stage[t].w = __uint_as_float(below + inc - cells);
+        if (t < n_out) stage[t].w = __uint_as_float(below + inc - rows);
         __syncthreads();
         const uint32_t per = (items + WG - 1) / WG;
         uint32_t i = t * per;
         const uint32_t i1 = min(items, i + per);
         if (i < i1) {
             // the last outlier whose first item is at or before i (one with no
-            // cells shares its first item with the next, and is passed over)
+            // rows shares its first item with the next, and is passed over)
             uint32_t lo = 0, hi = n_out;
             while (hi - lo > 1u) {
                 const uint32_t mid = (lo + hi) >> 1;
@@ -457,54 +573,50 @@ __device__ __noinline__ uint32_t gather_outliers(uint32_t Nc, const CCWork &w, c
             }
             uint32_t k = lo;
             float4 e = stage[k];
-            int side = near_side(e.z);
-            uint32_t q = i - __float_as_uint(e.w);
+            uint32_t side = near_side(e.z), q = i - __float_as_uint(e.w);
 #pragma unroll 1
             for (; i < i1; i++) {
-                if (q == (uint32_t)(side * side)) {
-                    // the next outlier with cells
+                if (q == side) {
+                    // the next outlier with rows
                     do {
                         e = stage[++k];
                         side = near_side(e.z);
-                    } while (side == 0 && k + 1u < n_out);
+                    } while (side == 0u && k + 1u < n_out);
                     q = 0;
                 }
-                const float2 p = make_float2(e.x, e.y);
-                const int R = side >> 1;
-                const int cx = scell(p.x, inv_h) + (int)(q % (uint32_t)side) - R;
-                const int cy = scell(p.y, inv_h) + (int)(q / (uint32_t)side) - R;
-                scan_cell(outs[k], p, e.z, cx, cy);
+                scan_row(outs[k], make_float2(e.x, e.y), e.z, side, q);
                 q++;
             }
         }
     }
-    // more outliers than one stage holds: a wavefront per outlier, its lanes
-    // over the cells
-    for (uint32_t k = wave; k < n_out && !one_tile; k += WG / 64) {
+    // more outliers than one stage holds: 16 lanes an outlier, over its rows
+    for (uint32_t k = threadIdx.x >> 4; k < n_out && !one_tile; k += WG / 16) {
         const uint32_t c = outs[k];
-        const float2 p = w.ref[c];
         const float ec = crad[c] + w.skin[c];
-        const int side = near_side(ec);
-        if (side == 0) continue;
-        const int R = side >> 1;
-        const int cx0 = scell(p.x, inv_h), cy0 = scell(p.y, inv_h);
-        for (int q = (int)lane; q < side * side; q += 64)
-            scan_cell(c, p, ec, cx0 + (q % side) - R, cy0 + (q / side) - R);
+        const uint32_t side = near_side(ec);
+        for (uint32_t q = lane & 15u; q < side; q += 16u) scan_row(c, w.ref[c], ec, side, q);
     }
     uint32_t n_far = 0;
-    for (uint32_t k = 0; k < n_out; k++) {
-        const uint32_t c = outs[k];
-        const float ec = crad[c] + w.skin[c];
-        if (reach_of(ec) <= 8.0) continue;
-        n_far++;
-        const float2 p = w.ref[c];
-        for (uint32_t s = threadIdx.x; s < Nc; s += WG) {
-            const float4 r = w.rec[s];
-            const uint32_t o = __float_as_uint(r.w);
-            if (o & kOutlierBit) continue;
-            float ex = p.x - r.x, ey = p.y - r.y;
-            float lim = ec + r.z;
-            if (ex * ex + ey * ey < lim * lim) { add(c, o); add(o, c); }
+    // every wavefront finds the far ones, 64 outliers at a time (one after the
+    // other they cost a dependent load and a division each: 0.4 us, for each of
+    // up to kOutCap outliers and twice a list)
+    for (uint32_t k0 = 0; k0 < n_out; k0 += 64u) {
+        const uint32_t k = k0 + lane;
+        bool is_far = false;
+        if (k < n_out) is_far = near_side(one_tile ? stage[k].z : crad[outs[k]] + w.skin[outs[k]]) == 0u;
+        for (uint64_t m = __ballot(is_far); m; m &= m - 1u) {
+            n_far++;
+            const uint32_t c = uni((uint32_t)outs[k0 + (uint32_t)__ffsll((unsigned long long)m) - 1u]);
+            const float2 p = w.ref[c];
+            const float ec = crad[c] + w.skin[c];
+            for (uint32_t s = threadIdx.x; s < Nc; s += WG) {
+                const float4 r = w.rec[s];
+                const uint32_t o = __float_as_uint(r.w);
+                if (o & kOutlierBit) continue;
+                float ex = p.x - r.x, ey = p.y - r.y;
+                float lim = ec + r.z;
+                if (ex * ex + ey * ey < lim * lim) { add(c, o); add(o, c); }
+            }
         }
     }
     // outlier pairs: a wavefront takes outlier a, its lanes the staged ones
@@ -609,6 +721,18 @@ __device__ __forceinline__ uint32_t list_rank(const CCWork &w, const uint16_t *a
     return lo;
 }
 
+// Whether x is in c's candidate list.
+__device__ __forceinline__ bool is_candidate(const CCWork &w, uint32_t c, uint32_t x) {
+    const uint16_t *my = w.cand + w.off[c];
+    uint32_t lo = 0, hi = w.cnt[c];
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1, v = my[mid];
+        if (v == x) return true;
+        if (v < x) lo = mid + 1; else hi = mid;
+    }
+    return false;
+}
+
 // Whether the pair (c, x), missing from the active lists, would have
 // overlapped when the reference tests it.  Its turn comes after the pairs of
 // c with smaller partners and those of x with smaller partners (the
@@ -635,23 +759,29 @@ __device__ __forceinline__ bool missed_pair_touches(const CCWork &w, const uint1
 }
 
 // A sweep in which some circles moved further than 0.8 of their skins is
-// still exact when no pair missing from the list touched at its turn.  Pairs
+// still exact when no pair missing from the lists touched at its turn.  Pairs
 // of two circles within their skins stayed apart by construction; this looks
 // at every pair with a circle beyond its skin (`over`, with -v in vb; the
 // others hold v <= vmax, v being a circle's bound on its distance from its
-// list-build position, relative to the scene shift, over the whole sweep).
-// A pair whose list-build positions are more than r_c + r_x + v_c + v_x apart
-// stayed apart; the rest get the exact test above.
+// list-build position, relative to the common shift u, over the whole sweep).
+// During the sweep such a circle c was within path_c of its start, and a circle
+// x within its skin within v_x of where it was listed, shifted by u: if the two
+// are more than r_c + r_x + path_c + v_x apart there, they stayed apart; the
+// rest get the exact test above.  So only the cells around c's start are
+// searched, however far c has come since the list was built.
 //
 // With few overruns (at most kOutCap, listed in LDS) pairs of two overrun
 // circles are tested all against all and the grid scan skips them; with more
-// (listed in the workspace) the grid scan covers them too, vmax then being
+// (listed in the workspace; only right after a list build, when every circle's
+// start is its listed position) the grid scan covers them too, vmax then being
 // the largest bound of any circle, and a pair of two overruns is tested from
 // both ends.
 template <int WG, typename Idx>
 __device__ __noinline__ int overruns_check(const CCWork &w, const uint16_t *act, const float *crad, const float *vb, const Idx *over,
-                              uint32_t n_over, float vmax, float rmax, double h, double inv_h, uint32_t tmask,
+                              uint32_t n_over, float vmax, float2 u, float rmax, double h, CCGrid g,
                               float *s_red, bool scan_overruns) {
+    const GridStart<false> start{to_global(g.start)};
+    const uint32_t Nc = uni(g.Nc);
     // rounding margin: a fifth of the overrun circle's skin (the margin the
     // skin test leaves too) plus about 80 ulps of the coordinates
     auto margin = [&](float2 p, float sk) { return 0.2f * sk + 1e-5f * (fabsf(p.x) + fabsf(p.y) + 1.0f); };
@@ -660,19 +790,22 @@ __device__ __noinline__ int overruns_check(const CCWork &w, const uint16_t *act,
         return !(sqrtf(dx * dx + dy * dy) <= lim);  // NaN: a non-finite circle touches nothing
     };
     float bad = 0.0f, far = 0.0f;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    for (uint32_t k = wave; k < n_over; k += WG / 64) {
+    // 16 lanes a circle, over the rows of its cells
+    for (uint32_t k = threadIdx.x >> 4; k < n_over; k += WG / 16) {
         const uint32_t c = over[k];
-        const float2 p = w.ref[c];
-        const float rc = crad[c], vc = -vb[c], mc = margin(p, w.skin[c]);
+        float2 p = w.save[c];
+        if (!(fabsf(p.x) <= 3.0e38f) || !(fabsf(p.y) <= 3.0e38f)) continue;  // touches nothing
+        p.x = p.x - u.x; p.y = p.y - u.y;
+        const float rc = crad[c], vc = w.path[c], mc = margin(p, fminf(w.skin[c], rmax)) + 1e-5f * (fabsf(u.x) + fabsf(u.y));
         const double reach = ((double)rc + (double)vc + (double)mc + (double)rmax + (double)vmax) / h;
         if (!(reach <= 8.0)) { far = 1.0f; continue; }
-        const int R = (int)ceil(reach), side = 2 * R + 1;
-        const int cx0 = scell(p.x, inv_h), cy0 = scell(p.y, inv_h);
-        for (int q = (int)lane; q < side * side; q += 64) {
-            const uint32_t kk = cell_hash(cx0 + (q % side) - R, cy0 + (q / side) - R) & tmask;
-            for (uint32_t s = w.start[kk], s1 = w.start[kk + 1]; s < s1; s++) {
-                const float4 r = w.rec[s];
+        const uint32_t R = (uint32_t)(int)ceil(reach), side = 2u * R + 1u;
+        const uint32_t cx = (uint32_t)scell(p.x, g.inv_h) - R, cy = (uint32_t)scell(p.y, g.inv_h) - R;
+        for (uint32_t q = threadIdx.x & 15u; q < side; q += 16u) {
+            uint32_t s0;
+            const uint32_t len = grid_row(g, cx, cy + q, side, start, s0);
+            for (uint32_t t = 0; t < len; t++) {
+                const float4 r = w.rec[s0 + t < Nc ? s0 + t : s0 + t - Nc];
                 const uint32_t x = __float_as_uint(r.w) & ~kOutlierBit;
                 float vx = vb[x];
                 if (x == c) continue;
@@ -681,7 +814,7 @@ __device__ __noinline__ int overruns_check(const CCWork &w, const uint16_t *act,
                     vx = -vx;
                 }
                 if (apart(p, make_float2(r.x, r.y), ((rc + crad[x]) + (vc + vx)) + mc)) continue;
-                if (missed_pair_touches(w, act, crad, c, x)) bad = 1.0f;
+                if (missed_pair_touches(w, act, crad, c, x)) bad = fmaxf(bad, is_candidate(w, c, x) ? 1.0f : 2.0f);
             }
         }
     }
@@ -690,14 +823,14 @@ __device__ __noinline__ int overruns_check(const CCWork &w, const uint16_t *act,
         const uint32_t a = q / n_over, b = q - a * n_over;
         if (a >= b) continue;
         const uint32_t c = over[a], o = over[b];
-        const float2 p = w.ref[c];
-        const float lim = ((crad[c] + crad[o]) + (-vb[c] - vb[o])) + margin(p, w.skin[c] + w.skin[o]);
-        if (apart(p, w.ref[o], lim)) continue;
-        if (missed_pair_touches(w, act, crad, c, o)) bad = 1.0f;
+        const float lim = ((crad[c] + crad[o]) + (w.path[c] + w.path[o])) * (1.0f + 0x1p-16f);
+        if (apart(w.save[c], w.save[o], lim)) continue;
+        if (missed_pair_touches(w, act, crad, c, o)) bad = fmaxf(bad, is_candidate(w, c, o) ? 1.0f : 2.0f);
     }
-    // 0: every missing pair stayed apart; 1: one touched; 2: an overrun too
-    // far to search (the sweep is redone without knowing)
-    return (int)wg_max<WG>(fmaxf(bad, 2.0f * far), s_red);
+    // 0: every missing pair stayed apart; 1: one touched, but only candidates
+    // that the active lists left out; 2: one that the candidate lists do not
+    // hold; 3: an overrun too far to search (the sweep is redone without knowing)
+    return (int)wg_max<WG>(fmaxf(bad, 3.0f * far), s_red);
 }
 
 // A sweep in which some circles (near, listed in fill) moved further than 0.8 of
@@ -724,6 +857,46 @@ __device__ __noinline__ int near_check(const CCWork &w, const uint16_t *act, con
         }
     }
     return (int)wg_max<WG>(bad, s_red);
+}
+
+// Whether one of the circles that drifted beyond their skins (`over`, nd of them,
+// with -v in vb; the others hold v <= vmax) is now, before the sweep, in reach of
+// a circle that its candidate list does not hold, reach being that of the active
+// lists (radii and margins).  Such a pair would most likely touch and cost a
+// second run of the sweep; a new list beforehand costs less.
+template <int WG>
+__device__ __noinline__ bool drifted_meet(const float2 *P, uint32_t Np, const CCWork &w, const float *crad,
+                                          const float *vb, const uint16_t *over, uint32_t nd, float vmax, float2 u,
+                                          float mbase, float rmax, double h, CCGrid g, float *s_red) {
+    const GridStart<false> start{to_global(g.start)};
+    const uint32_t Nc = uni(g.Nc), lane = threadIdx.x & 15u;
+    float met = 0.0f;
+    auto meets = [&](uint32_t c, float2 p, float ec, uint32_t x) {
+        const float2 q = P[Np + x];
+        const float dx = p.x - q.x, dy = p.y - q.y, lim = ec + (crad[x] + fmaxf(mbase, w.need[x]));
+        return dx * dx + dy * dy < lim * lim && !is_candidate(w, c, x);
+    };
+    for (uint32_t k = threadIdx.x >> 4; k < nd; k += WG / 16) {
+        const uint32_t c = over[k];
+        const float2 p = P[Np + c];
+        const float mc = fmaxf(mbase, w.need[c]), ec = crad[c] + mc;
+        const float2 pu = make_float2(p.x - u.x, p.y - u.y);
+        const double reach = ((double)ec + (double)rmax + (double)mbase + (double)vmax) / h;
+        if (!(reach <= 8.0)) { met = 1.0f; continue; }
+        const uint32_t R = (uint32_t)(int)ceil(reach), side = 2u * R + 1u;
+        const uint32_t cx = (uint32_t)scell(pu.x, g.inv_h) - R, cy = (uint32_t)scell(pu.y, g.inv_h) - R;
+        for (uint32_t q = lane; q < side; q += 16u) {
+            uint32_t s0;
+            const uint32_t len = grid_row(g, cx, cy + q, side, start, s0);
+            for (uint32_t t = 0; t < len; t++) {
+                const uint32_t x = __float_as_uint(w.rec[s0 + t < Nc ? s0 + t : s0 + t - Nc].w) & ~kOutlierBit;
+                if (x != c && vb[x] >= 0.0f && meets(c, p, ec, x)) met = 1.0f;
+            }
+        }
+        for (uint32_t j = lane; j < nd; j += 16u)
+            if (j != k && meets(c, p, ec, over[j])) met = 1.0f;
+    }
+    return wg_max<WG>(met, s_red) > 0.0f;
 }
 
 // Sequential fallback of the circle-pair sweep, for a sweep whose candidate
@@ -1043,7 +1216,14 @@ __device__ __forceinline__ void fallback_sweep(float2 *P, uint32_t Np, uint32_t 
 // key[c] get list c's place and length, st[c] its round state (see rounds_core).
 // Returns the slots used; with more than cap of them nothing past cap is
 // written, and the caller chooses another place.
-constexpr float kActiveBase = 0.05f;  // base margin, in units of the largest radius
+// The base margin, in units of the largest radius, at level 0; each level
+// doubles it.  A sweep that had to run again because a pair touched beyond the
+// margins raises the scene's level by two, kLevelClean sweeps without one lower it: a
+// settling pile stays at level 0 (its rounds grow with the margins), a hot gas,
+// whose first contacts push circles by most of a radius, at the top (its rounds
+// are few: 16,000 circles ran every sweep twice at level 0).
+constexpr float kActiveBase = 0.05f;
+constexpr uint32_t kLevels = 4u, kLevelClean = 16u;
 constexpr uint32_t kCurMask = 0x00ffffffu;
 constexpr uint32_t kStamp8 = 0xffu;
 static_assert(kCandCap * 65536ull <= kCurMask + 1ull, "a list cursor must fit 24 bits");
@@ -1487,6 +1667,95 @@ __device__ __noinline__ uint32_t sort_lists(uint32_t Nc_, CCShared *sh, float *s
     return (uint32_t)wg_max<WG>((float)longest, s_red);
 }
 
+// The circles' records in bucket order (rec, start), their positions now in ref.
+// The counters are in LDS: 16 bits each, two to a word, so a circle's rank in its
+// bucket comes back from the count itself (kept with the bucket in key).
+template <int WG>
+__device__ __noinline__ void grid_in_lds(const float2 *P, uint32_t Np_, const float *crad, CCGrid g, float s_cell,
+                                         uint32_t lds_off_, const CCWork &w, uint32_t *s_wave) {
+    extern __shared__ float2 s_dyn[];
+    const uint32_t tid = threadIdx.x, Np = uni(Np_), Nc = uni(g.Nc), T = uni(g.T);
+    BD_LDS uint32_t *const word = to_lds((uint32_t *)((uint8_t *)s_dyn + uni(lds_off_)));
+    BD_LDS uint16_t *const half = (BD_LDS uint16_t *)word;
+    BD_GLOBAL u32x2 *const start = to_global((u32x2 *)w.start);
+    BD_GLOBAL f32x2 *const ref = to_global((f32x2 *)w.ref);
+    BD_GLOBAL uint32_t *const key = to_global(w.key);
+    BD_GLOBAL const float *const skin = to_global((const float *)w.skin), *const rad = to_global(crad);
+    BD_GLOBAL f32x4 *const rec = to_global((f32x4 *)w.rec);
+    const uint32_t words = T >> 1;  // (T is even)
+    for (uint32_t b = tid; b < words; b += WG) word[b] = 0u;
+    __syncthreads();
+#pragma unroll 2
+    for (uint32_t c = tid; c < Nc; c += WG) {
+        const float2 p = P[Np + c];
+        ref[c] = f32x2{p.x, p.y};
+        const uint32_t kk = grid_bucket(g, (uint32_t)scell(p.x, g.inv_h), (uint32_t)scell(p.y, g.inv_h));
+        const uint32_t sft = (kk & 1u) * 16u;
+        const uint32_t old = __hip_atomic_fetch_add(word + (kk >> 1), 1u << sft, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        key[c] = kk | ((old >> sft) & 0xffffu) << 16;
+    }
+    __syncthreads();
+    // exclusive scan: a lane takes a run of words
+    const uint32_t per = (words + WG - 1u) / WG, w0 = min(words, tid * per), w1 = min(words, w0 + per);
+    uint32_t sum = 0;
+    for (uint32_t i = w0; i < w1; i++) {
+        const uint32_t v = word[i];
+        sum += (v & 0xffffu) + (v >> 16);
+    }
+    const uint32_t inc = __ockl_wfscan_add_u32(sum, true), wave = uni(tid >> 6);
+    if ((tid & 63u) == 63u) s_wave[wave] = inc;
+    __syncthreads();
+    uint32_t run = inc - sum;
+#pragma unroll 1
+    for (uint32_t v = 0; v < wave; v++) run += s_wave[v];
+    for (uint32_t i = w0; i < w1; i++) {
+        const uint32_t v = word[i], mid = run + (v & 0xffffu);
+        word[i] = run | mid << 16;
+        start[i] = u32x2{run, mid};
+        run = mid + (v >> 16);
+    }
+    if (tid == 0) {
+        half[T] = (uint16_t)Nc;
+        w.start[T] = Nc;
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (uint32_t c = tid; c < Nc; c += WG) {
+        const uint32_t k = key[c];
+        const f32x2 p = ref[c];
+        const float sk = skin[c];
+        rec[half[k & 0xffffu] + (k >> 16)] =
+            f32x4{p.x, p.y, rad[c] + sk, __uint_as_float(c | (sk > s_cell ? kOutlierBit : 0u))};
+    }
+    __syncthreads();
+}
+
+// The same with the counters in the workspace (start, fill).
+template <int WG>
+__device__ __noinline__ void grid_in_memory(const float2 *P, uint32_t Np_, const float *crad, CCGrid g,
+                                            float s_cell, const CCWork &w, uint32_t *s_wave) {
+    const uint32_t tid = threadIdx.x, Np = uni(Np_), Nc = uni(g.Nc), T = uni(g.T);
+    for (uint32_t b = tid; b < T; b += WG) { w.start[b] = 0u; w.fill[b] = 0u; }
+    __syncthreads();
+    for (uint32_t c = tid; c < Nc; c += WG) {
+        const float2 p = P[Np + c];
+        w.ref[c] = p;
+        const uint32_t kk = grid_bucket(g, (uint32_t)scell(p.x, g.inv_h), (uint32_t)scell(p.y, g.inv_h));
+        w.key[c] = kk;
+        atomicAdd(&w.start[kk], 1u);
+    }
+    __syncthreads();
+    wg_scan_global<WG>(w.start, w.start, T, s_wave);  // bucket k = [start[k], start[k+1])
+    for (uint32_t c = tid; c < Nc; c += WG) {
+        const uint32_t kk = w.key[c];
+        const float2 p = w.ref[c];
+        const float sk = w.skin[c];
+        w.rec[w.start[kk] + atomicAdd(&w.fill[kk], 1u)] =
+            make_float4(p.x, p.y, crad[c] + sk, __uint_as_float(c | (sk > s_cell ? kOutlierBit : 0u)));
+    }
+    __syncthreads();
+}
+
 // A new candidate list for the circles where they are now.  The schedule's state
 // (skins, thresholds, pair count) goes to cs.  Returns 0, 1 when the list does
 // not fit the workspace (the skins have been reduced: try again), 2 when not
@@ -1498,7 +1767,6 @@ __device__ __noinline__ uint32_t build_lists(const float2 *P, uint32_t Np_, uint
     const int tid = threadIdx.x;
     const uint32_t Np = uni(Np_), Nc = uni(Nc_), T = uni(T_);
     const float rmax = uni(rmax_);
-    const uint32_t tmask = T - 1;
     const CCWork &w = sh->work;
     float sbase = uni(sh->cs.skin);
     const uint32_t since_build = uni(sh->cs.since_build);
@@ -1515,9 +1783,8 @@ __device__ __noinline__ uint32_t build_lists(const float2 *P, uint32_t Np_, uint
         w.skin[c] = sk;
         smax = fmaxf(smax, sk);
         nsmin = fmaxf(nsmin, -sk);
-        int b = 0;
-        if (sk > sbase) b = sk <= 3.0e38f ? min(32, 1 + (int)floorf(log2f(sk / sbase))) : 32;
-        atomicAdd(&sh->hist[b], 1u);
+        if (sk > sbase)
+            atomicAdd(&sh->hist[sk <= 3.0e38f ? min(32, 1 + (int)floorf(log2f(sk / sbase))) : 32], 1u);
     }
     smax = wg_max<WG>(smax, s_red);
     const float smin = -wg_max<WG>(nsmin, s_red);
@@ -1537,49 +1804,39 @@ __device__ __noinline__ uint32_t build_lists(const float2 *P, uint32_t Np_, uint
     __syncthreads();
     const uint32_t n_out = uni(sh->nout);
     const double h = cell_size(rmax, s_cell);
-    const double inv_h = 1.0 / h;
-    for (uint32_t b = tid; b <= T; b += WG) w.start[b] = 0u;
-    for (uint32_t b = tid; b < T; b += WG) w.fill[b] = 0u;
-    __syncthreads();
-    for (uint32_t c = tid; c < Nc; c += WG) {
-        float2 p = P[Np + c];
-        w.ref[c] = p;
-        uint32_t kk = cell_hash(scell(p.x, inv_h), scell(p.y, inv_h)) & tmask;
-        w.key[c] = kk;
-        atomicAdd(&w.start[kk], 1u);
-    }
-    __syncthreads();
-    wg_scan_global<WG>(w.start, T + 1, s_u32);  // bucket k = [start[k], start[k+1])
-    for (uint32_t c = tid; c < Nc; c += WG) {
-        uint32_t kk = w.key[c];
-        float2 p = w.ref[c];
-        float sk = w.skin[c];
-        w.rec[w.start[kk] + atomicAdd(&w.fill[kk], 1u)] =
-            make_float4(p.x, p.y, crad[c] + sk, __uint_as_float(c | (sk > s_cell ? kOutlierBit : 0u)));
-    }
-    __syncthreads();
+    const CCGrid g = cc_grid(Np, Nc, T, h, w.start);
+    const uint32_t lds_off = sh->free_off;
+    // the buckets' counters in the free LDS when they fit (two to a word, and one
+    // more for the end)
+    const bool in_lds = 2u * g.T + 4u <= sh->free_bytes && Nc < 65536u;
+    if (in_lds) grid_in_lds<WG>(P, Np, crad, g, s_cell, lds_off, w, s_u32);
+    else grid_in_memory<WG>(P, Np, crad, g, s_cell, w, s_u32);
     // counts: normal circles gather their normal partners into a slot of
     // kSlot entries (in traj, free until the sweep) and keep the count in
     // stamp; then outliers add themselves to their partners' counts
     uint16_t *const slot = (uint16_t *)w.traj;
+    auto gather = [&](uint32_t c, uint16_t *out, uint32_t cap) {
+        const float2 p = w.ref[c];
+        const float ec = crad[c] + w.skin[c];
+        return in_lds ? gather_normal<true>(c, w, g, lds_off, p, ec, out, cap)
+                      : gather_normal<false>(c, w, g, lds_off, p, ec, out, cap);
+    };
     for (uint32_t c = tid; c < Nc; c += WG) {
-        const float sk = w.skin[c];
-        uint32_t n = sk > s_cell ? 0u
-                                 : gather_normal(c, w, w.ref[c], crad[c] + sk, inv_h, tmask,
-                                                 slot + (size_t)c * kSlot, kSlot);
+        const uint32_t n = w.skin[c] > s_cell ? 0u : gather(c, slot + (size_t)c * kSlot, kSlot);
         w.cnt[c] = n;
         w.stamp[c] = n;
     }
     __syncthreads();
-    const uint32_t n_far =
-        gather_outliers<WG, 0>(Nc, w, crad, sh->out, n_out, rmax, s_cell, h, inv_h, tmask, nullptr,
-                              (float4 *)s_wl, s_u32);
-    __syncthreads();
+    uint32_t n_far = 0u;
+    if (n_out) {
+        n_far = in_lds ? gather_outliers<WG, 0, true>(w, g, lds_off, crad, sh->out, n_out, rmax, s_cell, h, nullptr,
+                                                      (float4 *)s_wl, s_u32)
+                       : gather_outliers<WG, 0, false>(w, g, lds_off, crad, sh->out, n_out, rmax, s_cell, h, nullptr,
+                                                       (float4 *)s_wl, s_u32);
+        __syncthreads();
+    }
     const uint64_t tb1 = wall_clock64();
-    for (uint32_t c = tid; c < Nc; c += WG) w.off[c] = w.cnt[c];
-    if (tid == 0) w.off[Nc] = 0u;
-    __syncthreads();
-    wg_scan_global<WG>(w.off, Nc + 1, s_u32);
+    wg_scan_global<WG>(w.cnt, w.off, Nc, s_u32);
     const uint32_t total = uni(w.off[Nc]);
     // (one slot a circle stays for the active lists' terminators)
     if (total > (kCandCap - 1u) * Nc) {
@@ -1600,24 +1857,29 @@ __device__ __noinline__ uint32_t build_lists(const float2 *P, uint32_t Np_, uint
     // lists: normal partners first (from the slot, or gathered again when
     // they did not fit it), outliers append at a cursor (in head)
     for (uint32_t c = tid; c < Nc; c += WG) {
-        const float sk = w.skin[c];
         uint32_t own = 0;
-        if (sk <= s_cell) {
+        if (w.skin[c] <= s_cell) {
             own = w.stamp[c];
             uint16_t *dst = w.cand + w.off[c];
             if (own <= kSlot) {
                 const uint16_t *src = slot + (size_t)c * kSlot;
                 for (uint32_t i = 0; i < own; i++) dst[i] = src[i];
             } else {
-                gather_normal(c, w, w.ref[c], crad[c] + sk, inv_h, tmask, dst, own);
+                gather(c, dst, own);
             }
         }
         w.head[c] = w.off[c] + own;
     }
     __syncthreads();
-    gather_outliers<WG, 1>(Nc, w, crad, sh->out, n_out, rmax, s_cell, h, inv_h, tmask, w.head, (float4 *)s_wl,
-                           s_u32);
-    __syncthreads();
+    if (n_out) {
+        if (in_lds)
+            gather_outliers<WG, 1, true>(w, g, lds_off, crad, sh->out, n_out, rmax, s_cell, h, w.head, (float4 *)s_wl,
+                                         s_u32);
+        else
+            gather_outliers<WG, 1, false>(w, g, lds_off, crad, sh->out, n_out, rmax, s_cell, h, w.head, (float4 *)s_wl,
+                                          s_u32);
+        __syncthreads();
+    }
     const uint64_t tb2 = wall_clock64();
     const uint32_t max_list = uni(sort_lists<WG>(Nc, sh, s_red));
     // base skin: rebuilds every few sweeps cost more than larger lists
@@ -1625,7 +1887,7 @@ __device__ __noinline__ uint32_t build_lists(const float2 *P, uint32_t Np_, uint
     else if (since_build > 32) sbase = fmaxf(0.8f * sbase, 0.05f * fmaxf(rmax, 1e-3f));
     const uint64_t tb3 = wall_clock64();
     if (tid == 0) {
-        sh->cs = CCShared::Steer{sbase, 1u, total / 2, 0u, s_cell, smin};
+        sh->cs = CCShared::Steer{sbase, 1u, total / 2, 0u, s_cell, smin, sh->cs.level, sh->cs.clean};
         sh->cnt.n_out = n_out;
         sh->cnt.n_far = n_far;
         sh->cnt.smax = smax;
@@ -1664,7 +1926,6 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
     const uint32_t Np = uni(Np_), Nc = uni(Nc_), T = uni(T_);
     const bool uni_r = uni((uint32_t)uni_r_) != 0u;
     const float runi = uni(runi_), rmax = uni(rmax_);
-    const uint32_t tmask = T - 1;
     const CCWork &w = sh->work;
     CCShared::Steer &cs = sh->cs;  // written by lane 0, read after a barrier
     uint32_t widen = 0u;  // attempts of this sweep that left a touching pair out of the active lists
@@ -1679,27 +1940,45 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
             __syncthreads();
             return 0u;
         }
+        const float mbase = kActiveBase * (float)(1u << uni(cs.level)) * fmaxf(rmax, 1e-3f);
         bool rebuild = uni(cs.list_valid) == 0u;
+        uint32_t drifted = 0u;  // circles beyond their skins before the sweep
         float2 u = make_float2(0.0f, 0.0f);
         if (!rebuild) {
             // drift since the list was built, relative to a common shift u, as a
             // fraction of each circle's skin (at most box / smallest skin, with
             // a margin for rounding, when the displacements' bounding box is
             // small; else each circle is measured)
-            const Drift dr = drift_box<WG>(P, Np, Nc, w.ref, sh->red4);
+            const Drift dr = drift_box<WG, true>(P, Np, Nc, w.ref, sh->red4);
             u = make_float2(dr.ux, dr.uy);
-            float drift = drift_share(dr.box, uni(cs.smin));
-            if (drift < INFINITY && !(drift <= kDriftRebuild)) {
-                float m = 0.0f;
-#pragma unroll 4
-                for (uint32_t c = tid; c < Nc; c += WG)
-                    m = fmaxf(m, moved_bound(P[Np + c], w.ref[c], u, 0.0f) / w.skin[c]);
-                drift = wg_max<WG>(m, s_red);
+            if (!(drift_share(dr.box, uni(cs.smin)) <= kDriftRebuild)) {
+                if (tid == 0) sh->nout = 0u;
+                __syncthreads();
+                float *vb = (float *)w.stamp;
+                float vmax = 0.0f;
+                for (uint32_t c = tid; c < Nc; c += WG) {
+                    const float v = moved_bound(P[Np + c], w.ref[c], u, 0.0f);
+                    const bool in = v <= kDriftRebuild * w.skin[c];
+                    vb[c] = in ? v : -v;
+                    if (in) {
+                        vmax = fmaxf(vmax, v);
+                    } else {
+                        const uint32_t k = atomicAdd(&sh->nout, 1u);
+                        if (k < kOutCap) sh->out[k] = (uint16_t)c;
+                    }
+                }
+                vmax = wg_max<WG>(vmax, s_red);
+                drifted = uni(sh->nout);
+                rebuild = drifted > min(kDriftedBase + Nc / kDriftedShare, kOutCap);
+                if (drifted && !rebuild) {
+                    const double h = cell_size(rmax, uni(cs.s_cell));
+                    rebuild = drifted_meet<WG>(P, Np, w, crad, vb, sh->out, drifted, vmax, u, mbase, rmax, h,
+                                               cc_grid(Np, Nc, T, h, w.start), s_red);
+                }
             }
-            rebuild = !(drift <= kDriftRebuild);
             // no candidate pair at all and every circle within its skin: no
             // pair can overlap during the sweep, which therefore changes nothing
-            if (!rebuild && uni(cs.pairs) == 0u) {
+            if (!rebuild && drifted == 0u && uni(cs.pairs) == 0u) {
                 if (tid == 0) cs.since_build++;
                 return 0u;
             }
@@ -1713,14 +1992,14 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
                 continue;
             }
             u = make_float2(0.0f, 0.0f);
+            drifted = 0u;
         }
         // ---- sweep: the active pairs in rounds
-        const float mbase = kActiveBase * fmaxf(rmax, 1e-3f);
         // a redo widens the margins, then takes every candidate
         const float mscale = widen == 0u ? 1.0f : widen == 1u ? 4.0f : INFINITY;
         const uint32_t pairs = uni(cs.pairs);
         const uint32_t active =
-            pairs ? uni(sweep_rounds<WG>(P, Np, Nc, crad, uni_r, runi, mbase, mscale, sh, s_wl, pairs)) : 0u;
+            pairs || drifted ? uni(sweep_rounds<WG>(P, Np, Nc, crad, uni_r, runi, mbase, mscale, sh, s_wl, pairs)) : 0u;
         if (active == kNone) {
             // more pairs in reach of each other than the workspace holds
             if (widen == 0u) fallback = true;
@@ -1729,7 +2008,7 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
             __syncthreads();
             continue;
         }
-        if (active == 0u) {
+        if (active == 0u && drifted == 0u) {
             // no pair can touch, and nothing has moved: the skins hold (the
             // drift since the list was built is within kDriftRebuild of them)
             for (uint32_t c = tid; c < Nc; c += WG) w.need[c] = 0.75f * w.need[c];
@@ -1746,10 +2025,11 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
         // builds)
         float vmax = 0.0f, vall = 0.0f;
         float *vb = (float *)w.stamp;
-        if (tid == 0) { sh->nout = 0u; sh->nnear = 0u; }
+        if (tid == 0) { sh->nout = 0u; sh->nnear = 0u; if (!active) sh->stalled = 0u; }
         __syncthreads();
         for (uint32_t c = tid; c < Nc; c += WG) {
             float pth = w.path[c];
+            if (!active) w.path[c] = pth = 0.0f;  // no round has run
             const float nd = w.need[c];
             float v = moved_bound(w.save[c], w.ref[c], u, pth);
             // the sweep's own pushes, decaying slowly so circles in lasting contact keep their skin
@@ -1775,29 +2055,39 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
         const bool missed_near = check != 0;
         if (check == 0 && n_over) {
             const double h = cell_size(rmax, uni(cs.s_cell));  // the grid of the list build
-            if (n_over > kOutCap) {
+            const CCGrid g = cc_grid(Np, Nc, T, h, w.start);
+            if (n_over > kOutCap && !rebuild) {
+                check = 3;  // too many to tell with an old list
+            } else if (n_over > kOutCap) {
                 vall = fmaxf(wg_max<WG>(vall, s_red), vmax);
-                check = overruns_check<WG>(w, act, crad, vb, w.wl, n_over, vall, rmax, h, 1.0 / h, tmask, s_red, true);
+                check = overruns_check<WG>(w, act, crad, vb, w.wl, n_over, vall, u, rmax, h, g, s_red, true);
             } else {
-                check = overruns_check<WG>(w, act, crad, vb, sh->out, n_over, vmax, rmax, h, 1.0 / h, tmask, s_red,
-                                           false);
+                check = overruns_check<WG>(w, act, crad, vb, sh->out, n_over, vmax, u, rmax, h, g, s_red, false);
             }
         }
         if (check == 0) {
             if (tid == 0) {
                 cs.since_build++;
                 if (n_over) sh->cnt.kept++;
+                if (widen == 0u && ++cs.clean >= kLevelClean) {
+                    cs.clean = 0u;
+                    if (cs.level) cs.level--;
+                }
             }
             return 0u;
         }
-        if (check == 2 && tid == 0) sh->cnt.unchecked++;
+        if (check == 3 && tid == 0) sh->cnt.unchecked++;
         // undo; the next attempt has the margins (and skins) the circles showed
         // they need
         for (uint32_t c = tid; c < Nc; c += WG) P[Np + c] = w.save[c];
-        const bool same_list = missed_near && widen < 2u;
+        const bool same_list = check == 1 && widen < 2u;
         if (tid == 0) {
             sh->cnt.redos++;
             if (!same_list) cs.list_valid = 0u;
+            if (missed_near) {
+                cs.clean = 0u;
+                if (widen == 0u) cs.level = min(cs.level + 2u, kLevels);
+            }
         }
         __syncthreads();
         if (same_list) attempt--;
@@ -1811,7 +2101,7 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
 template <int WG>
 __device__ __forceinline__ bool quiet_sweep(const float2 *P, uint32_t Np, uint32_t Nc, CCShared *sh) {
     if (uni(sh->cs.list_valid) == 0u || uni(sh->cs.pairs) != 0u || uni(sh->fb_streak) != 0u) return false;
-    const Drift dr = drift_box<WG>(P, Np, Nc, sh->work.ref, sh->red4);
+    const Drift dr = drift_box<WG, false>(P, Np, Nc, sh->work.ref, sh->red4);
     if (!(drift_share(dr.box, uni(sh->cs.smin)) <= kDriftRebuild)) return false;
     if (threadIdx.x == 0) sh->cs.since_build++;
     return true;
@@ -2156,7 +2446,8 @@ __device__ __forceinline__ void run_scene(const SceneDesc *__restrict__ dp, uint
 
     uint32_t err = uni(st->err);
     if (tid == 0) {
-        s_cc->cs = CCShared::Steer{st->skin, st->list_valid, st->pairs, st->since_build, st->s_cell, st->smin};
+        s_cc->cs = CCShared::Steer{st->skin, (uint32_t)st->list_valid & 1u, st->pairs, st->since_build, st->s_cell, st->smin,
+                                   (uint32_t)st->list_valid >> 1, 0u};
         s_cc->fb_streak = 0u;
         CCShared::Counts &k = s_cc->cnt;
         k = CCShared::Counts{};
@@ -2254,7 +2545,7 @@ __device__ __forceinline__ void run_scene(const SceneDesc *__restrict__ dp, uint
     if (tid == 0) {
         const CCShared::Steer &cs = s_cc->cs;
         st->skin = cs.skin;
-        st->list_valid = cs.list_valid ? 1u : 0u;
+        st->list_valid = (uint8_t)((cs.list_valid ? 1u : 0u) | (cs.level << 1));
         st->err = err;
         const CCShared::Counts &k = s_cc->cnt;
         st->rounds += k.rounds;

@@ -65,3 +65,35 @@ def test_clump(n):
         s.update(DT)
         assert o.update(DT) == 0
     assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
+
+
+@pytest.mark.parametrize("lds", [0, 144 * 1024])
+@pytest.mark.parametrize("n,span", [(15, 3.0), (16, 3.0), (17, 40.0), (31, 6.0), (32, 1000.0), (700, 30.0), (2049, 90.0),
+                                    (13312, 240.0), (13313, 240.0)])
+def test_grid_edges(n, span, lds):
+    # tables too small for separate rows of cells, the first that has them, and
+    # the largest counters in LDS and the first of half as many; counters in LDS
+    # and in memory; some circles fast enough to outlie (n = 2049: more than one
+    # stage of a 128-lane workgroup holds) and one far away
+    rng = np.random.default_rng(n)
+    c = np.zeros((n, 7), np.float32)
+    c[:, 0:2] = rng.uniform(0.0, span, (n, 2))
+    speed = np.where(rng.uniform(size=n) < 0.1, 30.0, 2.0)[:, None]
+    c[:, 2:4] = c[:, 0:2] - speed * rng.standard_normal((n, 2)) * (DT / 4)
+    c[:, 6] = 0.35
+    c[0, 0:4] += 5000.0
+    s = Solver()
+    s.gravity, s.bounds = (0.0, 0.0), ((-100.0, -100.0), (6000.0, 6000.0))
+    s.set_sub_steps(4)
+    s.add_circles(c)
+    o = to_oracle(s, 32, candidate_mode=True)
+    b = Batch()
+    b.add_scene(s)
+    b.config = dict(wg_small=128, wg_large=1024, split_points=4096, lds_small=lds, lds_large=lds, steps_per_launch=1,
+                    use_graph=0, split_tiny=64, wg_tiny=64, lds_tiny=lds)
+    b.update(DT, 2)
+    b.sync()
+    for _ in range(2):
+        assert o.update(DT) == 0
+    b.read_scene(0, s)
+    assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
