@@ -5,11 +5,11 @@
 //              layers reproduce the sequential Gauss-Seidel order exactly
 //              (src/solver.rs:143-153)
 //   circles    candidate pairs from a hierarchical hashed cell broadphase
-//              (per-circle margins, counting sort with wave prefix scans), the
+//              (per-circle margins, counting sort that numbers the circles), the
 //              connected components of the candidate graph (union-find), and an
 //              exact replay of the reference's (i, j) lexicographic sweep
-//              (src/solver.rs:168-177) per component: by one lane, by one
-//              wavefront in LDS, or by a workgroup in global memory, by size;
+//              (src/solver.rs:168-177) per component: by lanes of a wavefront,
+//              a circle to each, or by a workgroup in LDS or in global memory;
 //              a sweep whose circles left their margins is checked pair by pair
 //              at each skipped pair's turn and redone only if one met
 //   polygons   one workgroup replays the polygon-pair loop (src/solver.rs:178-187)
@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/bendy2d.h"
@@ -191,42 +192,73 @@ __global__ void k_zero_acc0(float2 *acc0, uint32_t n) {
 //
 // Margins can differ by orders of magnitude (a jammed ring of circles around a
 // collider beside quiet gas), so the grid is hierarchical: circle i sits at
-// level L_i, the smallest L with m_i <= lim_L = s0 4^L, in a grid of cell size
-// h_L = 2 (rmax + lim_L) (x1.001); all levels share one hash table keyed by
-// (L, cell).  Circle i scans the levels L <= L_i over the cells that its reach
-// plus level L's largest reach covers, and the levels above L_i over the 3x3
-// cells around its own cell there.  Both sides of a pair find it, so each
-// circle writes its own list without atomics.
+// level L_i, the smallest L with m_i <= lim_L = lim_0 4^L, in a grid of cell size
+// h_L = 2 (rmax + lim_L) (x1.001); all levels share one table of T buckets, cell
+// (x, y) of level L in bucket (x + y stride + L c) mod T with stride about
+// 0.618 T: the cells of a row are consecutive buckets.  Circle i scans the levels
+// L <= L_i over the cells that its reach plus level L's largest reach covers, and
+// the levels above L_i over the 3x3 cells around its own cell there, a run of
+// records per row.  Both sides of a pair find it, so each circle writes its own
+// list without atomics.
+//
+// The counting sort that fills the buckets also numbers the circles: slot s is
+// place s in bucket order, and every array of the sweep after the sort goes by
+// slot.  The circles that a wavefront's 64 slots meet lie in a few runs of
+// neighbouring slots, where by circle number every access took a cache line of
+// its own (262,144 circles, 32 sweeps and the upload: 32.7 ms, 23.6 by slot; with
+// what follows 13.2).
+// Only the order of the pairs is by circle number: lists are sorted by it, and an
+// entry holds the partner's slot and, in kLater, whether its number is larger.
 //
 // The sweep then runs per connected component of the candidate graph: pairs
 // of different components share no circle, so they commute, and within one
-// component the reference's (i, j) order (src/solver.rs:168-177) is kept.
-// Components of at most kLaneMax circles are replayed pair by pair by one
-// lane; larger ones by a workgroup with the round protocol: pair (i, j) runs
-// once j is the next unprocessed partner of i and i the next of j.
+// component the reference's (i, j) order (src/solver.rs:168-177) is kept by the
+// round protocol: pair (i, j) runs once j is the next unprocessed partner of i and
+// i the next of j.  Components of up to 4, 16 and 64 circles run in as many lanes
+// of a wavefront, a circle to a lane; larger ones in a workgroup, in LDS or, above
+// kLdsMembers circles, in global memory.
+//
+// The host waits once a sweep, for its verdict: lists are handed their space by
+// one atomic per workgroup, out of what earlier sweeps needed (a sweep whose
+// lists do not fit changes nothing and runs again with more), components
+// likewise, and the check of overruns takes their number from device memory.
+// Counters that many wavefronts add to are added to once a workgroup: 4,096
+// atomics on one word take about 30 us (k_cg_check 34 -> 11 us).
 
 constexpr int kLevels = 12;
-constexpr uint32_t kSlotG = 8;  // candidates kept by the counting pass
-constexpr uint32_t kLvlShift = 26;  // bucket record .w: index | level << 26
+constexpr uint32_t kSlotG = 8;  // candidates kept by the counting scan
+constexpr uint32_t kLvlShift = 26;  // bucket record .w: circle | level << 26
 constexpr uint32_t kIdxMaskG = (1u << kLvlShift) - 1u;
-constexpr uint32_t kLaneMax = 4;
-constexpr uint32_t kLdsMembers = 128, kLdsEntries = 1024;
-constexpr int64_t kMaxScanCells = 1024;
+constexpr uint32_t kLater = 0x80000000u;   // list entry: the partner's number is larger
+constexpr uint32_t kParent = 0x40000000u;  // list entry: the parent that the circle starts with (k_cg_union)
+constexpr uint32_t kLaneList = 32;  // list entries of a circle that a lane holds
+constexpr uint32_t kLdsMembers = 1024, kLdsEntries = 8192;
+// component queues: for 4, 16 and 64 lanes, a workgroup in LDS, one in memory
+constexpr uint32_t kQueues = 5, kQueueLds = 3, kQueueBig = 4;
+// A reach over more cells than kMaxScanCells in one level scans every circle.  One
+// over more than kOwnScanCells (a circle above level 0; level 0 takes up to 3 x 3)
+// is scanned by 16 lanes, kPieceCells cells of a row to each at a time: left to
+// its own lane it held up the launch.
+constexpr int64_t kMaxScanCells = 1024, kOwnScanCells = 32;
+constexpr int kPieceCells = 4;
 constexpr uint32_t kNoneG = 0xffffffffu;
 constexpr int kCompWG = 256;
+constexpr uint32_t kCheckPer = 4;  // slots a thread of k_cg_ranges and k_cg_check
 
 // Per-sweep grid of every level, in device memory.
 struct CGrid {
     double inv_h[kLevels];
-    float lim[kLevels];        // largest margin of level L: s0 * 4^L
+    float lim[kLevels];        // largest margin of level L: lim_0 * 4^L
     float reach_max[kLevels];  // largest reach of level L: rmax + lim
 };
 
-// Control words of a sweep (zeroed with the bucket counters).
+// Control words of a sweep (zeroed with the bucket counters, which follow them;
+// the two at kCtlTotal are one 64-bit counter).
 enum : uint32_t {
-    kCtlMask = 0, kCtlOver, kCtlBad, kCtlRounds, kCtlNbig, kCtlQueue, kCtlInf, kCtlMissed, kCtlQuiet, kCtlNmid,
-    kCtlEmax = 16, kCtlWords = kCtlEmax + kLevels
+    kCtlTotal = 0, kCtlMask = 2, kCtlOver, kCtlBad, kCtlRounds, kCtlInf, kCtlMissed, kCtlQuiet, kCtlMembers, kCtlFull,
+    kCtlQueue = 12, kCtlEmax = kCtlQueue + kQueues, kCtlWords = 32
 };
+static_assert(kCtlEmax + kLevels <= (int)kCtlWords, "control words");
 
 __device__ __forceinline__ int cell_coord_d(double x, double inv_h) {
     double c = floor(x * inv_h);
@@ -239,78 +271,153 @@ __device__ __forceinline__ int cell_coord_d(double x, double inv_h) {
 // or non-finite coordinates stay finite.
 __device__ __forceinline__ int cell_coord(float x, double inv_h) { return cell_coord_d((double)x, inv_h); }
 
-__device__ __forceinline__ uint32_t level_hash(uint32_t L, int cx, int cy) {
-    return cell_hash(cx, cy) ^ (L * 0x9e3779b9u);
+// Largest margin and inverse cell size of level L.
+__device__ __forceinline__ float level_lim(float lim0, uint32_t L) { return ldexpf(lim0, 2 * (int)L); }
+__device__ __forceinline__ double level_inv_h(float rmax, float lim) {
+    return 1.0 / ((2.0 * (double)(rmax + lim)) * 1.001 + 1e-30);
 }
 
-__global__ void k_cg_grid(float s0, float rmax, CGrid *__restrict__ g) {
-    const int L = threadIdx.x;
-    if (L >= kLevels) return;
-    const float lim = ldexpf(s0, 2 * L);
-    const float rm = rmax + lim;
-    g->lim[L] = lim;
-    g->reach_max[L] = rm;
-    g->inv_h[L] = 1.0 / ((2.0 * (double)rm) * 1.001 + 1e-30);
+// Margin of a circle that needs `need`, and its level.
+__device__ __forceinline__ float level_margin(float s0, float lim0, float need, uint32_t &L) {
+    const float m = fmaxf(s0, need);
+    L = 0;
+    while (L + 1 < (uint32_t)kLevels && m > level_lim(lim0, L)) L++;
+    return fminf(m, level_lim(lim0, L));
 }
 
+struct Buckets {
+    uint32_t nc, tmask, stride;
+    const uint32_t *__restrict__ start;
+    const float4 *__restrict__ rec;
+};
+
+__device__ __forceinline__ uint32_t bucket_of(uint32_t tmask, uint32_t stride, uint32_t L, int cx, int cy) {
+    return ((uint32_t)cx + (uint32_t)cy * stride + L * 0x9e3779b9u) & tmask;
+}
+
+// Calls f(slot, record) for the records of level L in the cells x0 .. x1 of the
+// rows y, y + step, ... <= y1.  A row's cells are one run of slots, going on at
+// slot 0 after the last; three rows are looked up at a time and their runs read as
+// one, kU records in flight (row by row every level cost three chains of dependent
+// loads, for mostly empty runs).  near(record) is asked first: a run may hold
+// other cells' and levels' records.
+template <typename N, typename F>
+__device__ __forceinline__ void scan_rows(const Buckets &b, uint32_t L, int x0, int x1, int y, int y1, int step,
+                                          double ih, N near, F f) {
+    const uint32_t nx = (uint32_t)(x1 - x0) + 1u, T = b.tmask + 1u;
+    constexpr uint32_t kU = 4;
+    for (; y <= y1; y += 3 * step) {
+        uint32_t s0[3], len[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            s0[k] = 0u;
+            len[k] = 0u;
+            if (y + k * step > y1) continue;
+            len[k] = b.nc;  // (as many cells as buckets: all records)
+            if (nx <= b.tmask) {
+                const uint32_t at = bucket_of(b.tmask, b.stride, L, x0, y + k * step), e = at + nx;
+                s0[k] = b.start[at];
+                const uint32_t s1 = b.start[e > T ? e - T : e];
+                len[k] = e > T ? b.nc - s0[k] + s1 : s1 - s0[k];
+            }
+        }
+        const uint32_t p1 = len[0], p2 = p1 + len[1], total = p2 + len[2];
+        for (uint32_t t0 = 0; t0 < total; t0 += kU) {
+            float4 q[kU];
+            uint32_t s[kU];
+            int cy[kU];
+#pragma unroll
+            for (uint32_t u = 0; u < kU; u++) {
+                const uint32_t t = min(t0 + u, total - 1u);
+                s[u] = t < p1 ? s0[0] + t : t < p2 ? s0[1] + (t - p1) : s0[2] + (t - p2);
+                cy[u] = t < p1 ? y : t < p2 ? y + step : y + 2 * step;
+                if (s[u] >= b.nc) s[u] -= b.nc;
+                q[u] = b.rec[s[u]];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kU; u++) {
+                if (t0 + u >= total || !near(q[u])) continue;
+                if ((__float_as_uint(q[u].w) >> kLvlShift) != L) continue;
+                if (cell_coord(q[u].y, ih) != cy[u]) continue;
+                const int cx = cell_coord(q[u].x, ih);
+                if (cx < x0 || cx > x1) continue;
+                f(s[u], q[u]);
+            }
+        }
+    }
+}
+
+// The levels' grid, each circle's bucket and its rank there.  Thread t takes the
+// circle that was in slot t in the sweep before: its neighbours in the wavefront
+// then count into the same few cache lines of counters, and go to neighbouring
+// slots in the scatter (by number each atomic was a request of its own).  The
+// circles' needs are kept by that slot too.
 __global__ void __launch_bounds__(256) k_cg_prep(const float2 *__restrict__ pos, uint32_t cbase,
-                                                 const float *__restrict__ crad, const float *__restrict__ need,
-                                                 const CGrid *__restrict__ g, uint32_t nc, uint32_t tmask,
-                                                 float2 *__restrict__ save, float *__restrict__ exc,
-                                                 float *__restrict__ marg, float *__restrict__ reach,
-                                                 uint8_t *__restrict__ lvl, uint32_t *__restrict__ key,
-                                                 uint32_t *__restrict__ count, uint32_t *__restrict__ par,
+                                                 const float *__restrict__ need, const uint32_t *__restrict__ order,
+                                                 float s0, float lim0, float rmax, uint32_t nc, uint32_t tmask,
+                                                 uint32_t stride, CGrid *__restrict__ g,
+                                                 uint2 *__restrict__ key, uint32_t *__restrict__ count,
                                                  uint32_t *__restrict__ ctl) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < (uint32_t)kLevels) {
+        const float lim = level_lim(lim0, t);
+        g->lim[t] = lim;
+        g->reach_max[t] = rmax + lim;
+        g->inv_h[t] = level_inv_h(rmax, lim);
+    }
     uint32_t bit = 0;
-    if (i < nc) {
+    if (t < nc) {
+        const uint32_t i = order[t];
         const float2 p = pos[cbase + i];
-        save[i] = p;
-        exc[i] = 0.0f;
-        par[i] = i;
-        float m = fmaxf(g->lim[0], need[i]);
-        uint32_t L = 0;
-        while (L + 1 < (uint32_t)kLevels && m > g->lim[L]) L++;
-        m = fminf(m, g->lim[L]);
-        marg[i] = m;
-        reach[i] = crad[i] + m;
-        lvl[i] = (uint8_t)L;
-        const double ih = g->inv_h[L];
-        const uint32_t k = level_hash(L, cell_coord(p.x, ih), cell_coord(p.y, ih)) & tmask;
-        key[i] = k;
-        atomicAdd(&count[k], 1u);
+        uint32_t L;
+        (void)level_margin(s0, lim0, need[t], L);
+        const double ih = level_inv_h(rmax, level_lim(lim0, L));
+        const uint32_t k = bucket_of(tmask, stride, L, cell_coord(p.x, ih), cell_coord(p.y, ih));
+        key[t] = make_uint2(k, atomicAdd(&count[k], 1u));
         bit = 1u << L;
     }
-    // occupied levels above 0 (level 0 counts as occupied): one atomic per
-    // wavefront that holds such a level, so the common all-level-0 wavefront
-    // takes none
+    // occupied levels above 0 (level 0 counts as occupied): an atomic only where
+    // a wavefront holds a level not yet seen in the word
     for (int o = 32; o > 0; o >>= 1) bit |= __shfl_xor(bit, o);
-    if ((threadIdx.x & 63u) == 0u && (bit & ~1u)) atomicOr(&ctl[kCtlMask], bit);
+    bit &= ~1u;
+    if ((threadIdx.x & 63u) == 0u && bit &&
+        (bit & ~__hip_atomic_load(&ctl[kCtlMask], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+        atomicOr(&ctl[kCtlMask], bit);
 }
 
-__global__ void __launch_bounds__(256) k_cg_scatter(const float2 *__restrict__ save, const float *__restrict__ reach,
-                                                    const uint8_t *__restrict__ lvl, const uint32_t *__restrict__ key,
-                                                    uint32_t nc, const uint32_t *__restrict__ start,
-                                                    uint32_t *__restrict__ fill, float4 *__restrict__ rec) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc) return;
-    const uint32_t k = key[i];
-    const uint32_t s = start[k] + atomicAdd(&fill[k], 1u);
-    const float2 p = save[i];
-    rec[s] = make_float4(p.x, p.y, reach[i], __uint_as_float(i | ((uint32_t)lvl[i] << kLvlShift)));
+// Each circle's record to its slot: position, reach, number and level in rec;
+// radius, margin and need in aux.
+__global__ void __launch_bounds__(256) k_cg_scatter(const float2 *__restrict__ pos, uint32_t cbase,
+                                                    const float *__restrict__ crad, const float *__restrict__ need,
+                                                    const uint32_t *__restrict__ order, float s0, float lim0,
+                                                    const uint2 *__restrict__ key, uint32_t nc,
+                                                    const uint32_t *__restrict__ start, float4 *__restrict__ rec,
+                                                    float4 *__restrict__ aux) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nc) return;
+    const uint32_t i = order[t];
+    const uint2 k = key[t];
+    const uint32_t s = start[k.x] + k.y;
+    const float2 p = pos[cbase + i];
+    const float nd = need[t], r = crad[i];
+    uint32_t L;
+    const float m = level_margin(s0, lim0, nd, L);
+    rec[s] = make_float4(p.x, p.y, r + m, __uint_as_float(i | (L << kLvlShift)));
+    aux[s] = make_float4(r, m, nd, 0.0f);
 }
 
-__device__ __forceinline__ void cswap_u32(uint32_t &a, uint32_t &b) {
-    const uint32_t lo = min(a, b), hi = max(a, b);
+template <typename T>
+__device__ __forceinline__ void cswap(T &a, T &b) {
+    const T lo = min(a, b), hi = max(a, b);
     a = lo; b = hi;
 }
 
 // Ascending sort of a list in global memory: insertion for short lists,
 // heapsort for long ones.
-__device__ void sort_list(uint32_t *a, uint32_t n) {
+__device__ __noinline__ void sort_list(uint64_t *a, uint32_t n) {
     if (n <= 32u) {
         for (uint32_t x = 1; x < n; x++) {
-            const uint32_t v = a[x];
+            const uint64_t v = a[x];
             uint32_t y = x;
             while (y > 0 && a[y - 1] > v) { a[y] = a[y - 1]; y--; }
             a[y] = v;
@@ -322,7 +429,7 @@ __device__ void sort_list(uint32_t *a, uint32_t n) {
             uint32_t child = 2u * root + 1u;
             if (child >= end) return;
             if (child + 1u < end && a[child] < a[child + 1u]) child++;
-            const uint32_t vr = a[root], vc = a[child];
+            const uint64_t vr = a[root], vc = a[child];
             if (!(vr < vc)) return;
             a[root] = vc; a[child] = vr;
             root = child;
@@ -330,120 +437,213 @@ __device__ void sort_list(uint32_t *a, uint32_t n) {
     };
     for (uint32_t s = n / 2u; s-- > 0;) sift(s, n);
     for (uint32_t e = n - 1u; e > 0; e--) {
-        const uint32_t t = a[0]; a[0] = a[e]; a[e] = t;
+        const uint64_t t = a[0]; a[0] = a[e]; a[e] = t;
         sift(0, e);
     }
 }
 
-// Candidates of circle i (see above).  MODE 0 counts them and keeps the
-// first kSlotG in slot; MODE 1 writes the list at off[i], from slot when it
-// fits there and by a second gather otherwise, and sorts it ascending.
-template <int MODE>
-__global__ void __launch_bounds__(256) k_cg_cand(const float2 *__restrict__ save, const float *__restrict__ reach,
-                                                 const uint8_t *__restrict__ lvl, const CGrid *__restrict__ g,
-                                                 const uint32_t *__restrict__ ctl, const uint32_t *__restrict__ start,
-                                                 const float4 *__restrict__ rec, uint32_t nc, uint32_t tmask,
-                                                 uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
-                                                 uint32_t *__restrict__ cand, uint32_t *__restrict__ slot) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (MODE == 0 && i == 0) cnt[nc] = 0u;  // the scan's last entry
-    if (i >= nc) return;
-    uint32_t *const keep = slot + (size_t)i * kSlotG;
-    uint32_t *out = MODE == 1 ? cand + off[i] : nullptr;
-    if (MODE == 1) {
-        const uint32_t n0 = cnt[i];
-        if (n0 <= kSlotG) {
-            uint32_t v[kSlotG];
-#pragma unroll
-            for (uint32_t k = 0; k < kSlotG; k++) v[k] = k < n0 ? keep[k] : kNoneG;
-#pragma unroll
-            for (uint32_t k = 2; k <= kSlotG; k <<= 1)
-#pragma unroll
-                for (uint32_t j = k >> 1; j > 0; j >>= 1)
-#pragma unroll
-                    for (uint32_t x = 0; x < kSlotG; x++) {
-                        const uint32_t l = x ^ j;
-                        if (l > x) {
-                            if ((x & k) == 0u) cswap_u32(v[x], v[l]);
-                            else cswap_u32(v[l], v[x]);
-                        }
-                    }
-#pragma unroll
-            for (uint32_t k = 0; k < kSlotG; k++)
-                if (k < n0) out[k] = v[k];
-            return;
-        }
+// Exclusive place of each thread's v among the workgroup's 256 threads; total is
+// the sum (64-bit: lists can be as long as the scene).  s_sum: 4 words of LDS.
+__device__ __forceinline__ uint64_t block_place(uint32_t v, uint64_t *s_sum, uint64_t &total) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint64_t inc = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t t = __shfl_up(inc, o);
+        if ((int)lane >= o) inc += t;
     }
-    const float2 p = save[i];
-    uint32_t n = 0;
-    // a circle at a non-finite position takes part in no pair
-    if (fabsf(p.x) <= 3.0e38f && fabsf(p.y) <= 3.0e38f) {
-        const float ri = reach[i];
-        const uint32_t Li = lvl[i];
-        const uint32_t mask = ctl[kCtlMask] | 1u;
-        const uint32_t below = mask & ((2u << Li) - 1u);  // levels <= Li
-        auto test = [&](uint32_t j, float qx, float qy, float rj) {
-            const float dx = p.x - qx, dy = p.y - qy, lim = ri + rj;
-            if (dx * dx + dy * dy < lim * lim) {
-                if (MODE == 1) out[n] = j;
-                else if (n < kSlotG) keep[n] = j;
-                n++;
-            }
-        };
-        auto visit = [&](uint32_t L, int cx, int cy, double ih) {
-            const uint32_t k = level_hash(L, cx, cy) & tmask;
-            for (uint32_t s = start[k], e = start[k + 1]; s < e; s++) {
-                const float4 q = rec[s];
-                const uint32_t w = __float_as_uint(q.w);
-                const uint32_t j = w & kIdxMaskG;
-                if ((w >> kLvlShift) != L || j == i) continue;
-                if (cell_coord(q.x, ih) != cx || cell_coord(q.y, ih) != cy) continue;
-                test(j, q.x, q.y, q.z);
-            }
-        };
-        // a reach spanning too many cells of a finer level scans every circle
-        bool brute = false;
-        for (uint32_t m = below; m; m &= m - 1u) {
-            const uint32_t L = (uint32_t)__ffs(m) - 1u;
-            const double R = ((double)ri + (double)g->reach_max[L]) * (1.0 + 1e-6);
-            const double ih = g->inv_h[L];
-            const int64_t nx = (int64_t)cell_coord_d((double)p.x + R, ih) - cell_coord_d((double)p.x - R, ih) + 1;
-            const int64_t ny = (int64_t)cell_coord_d((double)p.y + R, ih) - cell_coord_d((double)p.y - R, ih) + 1;
-            if (nx * ny > kMaxScanCells) brute = true;
-        }
-        if (brute) {
-            for (uint32_t j = 0; j < nc; j++) {
-                if (j == i) continue;
-                const float2 q = save[j];
-                test(j, q.x, q.y, reach[j]);
-            }
-        } else {
-            for (uint32_t m = below; m; m &= m - 1u) {
-                const uint32_t L = (uint32_t)__ffs(m) - 1u;
-                const double R = ((double)ri + (double)g->reach_max[L]) * (1.0 + 1e-6);
-                const double ih = g->inv_h[L];
-                const int x0 = cell_coord_d((double)p.x - R, ih), x1 = cell_coord_d((double)p.x + R, ih);
-                const int y0 = cell_coord_d((double)p.y - R, ih), y1 = cell_coord_d((double)p.y + R, ih);
-                for (int cy = y0; cy <= y1; cy++)
-                    for (int cx = x0; cx <= x1; cx++) visit(L, cx, cy, ih);
-            }
-            for (uint32_t m = mask & ~((2u << Li) - 1u); m; m &= m - 1u) {
-                const uint32_t L = (uint32_t)__ffs(m) - 1u;
-                const double ih = g->inv_h[L];
-                const int cx = cell_coord(p.x, ih), cy = cell_coord(p.y, ih);
-                for (int dy = -1; dy <= 1; dy++)
-                    for (int dx = -1; dx <= 1; dx++) visit(L, cx + dx, cy + dy, ih);
-            }
-        }
+    if (lane == 63u) s_sum[wave] = inc;
+    __syncthreads();
+    uint64_t base = 0;
+    total = 0;
+    for (uint32_t w = 0; w < 4u; w++) {
+        if (w < wave) base += s_sum[w];
+        total += s_sum[w];
     }
-    if (MODE == 0) cnt[i] = n;
-    else sort_list(out, n);
+    return base + inc - v;
 }
 
-// Union-find over the candidate graph.  parent[x] <= x always (a root is
-// hooked under the smaller root), so every value ever read is an ancestor.
+// Candidates of the circle in each slot (see above), in one go: count and keep
+// the first kSlotG in LDS, take space for the workgroup's lists, write them
+// sorted by circle number (longer ones from a second scan, through keys, the
+// trajectories' space).  What the rest of the sweep starts from goes by the way:
+// positions, excursions and parents (a circle hangs under the smallest slot of
+// its list at once, which leaves the union a third of the edges).
+__global__ void __launch_bounds__(256) k_cg_cand(Buckets bk, const CGrid *__restrict__ g, uint32_t cap,
+                                                 uint32_t *__restrict__ cnt, uint32_t *__restrict__ off,
+                                                 uint32_t *__restrict__ cand, uint64_t *__restrict__ keys,
+                                                 uint32_t *__restrict__ par, uint32_t *__restrict__ csize,
+                                                 float2 *__restrict__ spos, float *__restrict__ exc,
+                                                 uint32_t *__restrict__ order, const float4 *__restrict__ aux,
+                                                 float *__restrict__ need, uint32_t *__restrict__ ctl) {
+    __shared__ uint64_t s_keep[kSlotG][256];
+    __shared__ uint64_t s_sum[4], s_base;
+    __shared__ uint32_t s_n[256], s_o[256], s_wide[256], s_nwide;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, s = blockIdx.x * 256u + tid;
+    const uint32_t mask = ctl[kCtlMask] | 1u;
+    float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    bool on = false, wide = false;
+    if (s < bk.nc) {
+        r = bk.rec[s];
+        spos[s] = make_float2(r.x, r.y);
+        exc[s] = 0.0f;
+        csize[s] = 0u;
+        order[s] = __float_as_uint(r.w) & kIdxMaskG;
+        need[s] = aux[s].z;
+        // a circle at a non-finite position takes part in no pair
+        on = fabsf(r.x) <= 3.0e38f && fabsf(r.y) <= 3.0e38f;
+    }
+    // the cells of level L within reach of a circle
+    struct Span { int x0, x1, y0, y1; };
+    auto span = [&](const float4 &c, uint32_t L, double ih) {
+        const double R = ((double)c.z + (double)g->reach_max[L]) * (1.0 + 1e-6);
+        return Span{cell_coord_d((double)c.x - R, ih), cell_coord_d((double)c.x + R, ih),
+                    cell_coord_d((double)c.y - R, ih), cell_coord_d((double)c.y + R, ih)};
+    };
+    auto cells = [&](const float4 &c) {
+        int64_t most = 0;
+        for (uint32_t m = mask & ((2u << (__float_as_uint(c.w) >> kLvlShift)) - 1u); m; m &= m - 1u) {
+            const uint32_t L = (uint32_t)__ffs(m) - 1u;
+            const Span w = span(c, L, g->inv_h[L]);
+            most = max(most, ((int64_t)w.x1 - w.x0 + 1) * ((int64_t)w.y1 - w.y0 + 1));
+        }
+        return most;
+    };
+    // f(key) for every candidate of the circle c in slot self: all of them, or with
+    // SHARED those of the pieces that fall to this of 16 lanes
+    auto gather = [&](const float4 &c, uint32_t self, auto shared, auto f) {
+        constexpr bool kShared = decltype(shared)::value;
+        auto near = [&](const float4 &q) {
+            const float dx = c.x - q.x, dy = c.y - q.y, lim = c.z + q.z;
+            return dx * dx + dy * dy < lim * lim;
+        };
+        auto found = [&](uint32_t t, const float4 &q) {
+            if (t != self) f(((uint64_t)(__float_as_uint(q.w) & kIdxMaskG) << 32) | t);
+        };
+        if (kShared && cells(c) > kMaxScanCells) {
+            for (uint32_t t = tid & 15u; t < bk.nc; t += 16u) {
+                const float4 q = bk.rec[t];
+                if (near(q)) found(t, q);
+            }
+            return;
+        }
+        const uint32_t low = (2u << (__float_as_uint(c.w) >> kLvlShift)) - 1u;  // levels up to its own
+        for (uint32_t m = mask; m; m &= m - 1u) {
+            const uint32_t L = (uint32_t)__ffs(m) - 1u;
+            const double ih = g->inv_h[L];
+            Span w;
+            if ((low >> L) & 1u) w = span(c, L, ih);
+            else {
+                const int cx = cell_coord(c.x, ih), cy = cell_coord(c.y, ih);
+                w = Span{cx - 1, cx + 1, cy - 1, cy + 1};
+            }
+            if constexpr (!kShared) {
+                scan_rows(bk, L, w.x0, w.x1, w.y0, w.y1, 1, ih, near, found);
+            } else {
+                const uint32_t pieces = (uint32_t)(w.x1 - w.x0 + kPieceCells) / (uint32_t)kPieceCells;
+                const uint32_t items = pieces * (uint32_t)(w.y1 - w.y0 + 1);
+                for (uint32_t k = tid & 15u; k < items; k += 16u) {
+                    const int x = w.x0 + (int)(k % pieces) * kPieceCells, y = w.y0 + (int)(k / pieces);
+                    scan_rows(bk, L, x, min(x + kPieceCells - 1, w.x1), y, y, 1, ih, near, found);
+                }
+            }
+        }
+    };
+    if (tid == 0u) s_nwide = 0u;
+    __syncthreads();
+    if (on && cells(r) > kOwnScanCells) {
+        wide = true;
+        s_wide[atomicAdd(&s_nwide, 1u)] = tid;
+    }
+    // 16 lanes for each circle with a wide scan: f(its thread, place, key)
+    auto gather_wide = [&](auto f) {
+        for (uint32_t k = tid >> 4; k < s_nwide; k += 16u) {
+            const uint32_t st = s_wide[k], self = blockIdx.x * 256u + st;
+            if (s_n[st] == kNoneG) continue;  // (nothing to do)
+            gather(bk.rec[self], self, std::true_type{}, [&](uint64_t key) { f(st, atomicAdd(&s_n[st], 1u), key); });
+        }
+    };
+    s_n[tid] = 0u;
+    uint32_t n = 0;
+    if (on && !wide)
+        gather(r, s, std::false_type{}, [&](uint64_t key) {
+            if (n < kSlotG) s_keep[n][tid] = key;
+            n++;
+        });
+    __syncthreads();
+    gather_wide([&](uint32_t st, uint32_t k, uint64_t key) {
+        if (k < kSlotG) s_keep[k][st] = key;
+    });
+    __syncthreads();
+    if (wide) n = s_n[tid];
+    __syncthreads();
+    s_n[tid] = n > kSlotG ? 0u : kNoneG;
+    uint64_t total;
+    const uint64_t at = block_place(n, s_sum, total);
+    if (tid == 0u)
+        s_base = total ? atomicAdd((unsigned long long *)&ctl[kCtlTotal], (unsigned long long)total) : 0ull;
+    __syncthreads();
+    const uint64_t base = s_base;
+    if (base + total > cap) {  // uniform: nothing is replayed, the host makes room
+        if (tid == 0u) ctl[kCtlFull] = 1u;
+        return;
+    }
+    const uint32_t o0 = (uint32_t)(base + at);
+    s_o[tid] = o0;
+    __syncthreads();
+    if (n > kSlotG && !wide) {
+        uint32_t k = 0;
+        gather(r, s, std::false_type{}, [&](uint64_t key) { keys[o0 + k++] = key; });
+    }
+    gather_wide([&](uint32_t st, uint32_t k, uint64_t key) {
+        keys[s_o[st] + k] = key;
+    });
+    __syncthreads();
+    if (s >= bk.nc) return;
+    cnt[s] = n;
+    off[s] = o0;
+    const uint32_t i = __float_as_uint(r.w) & kIdxMaskG;
+    uint32_t low = s;
+    auto entry = [&](uint64_t key) {
+        return (uint32_t)key | ((uint32_t)(key >> 32) > i ? kLater : 0u) | ((uint32_t)key == low ? kParent : 0u);
+    };
+    if (n <= kSlotG) {
+        uint64_t v[kSlotG];
+#pragma unroll
+        for (uint32_t k = 0; k < kSlotG; k++) v[k] = k < n ? s_keep[k][tid] : ~0ull;
+#pragma unroll
+        for (uint32_t k = 2; k <= kSlotG; k <<= 1)
+#pragma unroll
+            for (uint32_t j = k >> 1; j > 0; j >>= 1)
+#pragma unroll
+                for (uint32_t x = 0; x < kSlotG; x++) {
+                    const uint32_t l = x ^ j;
+                    if (l > x) {
+                        if ((x & k) == 0u) cswap(v[x], v[l]);
+                        else cswap(v[l], v[x]);
+                    }
+                }
+#pragma unroll
+        for (uint32_t k = 0; k < kSlotG; k++)
+            if (k < n) low = min(low, (uint32_t)v[k]);
+#pragma unroll
+        for (uint32_t k = 0; k < kSlotG; k++)
+            if (k < n) cand[o0 + k] = entry(v[k]);
+    } else {
+        sort_list(keys + o0, n);
+        for (uint32_t k = 0; k < n; k++) low = min(low, (uint32_t)keys[o0 + k]);
+        for (uint32_t k = 0; k < n; k++) cand[o0 + k] = entry(keys[o0 + k]);
+    }
+    par[s] = low;
+}
+
+// Union-find over the candidate graph, by slot.  parent[x] <= x always (a root is
+// hooked under the smaller root), so every value ever read is an ancestor, also
+// one that another XCD has replaced since: the walks may read it from the caches
+// (their loads are of workgroup scope).  Hooking compares and swaps at device
+// scope: a stale root fails there and gives its parent; a stale partner that is
+// no root any more is still an ancestor to hang under, and smaller.
 __device__ __forceinline__ uint32_t uf_load(const uint32_t *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 __device__ uint32_t uf_find(uint32_t *par, uint32_t x) {
@@ -452,18 +652,21 @@ __device__ uint32_t uf_find(uint32_t *par, uint32_t x) {
         if (p == x) return x;
         const uint32_t g = uf_load(par + p);
         if (g == p) return p;
-        __hip_atomic_store(par + x, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // path halving
+        __hip_atomic_store(par + x, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);  // path halving
         x = g;
     }
 }
 
 __global__ void __launch_bounds__(256) k_cg_union(const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
-                                                  const uint32_t *__restrict__ cand, uint32_t nc, uint32_t *par) {
+                                                  const uint32_t *__restrict__ cand, uint32_t nc, uint32_t *par,
+                                                  const uint32_t *__restrict__ ctl) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc) return;
-    for (uint32_t s = off[i], e = s + cnt[i]; s < e; s++) {
-        uint32_t a = i, b = cand[s];
-        if (b < a) continue;  // each edge once, from its smaller end
+    if (i >= nc || ctl[kCtlFull]) return;
+    const uint32_t s0 = off[i], n = cnt[i];
+    for (uint32_t s = 0; s < n; s++) {
+        const uint32_t e = cand[s0 + s];
+        uint32_t a = e & kIdxMaskG, b = i;
+        if (a >= i || (e & kParent)) continue;  // each edge once, from its larger end
         for (;;) {
             a = uf_find(par, a);
             b = uf_find(par, b);
@@ -476,187 +679,252 @@ __global__ void __launch_bounds__(256) k_cg_union(const uint32_t *__restrict__ c
     }
 }
 
-// Component of each listed circle (its smallest index) and component sizes.
+// Component of each listed circle (its smallest slot), its place among the
+// component's members, and the components' sizes.
 __global__ void __launch_bounds__(256) k_cg_comp(const uint32_t *__restrict__ cnt, uint32_t nc, uint32_t *par,
-                                                 uint32_t *__restrict__ root, uint32_t *__restrict__ csize) {
+                                                 uint32_t *__restrict__ root, uint32_t *__restrict__ place,
+                                                 uint32_t *__restrict__ csize, const uint32_t *__restrict__ ctl) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc || cnt[i] == 0u) return;
+    if (i >= nc || ctl[kCtlFull] || cnt[i] == 0u) return;
     const uint32_t r = uf_find(par, i);
     root[i] = r;
-    atomicAdd(&csize[r], 1u);
+    place[i] = atomicAdd(&csize[r], 1u);
 }
 
-// Members of each component, grouped at cstart[root]; large components queue
-// for a workgroup.
+// Space for each component's members, and the queues by size, queue q at
+// queues + q nc.  One atomic per workgroup and counter.
+__global__ void __launch_bounds__(256) k_cg_ranges(const uint32_t *__restrict__ csize, uint32_t nc,
+                                                   uint32_t *__restrict__ cstart, uint32_t *__restrict__ queues,
+                                                   uint32_t *__restrict__ ctl) {
+    __shared__ uint64_t s_sum[4];
+    __shared__ uint32_t s_base[kQueues + 1], s_n[kQueues];
+    const uint32_t tid = threadIdx.x;
+    if (ctl[kCtlFull]) return;  // uniform
+    if (tid < kQueues) s_n[tid] = 0u;
+    __syncthreads();
+    uint32_t n[kCheckPer], at[kCheckPer], sum = 0;
+    auto queue_of = [](uint32_t m) {
+        return m <= 4u ? 0u : m <= 16u ? 1u : m <= 64u ? 2u : m <= kLdsMembers ? kQueueLds : kQueueBig;
+    };
+#pragma unroll
+    for (uint32_t u = 0; u < kCheckPer; u++) {
+        const uint32_t i = (blockIdx.x * kCheckPer + u) * 256u + tid;
+        n[u] = i < nc ? csize[i] : 0u;  // (0 but at roots)
+        sum += n[u];
+        if (n[u]) at[u] = atomicAdd(&s_n[queue_of(n[u])], 1u);
+    }
+    uint64_t total;
+    uint32_t place = (uint32_t)block_place(sum, s_sum, total);
+    if (tid <= kQueues) {
+        const uint32_t add = tid < kQueues ? s_n[tid] : (uint32_t)total;
+        s_base[tid] = add ? atomicAdd(&ctl[tid < kQueues ? kCtlQueue + tid : kCtlMembers], add) : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t u = 0; u < kCheckPer; u++) {
+        const uint32_t i = (blockIdx.x * kCheckPer + u) * 256u + tid;
+        if (n[u] == 0u) continue;
+        const uint32_t q = queue_of(n[u]);
+        queues[(size_t)q * nc + s_base[q] + at[u]] = i;
+        cstart[i] = s_base[kQueues] + place;
+        place += n[u];
+    }
+}
+
+// Members of each component, grouped at cstart[root].
 __global__ void __launch_bounds__(256) k_cg_members(const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ root,
-                                                    const uint32_t *__restrict__ csize,
+                                                    const uint32_t *__restrict__ place,
                                                     const uint32_t *__restrict__ cstart, uint32_t nc,
-                                                    uint32_t *__restrict__ cfill, uint32_t *__restrict__ members,
-                                                    uint32_t *__restrict__ midq, uint32_t *__restrict__ bigq,
-                                                    uint32_t *__restrict__ ctl) {
+                                                    uint32_t *__restrict__ members, const uint32_t *__restrict__ ctl) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t lane = threadIdx.x & 63u;
-    bool mid = false, big = false;
-    if (i < nc && cnt[i] != 0u) {
-        const uint32_t r = root[i];
-        members[cstart[r] + atomicAdd(&cfill[r], 1u)] = i;
-        if (r == i && csize[r] > kLaneMax) {
-            mid = csize[r] <= kLdsMembers;
-            big = !mid;
-        }
-    }
-    // queue appends: one atomic per wavefront and queue
-    const uint64_t bm = __ballot(mid), bb = __ballot(big);
-    const uint64_t below = (1ull << lane) - 1ull;
-    if (bm) {
-        uint32_t base = 0;
-        if (lane == 0u) base = atomicAdd(&ctl[kCtlNmid], (uint32_t)__popcll(bm));
-        base = __shfl(base, 0);
-        if (mid) midq[base + (uint32_t)__popcll(bm & below)] = i;
-    }
-    if (bb) {
-        uint32_t base = 0;
-        if (lane == 0u) base = atomicAdd(&ctl[kCtlNbig], (uint32_t)__popcll(bb));
-        base = __shfl(base, 0);
-        if (big) bigq[base + (uint32_t)__popcll(bb & below)] = i;
-    }
+    if (i >= nc || ctl[kCtlFull] || cnt[i] == 0u) return;
+    members[cstart[root[i]] + place[i]] = i;
 }
 
-// Pairs (c, j), j > c, of circle c's list in order, with live positions; the
-// calling lane owns every circle of the component.
-// Both circles' positions after each pair go to traj at the pair's entry in
-// their lists; head[j] counts j's pairs done so far, which is the index of
-// the current pair in j's list since each circle meets its pairs in list order.
-__device__ __forceinline__ void replay_list(uint32_t c, float2 *__restrict__ P, const float *__restrict__ crad,
-                                            const float2 *__restrict__ save, float *__restrict__ exc,
-                                            const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
-                                            const uint32_t *__restrict__ cand, uint32_t *__restrict__ head,
-                                            float2 *__restrict__ traj) {
-    float2 pc = P[c];
-    const float rc = crad[c];
-    const float2 sc = save[c];
-    float ec = exc[c];
-    for (uint32_t s = off[c], e = s + cnt[c]; s < e; s++) {
-        const uint32_t j = cand[s];
-        if (j <= c) continue;  // done at j's turn
-        float2 pj = P[j];
-        float qi = 0.0f, qj = 0.0f;
-        if (solve_circle_pair(pc.x, pc.y, pj.x, pj.y, rc, crad[j], qi, qj)) {
-            P[j] = pj;
-            const float2 sj = save[j];
-            exc[j] = excursion(exc[j], pj.x, pj.y, sj.x, sj.y);
-            ec = excursion(ec, pc.x, pc.y, sc.x, sc.y);
-        }
-        traj[s] = pc;
-        const uint32_t hj = head[j];
-        if (hj < cnt[j]) traj[off[j] + hj] = pj;  // always true for symmetric lists
-        head[j] = hj + 1u;
-    }
-    P[c] = pc;
-    exc[c] = ec;
+// The sweep's largest number of rounds: an atomic only for a new one (one for each
+// of 14,000 components took 100 us).
+__device__ __forceinline__ void note_rounds(uint32_t *ctl, uint32_t rounds) {
+    if (rounds > __hip_atomic_load(&ctl[kCtlRounds], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&ctl[kCtlRounds], rounds);
 }
 
-// Components of at most kLaneMax circles: the lane of the component's root
-// sorts its members and replays them in ascending order.
-__global__ void __launch_bounds__(256) k_cg_lane(float2 *__restrict__ pos, uint32_t cbase, const float *__restrict__ crad,
-                                                 const float2 *__restrict__ save, float *__restrict__ exc,
-                                                 const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
-                                                 const uint32_t *__restrict__ cand, const uint32_t *__restrict__ root,
-                                                 const uint32_t *__restrict__ csize,
-                                                 const uint32_t *__restrict__ cstart, uint32_t *__restrict__ members,
-                                                 uint32_t nc, uint32_t *__restrict__ head, float2 *__restrict__ traj) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc || cnt[i] == 0u || root[i] != i) return;
-    const uint32_t n = csize[i];
-    if (n > kLaneMax) return;
-    uint32_t *M = members + cstart[i];
-    uint32_t v[kLaneMax];
-#pragma unroll
-    for (uint32_t k = 0; k < kLaneMax; k++) v[k] = k < n ? M[k] : kNoneG;
-    // bitonic network, ascending
-#pragma unroll
-    for (uint32_t k = 2; k <= kLaneMax; k <<= 1)
-#pragma unroll
-        for (uint32_t j = k >> 1; j > 0; j >>= 1)
-#pragma unroll
-            for (uint32_t x = 0; x < kLaneMax; x++) {
-                const uint32_t l = x ^ j;
-                if (l > x) {
-                    if ((x & k) == 0u) cswap_u32(v[x], v[l]);
-                    else cswap_u32(v[l], v[x]);
-                }
+// Components of at most W circles, W = 4, 16 or 64: W lanes of a wavefront each, a
+// circle to a lane, its position in registers.  A round is: my next partner's next
+// partner, and if that is me, its position, by lane permutes; both lanes of a pair
+// then solve it alike and each keeps its own side.  Nothing is written between
+// rounds but the trajectory.  (20,011 circles 28 -> 11 us, 262,144 72 -> 45 us
+// against a wavefront with the state in LDS and a worklist for each component, and
+// a serial replay by one lane for those of up to 4.)  The lists, as places in the component, are
+// staged in LDS.  A component with a longer list than kLaneList joins the queue of
+// the LDS workgroups.
+template <uint32_t W>
+__device__ __forceinline__ void replay_lanes(uint32_t first, uint32_t step, const uint32_t *__restrict__ queue,
+                                             uint32_t nq, float2 *__restrict__ P, const float4 *__restrict__ aux,
+                                             const float4 *__restrict__ rec, float *__restrict__ exc,
+                                             const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
+                                             const uint32_t *__restrict__ cand, const uint32_t *__restrict__ csize,
+                                             const uint32_t *__restrict__ cstart, const uint32_t *__restrict__ members,
+                                             const uint32_t *__restrict__ place, uint32_t *__restrict__ lds_queue,
+                                             float2 *__restrict__ traj, uint32_t *__restrict__ ctl,
+                                             uint8_t (*s_list)[kLaneList + 4]) {
+    constexpr uint32_t kNone8 = 0xffu;
+    const uint32_t lane = threadIdx.x & 63u, k = lane & (W - 1u), base = lane & ~(W - 1u);
+    uint32_t most = 0;
+    for (uint32_t q0 = first; q0 < nq; q0 += step) {  // uniform per wavefront
+        const uint32_t q = q0 + lane / W;
+        uint32_t c = 0, m = 0, o = 0, r = 0;
+        float2 p = make_float2(0.0f, 0.0f), p0 = p;
+        float rad = 0.0f, e = 0.0f;
+        bool on = false, fits = true;
+        if (q < nq) {
+            r = queue[q];
+            on = k < csize[r];
+            if (on) {
+                c = members[cstart[r] + k];
+                m = cnt[c];
+                o = off[c];
+                const float4 v = rec[c];
+                p = p0 = make_float2(v.x, v.y);
+                rad = aux[c].x;
+                fits = m <= kLaneList;
             }
-#pragma unroll
-    for (uint32_t k = 0; k < kLaneMax; k++)
-        if (k < n) {
-            M[k] = v[k];
-            head[v[k]] = 0u;
         }
-    float2 *P = pos + cbase;
-    for (uint32_t k = 0; k < n; k++) replay_list(M[k], P, crad, save, exc, cnt, off, cand, head, traj);
+        // (all lanes of the component take part, or none)
+        const uint64_t group = (W == 64u ? ~0ull : ((1ull << (W & 63u)) - 1ull)) << base;
+        if (__ballot(!fits) & group) {
+            if (on && k == 0u) lds_queue[atomicAdd(&ctl[kCtlQueue + kQueueLds], 1u)] = r;
+            on = false;
+        }
+        if (!on) m = 0u;
+        constexpr uint32_t kU = 4;
+        for (uint32_t t0 = 0; t0 < m; t0 += kU) {
+            uint32_t v[kU];
+#pragma unroll
+            for (uint32_t u = 0; u < kU; u++) v[u] = cand[o + min(t0 + u, m - 1u)] & kIdxMaskG;
+#pragma unroll
+            for (uint32_t u = 0; u < kU; u++) v[u] = place[v[u]];
+#pragma unroll
+            for (uint32_t u = 0; u < kU; u++) s_list[lane][t0 + u] = (uint8_t)v[u];  // (kU - 1 past the end at most)
+        }
+        if (m) s_list[lane][m] = (uint8_t)kNone8;
+        uint32_t next = m ? s_list[lane][0] : kNone8, head = 0, rounds = 0;
+        for (;; rounds++) {
+            const int src = (int)(base + (next & (W - 1u)));
+            const uint32_t theirs = (uint32_t)__shfl((int)next, src);
+            const float2 pj = make_float2(__shfl(p.x, src), __shfl(p.y, src));
+            const float rj = __shfl(rad, src);
+            const bool ready = next != kNone8 && theirs == k;
+            if (!__ballot(ready)) break;
+            if (ready) {
+                const uint32_t after = s_list[lane][head + 1u];
+                float2 a = k < next ? p : pj, b = k < next ? pj : p;
+                float qi = 0.0f, qj = 0.0f;
+                if (solve_circle_pair(a.x, a.y, b.x, b.y, k < next ? rad : rj, k < next ? rj : rad, qi, qj)) {
+                    p = k < next ? a : b;
+                    e = excursion(e, p.x, p.y, p0.x, p0.y);
+                }
+                traj[o + head] = p;
+                head++;
+                next = after;
+            }
+        }
+        if (on) {
+            P[c] = p;
+            exc[c] = e;
+            if (head != m) atomicOr(&ctl[kCtlBad], 1u);
+        }
+        most = max(most, rounds);
+    }
+    if (lane == 0u && most) note_rounds(ctl, most);
 }
 
-// Components of kLaneMax+1 .. kLdsMembers circles: one wavefront each (a
-// grid stride over the queue), with the round protocol in LDS.  The members' positions, start
+// The components of up to 64 circles, largest first: the first workgroup past those
+// of each queue.
+struct LaneBlocks {
+    uint32_t end64, end16, end4;
+};
+
+__global__ void __launch_bounds__(64) k_cg_lanes(float2 *__restrict__ P, const float4 *__restrict__ aux,
+                                                 const float4 *__restrict__ rec, float *__restrict__ exc,
+                                                 const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
+                                                 const uint32_t *__restrict__ cand, const uint32_t *__restrict__ csize,
+                                                 const uint32_t *__restrict__ cstart,
+                                                 const uint32_t *__restrict__ members,
+                                                 const uint32_t *__restrict__ place, uint32_t *__restrict__ queues,
+                                                 uint32_t nc, LaneBlocks blk, float2 *__restrict__ traj,
+                                                 uint32_t *__restrict__ ctl) {
+    __shared__ uint8_t s_list[64][kLaneList + 4];
+    if (ctl[kCtlFull]) return;  // uniform
+    const uint32_t b = blockIdx.x;
+    uint32_t *const lds_queue = queues + (size_t)kQueueLds * nc;
+    if (b < blk.end64)
+        replay_lanes<64>(b, blk.end64, queues + 2 * (size_t)nc, ctl[kCtlQueue + 2], P, aux, rec, exc, cnt, off, cand,
+                         csize, cstart, members, place, lds_queue, traj, ctl, s_list);
+    else if (b < blk.end16)
+        replay_lanes<16>((b - blk.end64) * 4u, (blk.end16 - blk.end64) * 4u, queues + nc, ctl[kCtlQueue + 1], P, aux, rec,
+                         exc, cnt, off, cand, csize, cstart, members, place, lds_queue, traj, ctl, s_list);
+    else
+        replay_lanes<4>((b - blk.end16) * 16u, (blk.end4 - blk.end16) * 16u, queues, ctl[kCtlQueue], P, aux, rec, exc,
+                        cnt, off, cand, csize, cstart, members, place, lds_queue, traj, ctl, s_list);
+}
+
+// Components of 65 .. kLdsMembers circles, and smaller ones with long lists: a
+// workgroup each, with the round protocol in LDS.  The members' positions, start
 // positions, radii and excursions are staged into LDS and the lists remapped to
-// local indices (slot[c] = c's place among the members); the lists keep their
+// local indices (a circle's place among the members); the lists keep their
 // order, which is all the protocol depends on.  Positions after each pair go to
 // traj in global memory as in the other replays.  A component whose lists do
 // not fit joins the queue of the global-memory workgroups.
-__global__ void __launch_bounds__(64) k_cg_lds(float2 *__restrict__ pos, uint32_t cbase,
-                                               const float *__restrict__ crad, float *__restrict__ exc,
-                                               const float2 *__restrict__ save, const uint32_t *__restrict__ cnt,
-                                               const uint32_t *__restrict__ off, const uint32_t *__restrict__ cand,
-                                               const uint32_t *__restrict__ csize, const uint32_t *__restrict__ cstart,
-                                               const uint32_t *__restrict__ members, const uint32_t *__restrict__ midq,
-                                               uint32_t *__restrict__ bigq, uint32_t *__restrict__ slot,
-                                               float2 *__restrict__ traj, uint32_t *__restrict__ ctl) {
+__global__ void __launch_bounds__(256) k_cg_lds(float2 *__restrict__ P, const float4 *__restrict__ aux,
+                                                const float4 *__restrict__ rec, float *__restrict__ exc,
+                                                const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
+                                                const uint32_t *__restrict__ cand, const uint32_t *__restrict__ csize,
+                                                const uint32_t *__restrict__ cstart,
+                                                const uint32_t *__restrict__ members,
+                                                const uint32_t *__restrict__ place, uint32_t *__restrict__ queues,
+                                                uint32_t nc, float2 *__restrict__ traj, uint32_t *__restrict__ ctl) {
     __shared__ float2 s_p[kLdsMembers], s_s[kLdsMembers];
     __shared__ float s_r[kLdsMembers], s_e[kLdsMembers];
     __shared__ uint32_t s_off[kLdsMembers];
-    __shared__ uint16_t s_lb[kLdsMembers + 1], s_cnt[kLdsMembers], s_head[kLdsMembers], s_nxp[kLdsMembers],
+    __shared__ uint16_t s_lb[kLdsMembers], s_cnt[kLdsMembers], s_head[kLdsMembers], s_nxp[kLdsMembers],
         s_stamp[kLdsMembers];
     __shared__ uint16_t s_list[kLdsEntries];
     __shared__ uint32_t s_wl[2][kLdsMembers / 2 + 1];
     __shared__ uint32_t s_n[3], s_bad;
+    __shared__ uint64_t s_sum[4];
     constexpr uint16_t kNone16 = 0xffffu;
     const uint32_t tid = threadIdx.x;
-    const uint32_t nmid = ctl[kCtlNmid];
-    float2 *P = pos + cbase;
+    if (ctl[kCtlFull]) return;  // uniform
+    const uint32_t nmid = ctl[kCtlQueue + kQueueLds];
+    const uint32_t *const queue = queues + (size_t)kQueueLds * nc;
     for (uint32_t q = blockIdx.x; q < nmid; q += gridDim.x) {  // uniform per workgroup
-        const uint32_t r = midq[q], n = csize[r];
+        const uint32_t r = queue[q], n = csize[r];
         const uint32_t *M = members + cstart[r];
-        // stage; each lane takes kLdsMembers / 64 consecutive members for the scan
-        constexpr uint32_t kPer = kLdsMembers / 64u;
+        // stage; each thread takes consecutive members for the scan
+        constexpr uint32_t kPer = kLdsMembers / 256u;
         uint32_t sum = 0;
         for (uint32_t u = 0; u < kPer; u++) {
             const uint32_t k = tid * kPer + u;
             if (k < n) {
                 const uint32_t c = M[k];
-                slot[c] = k;
-                s_p[k] = P[c];
-                s_s[k] = save[c];
-                s_r[k] = crad[c];
-                s_e[k] = exc[c];
+                const float4 v = rec[c];
+                s_p[k] = s_s[k] = make_float2(v.x, v.y);
+                s_r[k] = aux[c].x;
+                s_e[k] = 0.0f;
                 s_off[k] = off[c];
                 const uint32_t m = cnt[c];
                 s_cnt[k] = (uint16_t)min(m, 0xffffu);
                 sum += m;
             }
         }
-        // exclusive list starts: a wavefront scan of the lanes' sums
-        uint32_t incl = sum;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t t = __shfl_up(incl, o);
-            if ((int)tid >= o) incl += t;
-        }
-        const uint32_t total = __shfl(incl, 63);
+        // exclusive list starts
+        uint64_t total;
+        uint32_t run = (uint32_t)block_place(sum, s_sum, total);
         if (total > kLdsEntries) {  // uniform: the lists do not fit
-            if (tid == 0) bigq[atomicAdd(&ctl[kCtlNbig], 1u)] = r;
+            if (tid == 0) queues[(size_t)kQueueBig * nc + atomicAdd(&ctl[kCtlQueue + kQueueBig], 1u)] = r;
             __syncthreads();
             continue;
         }
-        uint32_t run = incl - sum;
         for (uint32_t u = 0; u < kPer; u++) {
             const uint32_t k = tid * kPer + u;
             if (k < n) {
@@ -667,19 +935,19 @@ __global__ void __launch_bounds__(64) k_cg_lds(float2 *__restrict__ pos, uint32_
         if (tid == 0) { s_n[0] = 0u; s_n[1] = 0u; s_n[2] = 0u; s_bad = 0u; }
         __syncthreads();
         // local lists
-        for (uint32_t k = tid; k < n; k += 64u) {
+        for (uint32_t k = tid; k < n; k += 256u) {
             const uint32_t *src = cand + s_off[k];
             uint16_t *dst = s_list + s_lb[k];
-            for (uint32_t e = 0, m = s_cnt[k]; e < m; e++) dst[e] = (uint16_t)slot[src[e]];
+            for (uint32_t e = 0, m = s_cnt[k]; e < m; e++) dst[e] = (uint16_t)place[src[e] & kIdxMaskG];
         }
         __syncthreads();
-        for (uint32_t k = tid; k < n; k += 64u) {
+        for (uint32_t k = tid; k < n; k += 256u) {
             s_head[k] = 0;
             s_nxp[k] = s_cnt[k] ? s_list[s_lb[k]] : kNone16;
             s_stamp[k] = kNone16;
         }
         __syncthreads();
-        for (uint32_t k = tid; k < n; k += 64u) {
+        for (uint32_t k = tid; k < n; k += 256u) {
             const uint32_t o = s_nxp[k];
             if (o != kNone16 && k < o && s_nxp[o] == k) s_wl[0][atomicAdd(&s_n[0], 1u)] = k | (o << 16);
         }
@@ -687,7 +955,7 @@ __global__ void __launch_bounds__(64) k_cg_lds(float2 *__restrict__ pos, uint32_
         uint32_t cur = s_n[0], rounds = 0;
         for (; cur > 0; rounds++) {
             const uint32_t cb = rounds & 1u, nb = cb ^ 1u;
-            for (uint32_t k = tid; k < cur; k += 64u) {
+            for (uint32_t k = tid; k < cur; k += 256u) {
                 const uint32_t pr = s_wl[cb][k], c = pr & 0xffffu, o = pr >> 16;
                 float2 pi = s_p[c], pj = s_p[o];
                 const uint32_t hc = s_head[c], ho = s_head[o];
@@ -711,7 +979,7 @@ __global__ void __launch_bounds__(64) k_cg_lds(float2 *__restrict__ pos, uint32_
             }
             if (tid == 0) s_n[(rounds + 2u) % 3u] = 0u;
             __syncthreads();
-            for (uint32_t k = tid; k < cur; k += 64u) {
+            for (uint32_t k = tid; k < cur; k += 256u) {
                 const uint32_t pr = s_wl[cb][k];
                 for (int e = 0; e < 2; e++) {
                     const uint32_t x = e ? pr >> 16 : pr & 0xffffu, y = s_nxp[x];
@@ -723,7 +991,7 @@ __global__ void __launch_bounds__(64) k_cg_lds(float2 *__restrict__ pos, uint32_
             __syncthreads();
             cur = s_n[(rounds + 1u) % 3u];
         }
-        for (uint32_t k = tid; k < n; k += 64u) {
+        for (uint32_t k = tid; k < n; k += 256u) {
             const uint32_t c = M[k];
             P[c] = s_p[k];
             exc[c] = s_e[k];
@@ -732,7 +1000,7 @@ __global__ void __launch_bounds__(64) k_cg_lds(float2 *__restrict__ pos, uint32_
         __syncthreads();
         if (tid == 0) {
             if (s_bad) atomicOr(&ctl[kCtlBad], 1u);
-            atomicMax(&ctl[kCtlRounds], rounds);
+            note_rounds(ctl, rounds);
         }
         __syncthreads();
     }
@@ -744,34 +1012,31 @@ __global__ void __launch_bounds__(64) k_cg_lds(float2 *__restrict__ pos, uint32_
 // is the next one (kNoneG when done), so (x, y) is ready exactly when
 // nxp[x] == y and nxp[y] == x.  Every round applies at least one pair, so the
 // loop ends; a list left unfinished (a schedule that stalls) is reported.
-__global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ pos, uint32_t cbase,
-                                                      const float *__restrict__ crad, const float2 *__restrict__ save,
-                                                      float *__restrict__ exc, const uint32_t *__restrict__ cnt,
+__global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ P, const float4 *__restrict__ aux,
+                                                      const float4 *__restrict__ rec, float *__restrict__ exc,
+                                                      const uint32_t *__restrict__ cnt,
                                                       const uint32_t *__restrict__ off,
                                                       const uint32_t *__restrict__ cand,
                                                       const uint32_t *__restrict__ csize,
                                                       const uint32_t *__restrict__ cstart,
                                                       const uint32_t *__restrict__ members,
-                                                      const uint32_t *__restrict__ bigq, uint32_t nc,
+                                                      const uint32_t *__restrict__ queues, uint32_t nc,
                                                       uint32_t *__restrict__ head, uint32_t *__restrict__ nxp,
                                                       uint32_t *__restrict__ stamp, uint2 *__restrict__ wl,
                                                       float2 *__restrict__ traj, uint32_t *__restrict__ ctl) {
-    __shared__ uint32_t s_q, s_n[3], s_bad;
+    __shared__ uint32_t s_n[3], s_bad;
     const uint32_t tid = threadIdx.x;
-    const uint32_t nbig = ctl[kCtlNbig];
-    float2 *P = pos + cbase;
-    for (;;) {
-        if (tid == 0) s_q = atomicAdd(&ctl[kCtlQueue], 1u);
-        __syncthreads();
-        const uint32_t q = s_q;
-        if (q >= nbig) break;
+    if (ctl[kCtlFull]) return;  // uniform
+    const uint32_t nbig = ctl[kCtlQueue + kQueueBig];
+    const uint32_t *const bigq = queues + (size_t)kQueueBig * nc;
+    for (uint32_t q = blockIdx.x; q < nbig; q += gridDim.x) {  // uniform per workgroup
         const uint32_t r = bigq[q], base = cstart[r], n = csize[r];
         const uint32_t *M = members + base;
         uint2 *const W[2] = {wl + base, wl + nc + base};
         for (uint32_t k = tid; k < n; k += kCompWG) {
             const uint32_t c = M[k];
             head[c] = 0u;
-            nxp[c] = cnt[c] ? cand[off[c]] : kNoneG;
+            nxp[c] = cnt[c] ? cand[off[c]] & kIdxMaskG : kNoneG;
             stamp[c] = kNoneG;
         }
         if (tid == 0) { s_n[0] = 0u; s_n[1] = 0u; s_n[2] = 0u; s_bad = 0u; }
@@ -790,13 +1055,13 @@ __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ pos, 
                 float2 pi = P[c], pj = P[o];
                 const uint32_t hc = head[c], ho = head[o];
                 const uint32_t oc = off[c], oo = off[o];
-                const uint32_t xc = hc + 1u < cnt[c] ? cand[oc + hc + 1u] : kNoneG;
-                const uint32_t xo = ho + 1u < cnt[o] ? cand[oo + ho + 1u] : kNoneG;
+                const uint32_t xc = hc + 1u < cnt[c] ? cand[oc + hc + 1u] & kIdxMaskG : kNoneG;
+                const uint32_t xo = ho + 1u < cnt[o] ? cand[oo + ho + 1u] & kIdxMaskG : kNoneG;
                 float qi = 0.0f, qj = 0.0f;
-                if (solve_circle_pair(pi.x, pi.y, pj.x, pj.y, crad[c], crad[o], qi, qj)) {
+                if (solve_circle_pair(pi.x, pi.y, pj.x, pj.y, aux[c].x, aux[o].x, qi, qj)) {
                     P[c] = pi;
                     P[o] = pj;
-                    const float2 sc = save[c], so = save[o];
+                    const float4 sc = rec[c], so = rec[o];
                     exc[c] = excursion(exc[c], pi.x, pi.y, sc.x, sc.y);
                     exc[o] = excursion(exc[o], pj.x, pj.y, so.x, so.y);
                 }
@@ -830,58 +1095,61 @@ __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ pos, 
         __syncthreads();
         if (tid == 0) {
             if (s_bad) atomicOr(&ctl[kCtlBad], 1u);
-            atomicMax(&ctl[kCtlRounds], rounds);
+            note_rounds(ctl, rounds);
         }
-        __syncthreads();  // s_q, s_n and s_bad are rewritten for the next component
+        __syncthreads();  // s_n and s_bad are rewritten for the next component
     }
 }
 
-// Validity of the sweep and the circles' needs for the next one.  Circles
-// that went further than 0.9 of their margin are queued in overq, and for each
-// level the largest r + e among them goes to ctl[kCtlEmax + L] (as bits:
-// positive floats order like their bit patterns).  Atomics are taken once per
-// wavefront.
-__global__ void __launch_bounds__(256) k_cg_check(const float *__restrict__ exc, const float *__restrict__ marg,
-                                                  const float *__restrict__ crad, const uint8_t *__restrict__ lvl,
-                                                  float *__restrict__ need, float s0, uint32_t nc,
+// Validity of the sweep, the circles' needs for the next one, and their positions
+// back by circle number.  Circles that went further than 0.9 of their margin are
+// queued in overq, and for each level the largest r + e among them goes to
+// ctl[kCtlEmax + L] (as bits: positive floats order like their bit patterns).
+// Atomics are taken once per workgroup, of kCheckPer slots a thread.
+__global__ void __launch_bounds__(256) k_cg_check(const float *__restrict__ exc, const float4 *__restrict__ aux,
+                                                  const float4 *__restrict__ rec, const float2 *__restrict__ spos,
+                                                  const uint32_t *__restrict__ cnt, float *__restrict__ need, float s0,
+                                                  uint32_t nc, float2 *__restrict__ pos, uint32_t cbase,
                                                   uint32_t *__restrict__ overq, uint32_t *__restrict__ ctl) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t lane = threadIdx.x & 63u;
-    bool over = false, inf = false, quiet = false;
-    uint32_t L = 0, ebits = 0;
-    if (i < nc) {
-        const float e = exc[i];
-        over = !(e <= 0.9f * marg[i]);
-        inf = !(e <= 3.0e38f);
+    __shared__ uint32_t s_emax[kLevels], s_over, s_flags, s_base;
+    const uint32_t tid = threadIdx.x;
+    if (ctl[kCtlFull]) return;  // uniform: nothing was replayed
+    if (tid < (uint32_t)kLevels) s_emax[tid] = 0u;
+    if (tid == 0u) { s_over = 0u; s_flags = 0u; }
+    __syncthreads();
+    uint32_t at[kCheckPer];
+#pragma unroll
+    for (uint32_t u = 0; u < kCheckPer; u++) {
+        const uint32_t s = (blockIdx.x * kCheckPer + u) * 256u + tid;
+        at[u] = kNoneG;
+        if (s >= nc) continue;
+        const float4 a = aux[s], q = rec[s];
+        const uint32_t i = __float_as_uint(q.w) & kIdxMaskG;
+        const float e = exc[s];
+        const bool over = !(e <= 0.9f * a.y), inf = !(e <= 3.0e38f);
         // jammed circles swing from sweep to sweep: the need keeps twice the
         // excursion and forgets slowly
-        if (!inf) need[i] = fmaxf(2.0f * e, 0.9f * need[i]);
-        if (over && !inf) {
-            L = lvl[i];
-            ebits = __float_as_uint(crad[i] + e);
-            quiet = marg[i] <= s0;  // a circle at the base margin overran
+        if (!inf) need[s] = fmaxf(2.0f * e, 0.9f * a.z);
+        if (cnt[s]) pos[cbase + i] = spos[s];
+        if (over) {
+            at[u] = atomicAdd(&s_over, 1u);
+            // (bit 1: a circle at the base margin overran)
+            if (inf) atomicOr(&s_flags, 1u);
+            else atomicMax(&s_emax[__float_as_uint(q.w) >> kLvlShift], __float_as_uint(a.x + e));
+            if (!inf && a.y <= s0) atomicOr(&s_flags, 2u);
         }
     }
-    const uint64_t b = __ballot(over);
-    if (!b) return;  // uniform: the wavefront has no overrun
-    const uint64_t binf = __ballot(inf), bquiet = __ballot(quiet);
-    if (lane == 0u && binf) atomicOr(&ctl[kCtlInf], 1u);
-    if (lane == 0u && bquiet) atomicOr(&ctl[kCtlQuiet], 1u);
-    uint32_t base = 0;
-    if (lane == 0u) base = atomicAdd(&ctl[kCtlOver], (uint32_t)__popcll(b));
-    base = __shfl(base, 0);
-    if (over) overq[base + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = i;
-    // per-level maxima: one atomic per (wavefront, level present)
-    uint64_t todo = __ballot(ebits != 0u);
-    while (todo) {
-        const uint32_t src = (uint32_t)__ffsll((unsigned long long)todo) - 1u;
-        const uint32_t Ls = __shfl(L, (int)src);
-        const bool mine = ebits != 0u && L == Ls;
-        uint32_t m = mine ? ebits : 0u;
-        for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor(m, o));
-        if (lane == src) atomicMax(&ctl[kCtlEmax + Ls], m);
-        todo &= ~__ballot(mine);
-    }
+    __syncthreads();
+    const uint32_t n = s_over;
+    if (n == 0u) return;  // uniform
+    if (tid == 0u) s_base = atomicAdd(&ctl[kCtlOver], n);
+    if (tid == 1u && (s_flags & 1u)) atomicOr(&ctl[kCtlInf], 1u);
+    if (tid == 2u && (s_flags & 2u)) atomicOr(&ctl[kCtlQuiet], 1u);
+    if (tid < (uint32_t)kLevels && s_emax[tid]) atomicMax(&ctl[kCtlEmax + tid], s_emax[tid]);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t u = 0; u < kCheckPer; u++)
+        if (at[u] != kNoneG) overq[s_base + at[u]] = (blockIdx.x * kCheckPer + u) * 256u + tid;
 }
 
 // Exact check of a sweep with overruns, one wavefront per overrunning circle.
@@ -895,92 +1163,98 @@ __global__ void __launch_bounds__(256) k_cg_check(const float *__restrict__ exc,
 // pairs with partners below b, b its pairs with partners below a, and traj
 // holds each circle's position after each of its pairs.  If it overlapped
 // there, the sweep is marked for a redo; otherwise skipping it changed nothing.
-__global__ void __launch_bounds__(256) k_cg_verify(const float2 *__restrict__ save, const float *__restrict__ crad,
+__global__ void __launch_bounds__(256) k_cg_verify(Buckets bk, const float4 *__restrict__ aux,
                                                    const float *__restrict__ exc, const CGrid *__restrict__ g,
-                                                   const uint32_t *__restrict__ start, const float4 *__restrict__ rec,
-                                                   uint32_t nc, uint32_t tmask, const uint32_t *__restrict__ cnt,
-                                                   const uint32_t *__restrict__ off, const uint32_t *__restrict__ cand,
-                                                   const uint32_t *__restrict__ overq, uint32_t n_over,
+                                                   const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
+                                                   const uint32_t *__restrict__ cand,
+                                                   const uint32_t *__restrict__ overq,
                                                    const float2 *__restrict__ traj, uint32_t *__restrict__ ctl) {
-    const uint32_t k = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t lane = threadIdx.x & 63u;
-    if (k >= n_over) return;  // uniform per wavefront
-    const uint32_t i = overq[k];
-    const float2 p = save[i];
-    if (!(fabsf(p.x) <= 3.0e38f && fabsf(p.y) <= 3.0e38f)) return;
-    const float ai = crad[i] + exc[i];
+    const uint32_t n_over = ctl[kCtlFull] ? 0u : ctl[kCtlOver];
     const uint32_t mask = ctl[kCtlMask] | 1u;
-    const uint32_t *const list = cand + off[i];
-    const uint32_t nl = cnt[i];
-    bool missed = false;
-    // entries of a sorted list below v
-    auto rank = [&](const uint32_t *l, uint32_t n, uint32_t v) {
-        uint32_t lo = 0, hi = n;
+    auto number = [&](uint32_t s) { return __float_as_uint(bk.rec[s].w) & kIdxMaskG; };
+    // entries of slot s's list with numbers below v
+    auto rank = [&](uint32_t s, uint32_t v) {
+        const uint32_t *l = cand + off[s];
+        uint32_t lo = 0, hi = cnt[s];
         while (lo < hi) {
             const uint32_t mid = (lo + hi) >> 1;
-            if (l[mid] < v) lo = mid + 1u; else hi = mid;
+            if (number(l[mid] & kIdxMaskG) < v) lo = mid + 1u; else hi = mid;
         }
         return lo;
     };
-    auto test = [&](uint32_t j, float qx, float qy) {
-        const float lim = (ai + (crad[j] + exc[j])) * (1.0f + 0x1p-16f);
-        const float dx = p.x - qx, dy = p.y - qy;
-        if (!(dx * dx + dy * dy < lim * lim)) return;
-        const uint32_t ri = rank(list, nl, j);
-        if (ri < nl && list[ri] == j) return;  // listed: replayed in order
-        const uint32_t a = min(i, j), b = max(i, j);
-        const uint32_t ka = a == i ? ri : rank(cand + off[a], cnt[a], b);
-        const uint32_t kb = b == i ? ri : rank(cand + off[b], cnt[b], a);
-        const float2 pa = ka ? traj[off[a] + ka - 1u] : save[a];
-        const float2 pb = kb ? traj[off[b] + kb - 1u] : save[b];
-        const float ex = pa.x - pb.x, ey = pa.y - pb.y;
-        const float rs = crad[a] + crad[b];
-        if (ex * ex + ey * ey < rs * rs) missed = true;
-    };
-    auto reach_at = [&](uint32_t L) {
-        return ((double)ai + (double)fmaxf(g->reach_max[L], __uint_as_float(ctl[kCtlEmax + L]))) * (1.0 + 1e-4);
-    };
-    bool brute = false;
-    for (uint32_t m = mask; m; m &= m - 1u) {
-        const uint32_t L = (uint32_t)__ffs(m) - 1u;
-        const double R = reach_at(L), ih = g->inv_h[L];
-        const int64_t nx = (int64_t)cell_coord_d((double)p.x + R, ih) - cell_coord_d((double)p.x - R, ih) + 1;
-        const int64_t ny = (int64_t)cell_coord_d((double)p.y + R, ih) - cell_coord_d((double)p.y - R, ih) + 1;
-        if (nx * ny > kMaxScanCells) brute = true;
-    }
-    if (brute) {
-        for (uint32_t j = lane; j < nc; j += 64u) {
-            if (j == i) continue;
-            const float2 q = save[j];
-            test(j, q.x, q.y);
-        }
-    } else {
+    bool missed = false;
+    for (uint32_t k = (blockIdx.x * 256u + threadIdx.x) >> 6; k < n_over; k += gridDim.x * 4u) {  // uniform per wavefront
+        const uint32_t i = overq[k];
+        const float4 p = bk.rec[i];
+        if (!(fabsf(p.x) <= 3.0e38f && fabsf(p.y) <= 3.0e38f)) continue;
+        const float ai = aux[i].x + exc[i];
+        const uint32_t ni = __float_as_uint(p.w) & kIdxMaskG;
+        // a record's own reach covers r + e of a circle within its margin, the
+        // level's largest r + e that of an overrun
+        auto near_at = [&](float emax) {
+            return [=](const float4 &q) {
+                const float lim = (ai + fmaxf(q.z, emax)) * (1.0f + 0x1p-15f);
+                const float dx = p.x - q.x, dy = p.y - q.y;
+                return dx * dx + dy * dy < lim * lim;
+            };
+        };
+        auto test = [&](uint32_t j, const float4 &q) {
+            if (j == i) return;
+            const float lim = (ai + (aux[j].x + exc[j])) * (1.0f + 0x1p-16f);
+            const float dx = p.x - q.x, dy = p.y - q.y;
+            if (!(dx * dx + dy * dy < lim * lim)) return;
+            const uint32_t nj = __float_as_uint(q.w) & kIdxMaskG;
+            const uint32_t ri = rank(i, nj);
+            if (ri < cnt[i] && (cand[off[i] + ri] & kIdxMaskG) == j) return;  // listed: replayed in order
+            const uint32_t rj = rank(j, ni);
+            const float2 pi = ri ? traj[off[i] + ri - 1u] : make_float2(p.x, p.y);
+            const float2 pj = rj ? traj[off[j] + rj - 1u] : make_float2(q.x, q.y);
+            const bool first = ni < nj;
+            const float2 pa = first ? pi : pj, pb = first ? pj : pi;
+            const float ex = pa.x - pb.x, ey = pa.y - pb.y;
+            const float rs = first ? aux[i].x + aux[j].x : aux[j].x + aux[i].x;
+            if (ex * ex + ey * ey < rs * rs) missed = true;
+        };
+        auto reach_at = [&](uint32_t L) {
+            return ((double)ai + (double)fmaxf(g->reach_max[L], __uint_as_float(ctl[kCtlEmax + L]))) * (1.0 + 1e-4);
+        };
+        bool brute = false;
         for (uint32_t m = mask; m; m &= m - 1u) {
             const uint32_t L = (uint32_t)__ffs(m) - 1u;
             const double R = reach_at(L), ih = g->inv_h[L];
+            const int64_t nx = (int64_t)cell_coord_d((double)p.x + R, ih) - cell_coord_d((double)p.x - R, ih) + 1;
+            const int64_t ny = (int64_t)cell_coord_d((double)p.y + R, ih) - cell_coord_d((double)p.y - R, ih) + 1;
+            if (nx * ny > kMaxScanCells) brute = true;
+        }
+        if (brute) {
+            for (uint32_t j = lane; j < bk.nc; j += 64u) test(j, bk.rec[j]);
+            continue;
+        }
+        for (uint32_t m = mask; m; m &= m - 1u) {
+            const uint32_t L = (uint32_t)__ffs(m) - 1u;
+            const double R = reach_at(L), ih = g->inv_h[L];
+            const auto near = near_at(__uint_as_float(ctl[kCtlEmax + L]));
             const int x0 = cell_coord_d((double)p.x - R, ih), x1 = cell_coord_d((double)p.x + R, ih);
             const int y0 = cell_coord_d((double)p.y - R, ih), y1 = cell_coord_d((double)p.y + R, ih);
-            const uint32_t w = (uint32_t)(x1 - x0 + 1), cells = w * (uint32_t)(y1 - y0 + 1);
-            for (uint32_t c = lane; c < cells; c += 64u) {
-                const int cx = x0 + (int)(c % w), cy = y0 + (int)(c / w);
-                const uint32_t kb = level_hash(L, cx, cy) & tmask;
-                for (uint32_t s = start[kb], e = start[kb + 1]; s < e; s++) {
-                    const float4 q = rec[s];
-                    const uint32_t wq = __float_as_uint(q.w);
-                    const uint32_t j = wq & kIdxMaskG;
-                    if ((wq >> kLvlShift) != L || j == i) continue;
-                    if (cell_coord(q.x, ih) != cx || cell_coord(q.y, ih) != cy) continue;
-                    test(j, q.x, q.y);
-                }
+            // rows over the lanes, each cut into pieces of 4 cells
+            const uint32_t pieces = (uint32_t)(x1 - x0 + 4) >> 2, items = pieces * (uint32_t)(y1 - y0 + 1);
+            for (uint32_t c = lane; c < items; c += 64u) {
+                const int cx = x0 + (int)(c % pieces) * 4;
+                const int cy = y0 + (int)(c / pieces);
+                scan_rows(bk, L, cx, min(cx + 3, x1), cy, cy, 1, ih, near, test);
             }
         }
     }
     if (missed) atomicOr(&ctl[kCtlMissed], 1u);
 }
 
-__global__ void k_cc_restore(float2 *__restrict__ pos, uint32_t cbase, const float2 *__restrict__ save, uint32_t nc) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nc) pos[cbase + i] = save[i];
+// The positions that the sweep started from, back by circle number.
+__global__ void k_cc_restore(float2 *__restrict__ pos, uint32_t cbase, const float4 *__restrict__ rec, uint32_t nc) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nc) return;
+    const float4 q = rec[s];
+    pos[cbase + (__float_as_uint(q.w) & kIdxMaskG)] = make_float2(q.x, q.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -1093,6 +1367,10 @@ public:
         clean_ = 0;
         BD_HIP(cg_need_.alloc(std::max<uint32_t>(Nc_, 1)));
         if (Nc_) BD_HIP(hipMemsetAsync(cg_need_.p, 0, Nc_ * sizeof(float), stream_));
+        BD_HIP(cg_order_.alloc(std::max<uint32_t>(Nc_, 1)));
+        std::vector<uint32_t> order(Nc_);
+        for (uint32_t i = 0; i < Nc_; i++) order[i] = i;
+        if (Nc_) BD_HIP(hipMemcpyAsync(cg_order_.p, order.data(), Nc_ * 4, hipMemcpyHostToDevice, stream_));
         // the upload copies read host vectors that die at return
         BD_HIP(hipStreamSynchronize(stream_));
         return BD_OK;
@@ -1196,71 +1474,80 @@ private:
         const uint32_t nc = Nc_;
         const uint32_t nb = (nc + 255) / 256;
         uint32_t T = 1;
-        while (T < 2 * nc) T <<= 1;
-        const uint32_t tmask = T - 1;
-        // counters and control words, zeroed by one fill per attempt
-        const size_t zn = (size_t)(T + 1) + T + (nc + 1) + nc + kCtlWords;
-        BD_HIP(cg_zero_.alloc(zn));
-        uint32_t *const count = cg_zero_.p, *const fill = count + T + 1, *const csize = fill + T;
-        uint32_t *const cfill = csize + nc + 1, *const ctl = cfill + nc;
-        BD_HIP(cg_grid_.alloc(1));
-        BD_HIP(cc_save_.alloc(nc)); BD_HIP(cg_exc_.alloc(nc)); BD_HIP(cg_marg_.alloc(nc)); BD_HIP(cg_reach_.alloc(nc));
-        BD_HIP(cg_lvl_.alloc(nc)); BD_HIP(cc_key_.alloc(nc)); BD_HIP(cg_par_.alloc(nc)); BD_HIP(cg_root_.alloc(nc));
-        BD_HIP(cc_start_.alloc(T + 1)); BD_HIP(cg_rec_.alloc(nc));
-        BD_HIP(cc_cnt_.alloc(nc + 1)); BD_HIP(cc_off_.alloc(nc + 1));
-        BD_HIP(cg_cstart_.alloc(nc + 1)); BD_HIP(cg_members_.alloc(nc)); BD_HIP(cg_bigq_.alloc(nc));
-        BD_HIP(cc_head_.alloc(nc)); BD_HIP(cg_nxp_.alloc(nc)); BD_HIP(cg_stamp_.alloc(nc));
-        BD_HIP(cg_wl_.alloc(2 * (size_t)nc)); BD_HIP(cg_overq_.alloc(nc));
-        BD_HIP(cg_midq_.alloc(nc)); BD_HIP(cg_slot_.alloc(nc)); BD_HIP(cg_keep_.alloc((size_t)nc * kSlotG));
+        while (T < nc) T <<= 1;
+        const uint32_t tmask = T - 1, stride = (uint32_t)(0.618034 * (double)T) | 1u;
+        // control words and bucket counters, zeroed by one fill per attempt (the
+        // scan's last entry with them)
+        const size_t zn = kCtlWords + (size_t)T + 1;
+        const int rw = place_workspace(nc, T, zn, err);
+        if (rw) return rw;
+        uint32_t *const ctl = ws_.zero, *const count = ctl + kCtlWords;
+        if (!cand_cap_) cand_cap_ = std::max<uint64_t>(4ull * nc, 1024);
         for (int attempt = 0; attempt < 12; attempt++) {
-            fill_u32(cg_zero_.p, zn, 0u, st);
-            hipLaunchKernelGGL(k_cg_grid, dim3(1), dim3(32), 0, stream_, s0_, rmax_, cg_grid_.p);
-            hipLaunchKernelGGL(k_cg_prep, dim3(nb), dim3(256), 0, stream_, pos_.p, Np_, crad_.p, cg_need_.p, cg_grid_.p,
-                               nc, tmask, cc_save_.p, cg_exc_.p, cg_marg_.p, cg_reach_.p, cg_lvl_.p, cc_key_.p, count,
-                               cg_par_.p, ctl);
-            st.launches += 2;
-            int rc = exclusive_scan_u32(count, cc_start_.p, T + 1, stream_, scan_tmp_, st.launches, err);
+            BD_HIP(cc_cand_.alloc(cand_cap_));
+            BD_HIP(cg_traj_.alloc(cand_cap_));
+            // Level 0 takes margins up to 1.5 r_max, also while the base margin is
+            // less: circles in lasting contact need more than the base, and on level
+            // 1 each scans 5x5 cells of level 0 (limit s0 17.4 ms, 0.5 r_max 16.9, 1.0
+            // to 2.0 16.4 for 262,144 circles).
+            const float lim0 = std::max(s0_, 1.5f * rmax_);
+            fill_u32(ws_.zero, zn, 0u, st);
+            hipLaunchKernelGGL(k_cg_prep, dim3(nb), dim3(256), 0, stream_, pos_.p, Np_, cg_need_.p, cg_order_.p, s0_,
+                               lim0, rmax_, nc,
+                               tmask, stride, ws_.grid, ws_.key, count, ctl);
+            st.launches++;
+            int rc = exclusive_scan_u32(count, ws_.start, T + 1, stream_, scan_tmp_, st.launches, err);
             if (rc) return rc;
-            hipLaunchKernelGGL(k_cg_scatter, dim3(nb), dim3(256), 0, stream_, cc_save_.p, cg_reach_.p, cg_lvl_.p,
-                               cc_key_.p, nc, cc_start_.p, fill, cg_rec_.p);
-            hipLaunchKernelGGL(k_cg_cand<0>, dim3(nb), dim3(256), 0, stream_, cc_save_.p, cg_reach_.p, cg_lvl_.p,
-                               cg_grid_.p, ctl, cc_start_.p, cg_rec_.p, nc, tmask, cc_cnt_.p, nullptr, nullptr,
-                               cg_keep_.p);
-            st.launches += 2;
-            rc = exclusive_scan_u32(cc_cnt_.p, cc_off_.p, nc + 1, stream_, scan_tmp_, st.launches, err);
-            if (rc) return rc;
-            // total candidate entries -> size the list
-            BD_HIP(hipMemcpyAsync(host_ctl_, cc_off_.p + nc, 4, hipMemcpyDeviceToHost, stream_));
-            BD_HIP(hipStreamSynchronize(stream_));
-            const uint32_t total = host_ctl_[0];
-            BD_HIP(cc_cand_.alloc(std::max<uint32_t>(total, 1)));
-            BD_HIP(cg_traj_.alloc(std::max<uint32_t>(total, 1)));
-            hipLaunchKernelGGL(k_cg_cand<1>, dim3(nb), dim3(256), 0, stream_, cc_save_.p, cg_reach_.p, cg_lvl_.p,
-                               cg_grid_.p, ctl, cc_start_.p, cg_rec_.p, nc, tmask, cc_cnt_.p, cc_off_.p, cc_cand_.p,
-                               cg_keep_.p);
-            hipLaunchKernelGGL(k_cg_union, dim3(nb), dim3(256), 0, stream_, cc_cnt_.p, cc_off_.p, cc_cand_.p, nc,
-                               cg_par_.p);
-            hipLaunchKernelGGL(k_cg_comp, dim3(nb), dim3(256), 0, stream_, cc_cnt_.p, nc, cg_par_.p, cg_root_.p, csize);
-            st.launches += 3;
-            rc = exclusive_scan_u32(csize, cg_cstart_.p, nc + 1, stream_, scan_tmp_, st.launches, err);
-            if (rc) return rc;
-            hipLaunchKernelGGL(k_cg_members, dim3(nb), dim3(256), 0, stream_, cc_cnt_.p, cg_root_.p, csize,
-                               cg_cstart_.p, nc, cfill, cg_members_.p, cg_midq_.p, cg_bigq_.p, ctl);
-            hipLaunchKernelGGL(k_cg_lane, dim3(nb), dim3(256), 0, stream_, pos_.p, Np_, crad_.p, cc_save_.p, cg_exc_.p,
-                               cc_cnt_.p, cc_off_.p, cc_cand_.p, cg_root_.p, csize, cg_cstart_.p, cg_members_.p, nc,
-                               cc_head_.p, cg_traj_.p);
-            hipLaunchKernelGGL(k_cg_lds, dim3(kLdsGrid), dim3(64), 0, stream_, pos_.p, Np_, crad_.p, cg_exc_.p,
-                               cc_save_.p, cc_cnt_.p, cc_off_.p, cc_cand_.p, csize, cg_cstart_.p, cg_members_.p,
-                               cg_midq_.p, cg_bigq_.p, cg_slot_.p, cg_traj_.p, ctl);
-            hipLaunchKernelGGL(k_cg_comps, dim3(kCompGrid), dim3(kCompWG), 0, stream_, pos_.p, Np_, crad_.p,
-                               cc_save_.p, cg_exc_.p, cc_cnt_.p, cc_off_.p, cc_cand_.p, csize, cg_cstart_.p,
-                               cg_members_.p, cg_bigq_.p, nc, cc_head_.p, cg_nxp_.p, cg_stamp_.p, cg_wl_.p,
+            hipLaunchKernelGGL(k_cg_scatter, dim3(nb), dim3(256), 0, stream_, pos_.p, Np_, crad_.p, cg_need_.p, cg_order_.p,
+                               s0_, lim0, ws_.key, nc, ws_.start, ws_.rec, ws_.aux);
+            const Buckets bk{nc, tmask, stride, ws_.start, ws_.rec};
+            hipLaunchKernelGGL(k_cg_cand, dim3(nb), dim3(256), 0, stream_, bk, ws_.grid, (uint32_t)cand_cap_, ws_.cnt,
+                               ws_.off, cc_cand_.p, (uint64_t *)cg_traj_.p, ws_.par, ws_.csize, ws_.spos,
+                               ws_.exc, cg_order_.p, ws_.aux, cg_need_.p, ctl);
+            hipLaunchKernelGGL(k_cg_union, dim3(nb), dim3(256), 0, stream_, ws_.cnt, ws_.off, cc_cand_.p, nc,
+                               ws_.par, ctl);
+            hipLaunchKernelGGL(k_cg_comp, dim3(nb), dim3(256), 0, stream_, ws_.cnt, nc, ws_.par, ws_.root,
+                               ws_.place, ws_.csize, ctl);
+            hipLaunchKernelGGL(k_cg_ranges, dim3((nb + kCheckPer - 1) / kCheckPer), dim3(256), 0, stream_, ws_.csize, nc, ws_.cstart,
+                               ws_.queues, ctl);
+            hipLaunchKernelGGL(k_cg_members, dim3(nb), dim3(256), 0, stream_, ws_.cnt, ws_.root, ws_.place,
+                               ws_.cstart, nc, ws_.members, ctl);
+            // (a component for W lanes has more than W / 4 circles, one for 4 at least two)
+            LaneBlocks blk;
+            blk.end64 = std::min<uint32_t>(kLaneGrid, nc / 17 + 1);
+            blk.end16 = blk.end64 + std::min<uint32_t>(kLaneGrid, nc / 5 / 4 + 1);
+            blk.end4 = blk.end16 + std::min<uint32_t>(kLaneGrid, nc / 2 / 16 + 1);
+            hipLaunchKernelGGL(k_cg_lanes, dim3(blk.end4), dim3(64), 0, stream_, ws_.spos, ws_.aux, ws_.rec,
+                               ws_.exc, ws_.cnt, ws_.off, cc_cand_.p, ws_.csize, ws_.cstart, ws_.members,
+                               ws_.place, ws_.queues, nc, blk, cg_traj_.p, ctl);
+            hipLaunchKernelGGL(k_cg_lds, dim3(std::min<uint32_t>(kLdsGrid, nc / 65 + 1)), dim3(256), 0, stream_,
+                               ws_.spos, ws_.aux, ws_.rec, ws_.exc, ws_.cnt, ws_.off, cc_cand_.p,
+                               ws_.csize, ws_.cstart, ws_.members, ws_.place, ws_.queues, nc, cg_traj_.p, ctl);
+            hipLaunchKernelGGL(k_cg_comps, dim3(kCompGrid), dim3(kCompWG), 0, stream_, ws_.spos, ws_.aux, ws_.rec,
+                               ws_.exc, ws_.cnt, ws_.off, cc_cand_.p, ws_.csize, ws_.cstart,
+                               ws_.members, ws_.queues, nc, ws_.head, ws_.nxp, ws_.stamp, ws_.wl,
                                cg_traj_.p, ctl);
-            hipLaunchKernelGGL(k_cg_check, dim3(nb), dim3(256), 0, stream_, cg_exc_.p, cg_marg_.p, crad_.p, cg_lvl_.p,
-                               cg_need_.p, s0_, nc, cg_overq_.p, ctl);
-            st.launches += 5;
+            hipLaunchKernelGGL(k_cg_check, dim3((nb + kCheckPer - 1) / kCheckPer), dim3(256), 0, stream_, ws_.exc,
+                               ws_.aux, ws_.rec, ws_.spos, ws_.cnt, cg_need_.p, s0_, nc, pos_.p, Np_,
+                               ws_.overq, ctl);
+            hipLaunchKernelGGL(k_cg_verify, dim3(std::min<uint32_t>(nb, kVerifyGrid)), dim3(256), 0, stream_, bk,
+                               ws_.aux, ws_.exc, ws_.grid, ws_.cnt, ws_.off, cc_cand_.p, ws_.overq,
+                               cg_traj_.p, ctl);
+            st.launches += 11;
             BD_HIP(hipMemcpyAsync(host_ctl_, ctl, kCtlWords * sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
             BD_HIP(hipStreamSynchronize(stream_));
+            uint64_t total;
+            std::memcpy(&total, host_ctl_ + kCtlTotal, sizeof total);
+            if (host_ctl_[kCtlFull]) {
+                // nothing was replayed: the same attempt again, with room
+                if (total + total / 4 > 0xffffffffull) {
+                    err = "too many candidate circle pairs";
+                    return BD_ERR_CAPACITY;
+                }
+                cand_cap_ = total + total / 4;
+                attempt--;
+                continue;
+            }
             st.cc_pairs = total / 2;
             st.cc_rounds += host_ctl_[kCtlRounds];
             if (host_ctl_[kCtlBad]) {
@@ -1271,19 +1558,7 @@ private:
                 err = "circle pair sweep produced a non-finite push";
                 return BD_ERR_COLLISION;
             }
-            const uint32_t n_over = host_ctl_[kCtlOver];
-            bool missed = false;
-            if (n_over) {
-                hipLaunchKernelGGL(k_cg_verify, dim3((n_over + 3) / 4), dim3(256), 0, stream_, cc_save_.p, crad_.p,
-                                   cg_exc_.p, cg_grid_.p, cc_start_.p, cg_rec_.p, nc, tmask, cc_cnt_.p, cc_off_.p,
-                                   cc_cand_.p, cg_overq_.p, n_over, cg_traj_.p, ctl);
-                st.launches++;
-                BD_HIP(hipMemcpyAsync(host_ctl_ + kCtlMissed, ctl + kCtlMissed, sizeof(uint32_t),
-                                      hipMemcpyDeviceToHost, stream_));
-                BD_HIP(hipStreamSynchronize(stream_));
-                missed = host_ctl_[kCtlMissed] != 0u;
-            }
-            if (!missed) {
+            if (!host_ctl_[kCtlMissed]) {
                 // quiet sweeps let the base margin shrink back
                 if (++clean_ >= 16) {
                     s0_ = std::max(0.8f * s0_, s0_min());
@@ -1294,7 +1569,7 @@ private:
             }
             // a skipped pair may have met: undo, widen, redo
             st.cc_redos++;
-            hipLaunchKernelGGL(k_cc_restore, dim3(nb), dim3(256), 0, stream_, pos_.p, Np_, cc_save_.p, nc);
+            hipLaunchKernelGGL(k_cc_restore, dim3(nb), dim3(256), 0, stream_, pos_.p, Np_, ws_.rec, nc);
             st.launches++;
             clean_ = 0;
             // capped at 0.75 r_max: measured best over the gas box's run (0.25-1.0)
@@ -1304,6 +1579,42 @@ private:
         return BD_ERR_COLLISION;
     }
 
+    // The sweep's workspace, one allocation: 22 of them, and as many releases, took
+    // 1.5 to 4 ms of a scene's life (a clone rolled out for 32 sweeps: 16 ms).
+    struct Workspace {
+        uint32_t *zero, *start, *cnt, *off, *par, *root, *place, *csize, *cstart, *members, *queues, *overq, *head, *nxp,
+            *stamp;
+        float *exc;
+        float2 *spos;
+        float4 *rec, *aux;
+        uint2 *key, *wl;
+        CGrid *grid;
+    };
+
+    int place_workspace(uint32_t nc, uint32_t T, size_t zn, std::string &err) {
+        size_t at = 0;
+        auto take = [&](auto *&p, size_t count) {
+            using V = std::remove_reference_t<decltype(*p)>;
+            p = cg_arena_.p ? (V *)(cg_arena_.p + at) : nullptr;
+            at += (count * sizeof(V) + 255) & ~(size_t)255;
+        };
+        auto all = [&]() {
+            at = 0;
+            take(ws_.zero, zn);
+            take(ws_.grid, 1);
+            take(ws_.key, nc); take(ws_.start, (size_t)T + 1); take(ws_.rec, nc); take(ws_.aux, nc);
+            take(ws_.spos, nc); take(ws_.exc, nc); take(ws_.cnt, nc); take(ws_.off, nc);
+            take(ws_.par, nc); take(ws_.root, nc); take(ws_.place, nc); take(ws_.csize, nc);
+            take(ws_.cstart, nc); take(ws_.members, nc); take(ws_.queues, kQueues * (size_t)nc);
+            take(ws_.overq, nc); take(ws_.head, nc); take(ws_.nxp, nc); take(ws_.stamp, nc);
+            take(ws_.wl, 2 * (size_t)nc);
+        };
+        all();
+        BD_HIP(cg_arena_.alloc(at));
+        all();
+        return BD_OK;
+    }
+
     float s0_min() const { return 0.05f * std::max(rmax_, 1e-3f); }
 
     void fill_u32(uint32_t *p, size_t n, uint32_t v, Stats &st) {
@@ -1311,7 +1622,7 @@ private:
         st.launches++;
     }
 
-    static constexpr uint32_t kCompGrid = 256, kLdsGrid = 16384;
+    static constexpr uint32_t kCompGrid = 256, kLdsGrid = 512, kLaneGrid = 8192, kVerifyGrid = 1024;
     hipStream_t stream_;
     uint32_t Np_ = 0, Nc_ = 0, Ng_ = 0, N_ = 0, P_ = 0, depth_ = 0, ncol_ = 0, nplanes_ = 0;
     bool has_pins_ = false;
@@ -1328,14 +1639,14 @@ private:
     DevBuf<int4> colhdr_;
     DevBuf<float4> colgeo_, planes_;
     // circle schedule workspace
-    DevBuf<CGrid> cg_grid_;
-    DevBuf<uint32_t> cg_zero_, cc_key_, cc_cnt_, cc_off_, cc_head_, cc_start_, cc_cand_;
-    DevBuf<uint32_t> cg_par_, cg_root_, cg_cstart_, cg_members_, cg_bigq_, cg_nxp_, cg_stamp_, cg_overq_, cg_midq_, cg_slot_, cg_keep_;
-    DevBuf<float2> cc_save_, cg_traj_;
-    DevBuf<float> cg_need_, cg_exc_, cg_marg_, cg_reach_;
-    DevBuf<uint8_t> cg_lvl_;
-    DevBuf<float4> cg_rec_;
-    DevBuf<uint2> cg_wl_;
+    DevBuf<uint8_t> cg_arena_;
+    Workspace ws_;
+    DevBuf<uint32_t> cc_cand_;
+    DevBuf<float2> cg_traj_;
+    // by slot of the last sweep: the circles (by number after an upload), their needs
+    DevBuf<uint32_t> cg_order_;
+    DevBuf<float> cg_need_;
+    uint64_t cand_cap_ = 0;  // list entries there is room for
     ScanTemp scan_tmp_;
     uint32_t *host_ctl_ = nullptr;
 };

@@ -1,0 +1,69 @@
+"""Circle-pair sweeps of the GLOBAL engine against the f32 oracle bit for bit:
+components at the edges of the replays (4, 16 and 64 lanes, workgroups in LDS and
+in memory), lists at the edges of what they hold, more list entries than there was
+room for, circles that scan their cells alone, by 16 lanes and over every record."""
+import numpy as np
+import pytest
+
+from helpers import bits_equal, first_diff, state, to_oracle
+from bendy2d_amd import BD_ENGINE_GLOBAL, Solver
+
+pytestmark = pytest.mark.gpu
+
+DT = 1.0 / 60.0
+
+
+def check(circles, updates, span):
+    s = Solver()
+    s.set_engine(BD_ENGINE_GLOBAL)
+    s.gravity, s.bounds = (0.0, 0.0), ((-span, -span), (2 * span, 2 * span))
+    s.set_sub_steps(2)
+    s.add_circles(circles)
+    o = to_oracle(s, 32, candidate_mode=len(circles) > 2000)
+    for _ in range(updates):
+        s.update(DT)
+        assert o.update(DT) == 0
+        assert s.engine_used == BD_ENGINE_GLOBAL
+    assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
+
+
+def at(xy, r):
+    c = np.zeros((len(xy), 7), np.float32)
+    c[:, 0:2] = c[:, 2:4] = xy
+    c[:, 6] = r
+    return c
+
+
+@pytest.mark.parametrize("size", [2, 3, 4, 5, 15, 16, 17, 63, 64, 65, 200, 1024, 1025])
+def test_chains(size):
+    # rows of `size` circles, each overlapping the next, far apart, in an order
+    # that is not the rows'
+    rows = max(2, 130 // size)
+    xy = np.array([(0.9 * k, 20.0 * r + 0.05 * (k % 3)) for r in range(rows) for k in range(size)], np.float32)
+    rng = np.random.default_rng(size)
+    check(at(xy[rng.permutation(len(xy))], 0.5), 2, 5000.0)
+
+
+@pytest.mark.parametrize("n", [8, 9, 10, 33, 34, 64, 90, 92, 300])
+def test_clumps(n):
+    # everything touches everything: lists of n - 1 entries (kept by the counting
+    # scan up to 8, by a lane up to 32, by a workgroup up to 8,192 in all), beside
+    # a few loose pairs; 300: more entries than there was room for
+    rng = np.random.default_rng(n)
+    xy = np.concatenate([rng.uniform(-0.3, 0.3, (n, 2)), [(50.0, 0.0), (50.9, 0.0), (-40.0, 7.0), (-40.0, 7.5)]])
+    check(at(xy.astype(np.float32), 1.0), 3, 1000.0)
+
+
+@pytest.mark.parametrize("n", [2, 3, 7, 16, 17, 257, 4097])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_levels(n, mixed):
+    # a gas in which some circles are shot through the others (large pushes and
+    # margins) and, mixed, radii from 0.02 to 8; one circle far away
+    rng = np.random.default_rng(n)
+    span = 2.0 * np.sqrt(n)
+    r = np.where(rng.uniform(size=n) < 0.01, 8.0, rng.uniform(0.02, 0.6, n)) if mixed else np.full(n, 0.5)
+    c = at(rng.uniform(0.0, span, (n, 2)).astype(np.float32), r)
+    speed = np.where(rng.uniform(size=n) < 0.1, 60.0, 1.0)[:, None]
+    c[:, 2:4] -= (speed * rng.standard_normal((n, 2)) * DT / 2).astype(np.float32)
+    c[0, 0:4] += 3000.0
+    check(c, 3, 5000.0)
