@@ -159,7 +159,22 @@ public:
     int upload(const HostScene &s, const Plan &p, std::string &err) override {
         const uint32_t region_cap = kMaxRegionBytes / 8;
         TilePlan tp;
-        int rc = build_tile_plan(s, p, tile_points_, region_cap, tp, err);
+        // Unless the caller has set it, the tile is the smallest with which every
+        // tile still has a CU of its own, 512 to 2,048 points: a pass takes as long
+        // as one tile's layers, each a barrier and the links of a region over the
+        // lanes (3 substeps of 5 sweeps, 66,887 points 146 us with 2,048-point
+        // tiles, 103 with 512; 262,144 139 and 116 with 1,024, 134 with 512; 524,176
+        // 158, 177 and 267).  Tiles that share a CU, and halos that outgrow them (a
+        // deep link graph), cost more than smaller ones give.
+        uint32_t points = tile_points_;
+        if (!points) {
+            int dev = 0, cus = 0;
+            BD_HIP(hipGetDevice(&dev));
+            BD_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+            points = 512;
+            while (points < 2048 && ((uint64_t)p.N > (uint64_t)points * (uint32_t)cus || p.depth > kShallow)) points *= 2;
+        }
+        int rc = build_tile_plan(s, p, points, region_cap, tp, err);
         if (rc) return rc;
         N_ = p.N;
         perm_ = tp.perm;
@@ -305,6 +320,7 @@ public:
     }
 
     static constexpr int kMaxRegionBytes = 128 * 1024;
+    static constexpr uint32_t kShallow = 32;  // link layers
 
 private:
     hipStream_t stream_;
@@ -325,7 +341,7 @@ bool tiled_engine_fits(const HostScene &s, const Plan &p) {
 }
 
 Engine *make_tiled_engine(hipStream_t s, uint32_t tile_points, uint32_t wg) {
-    return new TiledEngine(s, tile_points ? tile_points : 2048, wg ? wg : 1024);
+    return new TiledEngine(s, tile_points, wg ? wg : 1024);
 }
 
 }  // namespace bd

@@ -59,7 +59,7 @@ struct bd_solver {
     int32_t engine_used = 0;
     // TILED shape: 2,048-point tiles, two workgroups of 1,024 per CU on the
     // 1024x1024 cloth (measured fastest of 1,024..8,192 points x 256..1,024 lanes)
-    uint32_t tile_points = 2048, tile_wg = 1024;
+    uint32_t tile_points = 0, tile_wg = 1024;  // (0: the engine chooses)
     hipStream_t stream = nullptr;
     int device = -1;
     Stats stats;

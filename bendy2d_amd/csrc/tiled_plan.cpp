@@ -60,29 +60,32 @@ bool build_pass(const Plan &p, const TilePlan &tp, const Incidence &inc, const s
     out = TilePass();
     out.L0 = L0; out.L1 = L1;
     std::vector<uint32_t> R;
-    std::vector<uint32_t> E;
+    std::vector<uint32_t> cur;  // per region point: end of its links of the layers not yet taken
     std::vector<std::vector<uint32_t>> per_layer(nl);
+    std::vector<uint32_t> dealt;
     for (uint32_t t = 0; t < tp.ntiles; t++) {
         const uint32_t s0 = t * T, s1 = std::min(N, s0 + T);
         const uint32_t stamp = ++stamp_base;
         R.clear();
-        for (uint32_t q = s0; q < s1; q++) { loc[q] = (int32_t)(q - s0); R.push_back(q); }
+        cur.clear();
+        for (uint32_t q = s0; q < s1; q++) { loc[q] = (int32_t)(q - s0); R.push_back(q); cur.push_back(inc.off[q + 1]); }
         for (auto &v : per_layer) v.clear();
         bool ok = true;
         for (uint32_t d = L1; d-- > L0;) {
             const size_t rn = R.size();
             for (size_t i = 0; i < rn; i++) {
                 const uint32_t q = R[i];
-                // the (at most one) link of layer d at point q
-                const uint32_t *b = inc.link.data() + inc.off[q], *e = inc.link.data() + inc.off[q + 1];
-                const uint32_t *it = std::lower_bound(b, e, d, [&](uint32_t k, uint32_t dd) { return link_layer[k] < dd; });
-                if (it == e || link_layer[*it] != d) continue;
-                const uint32_t k = *it;
+                // the (at most one) link of layer d at point q: its lists ascend by
+                // layer, and d only falls
+                uint32_t &at = cur[i];
+                while (at > inc.off[q] && link_layer[inc.link[at - 1]] > d) at--;
+                if (at == inc.off[q] || link_layer[inc.link[at - 1]] != d) continue;
+                const uint32_t k = inc.link[at - 1];
                 if (lstamp[k] == stamp) continue;
                 lstamp[k] = stamp;
                 per_layer[d - L0].push_back(k);
                 const uint32_t o = ia[k] == q ? ib[k] : ia[k];
-                if (loc[o] < 0) { loc[o] = (int32_t)R.size(); R.push_back(o); }
+                if (loc[o] < 0) { loc[o] = (int32_t)R.size(); R.push_back(o); cur.push_back(inc.off[o + 1]); }
             }
             if (((R.size() + 15) & ~size_t(15)) > region_cap) { ok = false; break; }  // slots fill whole blocks of 16
         }
@@ -103,13 +106,16 @@ bool build_pass(const Plan &p, const TilePlan &tp, const Incidence &inc, const s
                 // free: deal them out by the bank of their first end (slot
                 // mod 16, one 8-byte slot spans two banks), so that
                 // neighbouring lanes load from different banks.
-                std::vector<uint32_t> by_bank[16];
-                for (uint32_t k : v) by_bank[region_slot((uint32_t)loc[ia[k]]) & 15u].push_back(k);
-                size_t at[16] = {};
+                uint32_t at[17] = {}, end[16];
+                auto bank = [&](uint32_t k) { return region_slot((uint32_t)loc[ia[k]]) & 15u; };
+                for (uint32_t k : v) at[bank(k) + 1]++;
+                for (uint32_t q = 0; q < 16; q++) { at[q + 1] += at[q]; end[q] = at[q]; }
+                dealt.resize(v.size());
+                for (uint32_t k : v) dealt[end[bank(k)]++] = k;
                 for (size_t left = v.size(); left;) {
                     for (uint32_t q = 0; q < 16; q++) {
-                        if (at[q] == by_bank[q].size()) continue;
-                        const uint32_t k = by_bank[q][at[q]++];
+                        if (at[q] == end[q]) continue;
+                        const uint32_t k = dealt[at[q]++];
                         left--;
                         const Link12 &l = p.links[k];
                         LinkS r;
