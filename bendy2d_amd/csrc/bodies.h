@@ -137,4 +137,113 @@ __device__ __forceinline__ bool resolve_line(float2 self_center, float2 pa, floa
     return true;
 }
 
+// Polygon pair loop (src/solver.rs:178-187 -> Polygon::solve_polygon
+// src/polygon.rs:142-162) by one workgroup.  Edges run in order; within an edge the
+// other polygon's points are independent (each reads only the edge's ends as they
+// were before it, its own position and the two centres), and the hit with the
+// highest point index writes the ends ("last hit wins").  An edge that no point
+// hits changes nothing, so a step tests as many edges as the lanes hold, against
+// the positions as they are, and carries out the first that is hit; the edges
+// behind it are tested again.  (Edge by edge, 5 polygons of 12 points took 240
+// steps of two barriers, nearly all for nothing: an update 176 us, 46 now.)
+// P holds positions as 64-bit words (in LDS or memory); tab[p].x, .y are a
+// polygon's first point and point count; slot is 3 words of LDS.
+template <int WG, typename WP, typename TAB>
+__device__ __forceinline__ void poly_pair_loop(WP P, const TAB *tab, const float2 *ctr, uint32_t npoly,
+                                               uint32_t *slot) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    auto get = [&](uint32_t i) {
+        const uint64_t b = P[i];
+        return make_float2(__uint_as_float((uint32_t)b), __uint_as_float((uint32_t)(b >> 32)));
+    };
+    auto put = [&](uint32_t i, float2 v) {
+        P[i] = (uint64_t)__float_as_uint(v.x) | ((uint64_t)__float_as_uint(v.y) << 32);
+    };
+    // up to 64 polygons' table in registers, one to a lane
+    const bool held = npoly <= 64u;
+    const uint32_t hp = min(lane, npoly - 1u);
+    const uint32_t h_at = tab[hp].x, h_n = tab[hp].y;
+    const float2 h_c = ctr[hp];
+    struct Poly { uint32_t at, n; float2 c; };
+    auto poly = [&](uint32_t q) {
+        Poly r;
+        if (held) {
+            r.at = __builtin_amdgcn_readlane(h_at, q);
+            r.n = __builtin_amdgcn_readlane(h_n, q);
+            r.c.x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(h_c.x), q));
+            r.c.y = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(h_c.y), q));
+        } else {
+            r.at = tab[q].x;
+            r.n = tab[q].y;
+            r.c = ctr[q];
+        }
+        return r;
+    };
+    if (tid < 3u) slot[tid] = 0u;
+    __syncthreads();
+    uint32_t turn = 0;  // slots rotate: the one after next is cleared behind a barrier
+    auto winner = [&](uint32_t key) {
+        uint32_t *const now = &slot[turn % 3u];
+        if (key) atomicMax(now, key);
+        __syncthreads();
+        const uint32_t best = *now;
+        if (tid == 0u) slot[(turn + 2u) % 3u] = 0u;
+        turn++;
+        return best;
+    };
+    for (uint32_t i = 0; i < npoly; i++)
+        for (uint32_t j = i + 1; j < npoly; j++)
+            for (uint32_t dir = 0; dir < 2u; dir++) {
+                const Poly s = poly(dir ? j : i), o = poly(dir ? i : j);
+                const uint32_t E = s.n, K = o.n;
+                if (K == 0u) continue;
+                if (K <= (uint32_t)WG && E < 65536u) {
+                    const uint32_t per = (uint32_t)WG / K, le = tid / K, k = tid - le * K;
+                    for (uint32_t e0 = 0; e0 < E;) {
+                        const uint32_t e = e0 + le, ia = s.at + e, ib = s.at + (e + 1u == E ? 0u : e + 1u);
+                        float2 a2, b2, o2;
+                        const bool hit = le < per && e < E &&
+                                         resolve_line(s.c, get(ia), get(ib), get(o.at + k), o.c, a2, b2, o2);
+                        uint32_t first;  // the first edge that is hit
+                        bool mine, last;
+                        if constexpr (WG == 64) {
+                            const uint64_t hits = __ballot(hit);
+                            if (hits == 0ull) { e0 += per; continue; }
+                            first = (uint32_t)__builtin_amdgcn_readlane(e, __ffsll((unsigned long long)hits) - 1);
+                            mine = hit && e == first;
+                            last = lane == 63u - (uint32_t)__clzll((long long)__ballot(mine));
+                        } else {
+                            const uint32_t key = hit ? (E - e) << 16 | (k + 1u) : 0u;
+                            const uint32_t best = winner(key);
+                            if (best == 0u) { e0 += per; continue; }
+                            first = E - (best >> 16);
+                            mine = hit && e == first;
+                            last = key == best;
+                        }
+                        if (mine) put(o.at + k, o2);
+                        if (last) { put(ia, a2); put(ib, b2); }
+                        __syncthreads();
+                        e0 = first + 1u;
+                    }
+                    continue;
+                }
+                for (uint32_t e = 0; e < E; e++) {
+                    const uint32_t ia = s.at + e, ib = s.at + (e + 1u == E ? 0u : e + 1u);
+                    const float2 pa = get(ia), pb = get(ib);
+                    uint32_t mine = 0;
+                    float2 na = pa, nb = pb;
+                    for (uint32_t k = tid; k < K; k += WG) {
+                        float2 a2, b2, o2;
+                        if (resolve_line(s.c, pa, pb, get(o.at + k), o.c, a2, b2, o2)) {
+                            put(o.at + k, o2);
+                            na = a2; nb = b2; mine = k + 1u;
+                        }
+                    }
+                    const uint32_t best = winner(mine);
+                    if (mine && mine == best) { put(ia, na); put(ib, nb); }
+                    __syncthreads();
+                }
+            }
+}
+
 }  // namespace bd

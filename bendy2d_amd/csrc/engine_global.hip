@@ -69,53 +69,11 @@ __global__ void k_poly_centers(const float2 *__restrict__ pos, const uint2 *__re
     centers[p] = make_float2(sx / n, sy / n);
 }
 
-// Polygon pair loop (src/solver.rs:178-187 -> Polygon::solve_polygon
-// src/polygon.rs:142-162) in one workgroup.  Edges run in order; within an
-// edge the other polygon's points are independent (each reads only the stale
-// edge copies, its own position and the two centres), so they run across the
-// workgroup, and the hit with the highest point index writes the edge ends
-// ("last hit wins").
+// Polygon pair loop in one workgroup.
 __global__ void __launch_bounds__(256) k_poly_pairs(float2 *pos, const uint2 *__restrict__ ptab, uint32_t P,
                                                     const float2 *__restrict__ centers) {
-    __shared__ int s_last;
-    __shared__ float2 s_pa, s_pb;
-    for (uint32_t i = 0; i < P; i++) {
-        for (uint32_t j = i + 1; j < P; j++) {
-            for (int dir = 0; dir < 2; dir++) {
-                uint32_t si = dir == 0 ? i : j, oi = dir == 0 ? j : i;
-                uint2 st = ptab[si], ot = ptab[oi];
-                float2 sc = centers[si], oc = centers[oi];
-                for (uint32_t e = 0; e < st.y; e++) {
-                    uint32_t bid = (e + 1) % st.y;
-                    if (threadIdx.x == 0) {
-                        s_last = -1;
-                        s_pa = pos[st.x + e];
-                        s_pb = pos[st.x + bid];
-                    }
-                    __syncthreads();
-                    float2 pa = s_pa, pb = s_pb;
-                    int mine = -1;
-                    float2 na = make_float2(0.0f, 0.0f), nb = na;
-                    for (uint32_t k = threadIdx.x; k < ot.y; k += blockDim.x) {
-                        float2 op = pos[ot.x + k];
-                        float2 a2, b2, o2;
-                        if (resolve_line(sc, pa, pb, op, oc, a2, b2, o2)) {
-                            pos[ot.x + k] = o2;
-                            na = a2; nb = b2; mine = (int)k;
-                        }
-                    }
-                    if (mine >= 0) atomicMax(&s_last, mine);
-                    __syncthreads();
-                    if (mine >= 0 && mine == s_last) {
-                        pos[st.x + e] = na;
-                        pos[st.x + bid] = nb;
-                    }
-                    __threadfence_block();
-                    __syncthreads();
-                }
-            }
-        }
-    }
+    __shared__ uint32_t s_slot[3];
+    poly_pair_loop<256>((uint64_t *)pos, ptab, centers, P, s_slot);
 }
 
 // Fused per-body phase: EXT4 static colliders -> bounds -> Verlet.

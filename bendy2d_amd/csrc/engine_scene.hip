@@ -223,8 +223,7 @@ struct CCShared {
     uint32_t halt;           // the scene's time budget for this launch is spent
     float4 red4[32];         // the wavefronts' drift boxes and sums (see drift_box)
     uint32_t cnt3[3];        // worklist lengths, rotating (see the round loop)
-    uint32_t poly_last[2];   // polygon pairs: 1 + the last point of the other polygon that
-                             // hit the current edge, two slots used alternately
+    uint32_t poly_last[3];   // polygon pairs: see poly_pair_loop
     // LDS the sequential fallback may use for its grid: the scene's previous
     // positions when they are held in LDS (parked in q_global meanwhile), or
     // what the positions leave of the launch's LDS
@@ -2112,36 +2111,11 @@ __device__ __forceinline__ bool quiet_sweep(const float2 *P, uint32_t Np, uint32
 template <int WG>
 __device__ __noinline__ void poly_pairs(float2 *P, const uint4 *ptab, const float2 *ctr, uint32_t npoly,
                                         uint32_t *poly_last) {
-    const int tid = threadIdx.x;
-    if (tid == 0) { poly_last[0] = 0u; poly_last[1] = 0u; }
-    __syncthreads();
-    uint32_t turn = 0;
-    for (uint32_t i = 0; i < npoly; i++)
-        for (uint32_t j = i + 1; j < npoly; j++)
-            for (uint32_t dir = 0; dir < 2; dir++) {
-                const uint32_t si = dir ? j : i, oi = dir ? i : j;
-                const uint4 ts = ptab[si], to = ptab[oi];
-                const float2 sc = ctr[si], oc = ctr[oi];
-                for (uint32_t e = 0; e < ts.y; e++, turn++) {
-                    const uint32_t ia = ts.x + e, ib = ts.x + (e + 1 == ts.y ? 0u : e + 1);
-                    const float2 pa = P[ia], pb = P[ib];
-                    uint32_t mine = 0;
-                    float2 na = pa, nb = pb;
-                    for (uint32_t k = tid; k < to.y; k += WG) {
-                        float2 a2, b2, o2;
-                        if (resolve_line(sc, pa, pb, P[to.x + k], oc, a2, b2, o2)) {
-                            P[to.x + k] = o2;
-                            na = a2; nb = b2; mine = k + 1;
-                        }
-                    }
-                    uint32_t *slot = &poly_last[turn & 1u];
-                    if (mine) atomicMax(slot, mine);
-                    __syncthreads();
-                    if (mine && mine == *slot) { P[ia] = na; P[ib] = nb; }
-                    if (tid == 0) poly_last[(turn & 1u) ^ 1u] = 0u;
-                    __syncthreads();
-                }
-            }
+    extern __shared__ float2 s_dyn[];
+    if (((uint64_t)P >> 32) == ((uint64_t)s_dyn >> 32))
+        poly_pair_loop<WG>(to_lds((uint64_t *)P), ptab, ctr, uni(npoly), poly_last);
+    else
+        poly_pair_loop<WG>((uint64_t *)P, ptab, ctr, uni(npoly), poly_last);
 }
 
 // ---------------------------------------------------------------------------
