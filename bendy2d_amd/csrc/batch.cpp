@@ -273,6 +273,7 @@ struct bd_batch {
     std::vector<uint64_t> updates_run;
     DevBuf<uint8_t> arena;
     DevBuf<SceneState> states;
+    PinnedBuf staging;  // bd_batch_read_scene
     uint64_t arena_bytes = 0;
     uint64_t total_points = 0;
     bool uploaded = false;
@@ -472,16 +473,19 @@ int32_t bd_batch_read_scene(bd_batch *b, int64_t id, bd_solver *out) {
     }
     const SceneDesc &d = b->core.descs[id];
     SceneState st;
-    const uint8_t *chunk = b->arena.p + b->chunk_off[id];
-    std::vector<uint8_t> buf(b->images[id].init_bytes);
-    if ((!buf.empty() &&
-         hipMemcpyAsync(buf.data(), chunk, buf.size(), hipMemcpyDeviceToHost, b->core.stream) != hipSuccess) ||
-        hipMemcpyAsync(&st, b->states.p + id, sizeof(st), hipMemcpyDeviceToHost, b->core.stream) != hipSuccess ||
+    const uint64_t bytes = scene_read_bytes(d, b->images[id].init_bytes);
+    // through page-locked memory, without what the device never changes: 640
+    // scenes of up to 128 x 128 circles 27 -> 13 ms
+    const size_t at = (bytes + 255) & ~(size_t)255;
+    if (b->staging.alloc(at + sizeof(st)) != hipSuccess) return fail(BD_ERR_NOMEM, "scene readback buffer");
+    if ((bytes && hipMemcpyAsync(b->staging.p, b->arena.p + b->chunk_off[id], bytes, hipMemcpyDeviceToHost,
+                                 b->core.stream) != hipSuccess) ||
+        hipMemcpyAsync(b->staging.p + at, b->states.p + id, sizeof(st), hipMemcpyDeviceToHost, b->core.stream) !=
+            hipSuccess ||
         hipStreamSynchronize(b->core.stream) != hipSuccess)
         return fail(BD_ERR_DEVICE, "scene readback failed");
-    HostScene h;
-    scene_chunk_to_host(d, buf.data(), h);
-    int rc = solver_import_state(out, h, b->updates_run[id], err);
+    std::memcpy(&st, b->staging.p + at, sizeof(st));
+    int rc = import_scene_chunk(out, d, b->staging.p, b->updates_run[id], err);
     if (rc) return fail(rc, err);
     if (st.err) return fail(BD_ERR_COLLISION, "circle pair schedule failed for this scene");
     return BD_OK;

@@ -87,6 +87,10 @@ struct bd_solver;
 namespace bd {
 int solver_export(const bd_solver *s, HostScene &out, std::string &err);
 int solver_import_state(bd_solver *s, const HostScene &src, uint64_t updates, std::string &err);
+// The same from pos[N] and prev[N] (particles, then circles) of a scene without
+// polygons, in one pass over them.
+int solver_import_bodies(bd_solver *s, uint64_t np, uint64_t nc, const void *pos, const void *prev, uint64_t updates,
+                         std::string &err);
 const HostScene &solver_host(const bd_solver *s);
 
 #define BD_HIP(call)                                                                   \
@@ -97,6 +101,26 @@ const HostScene &solver_host(const bd_solver *s);
             return BD_ERR_DEVICE;                                                      \
         }                                                                              \
     } while (0)
+
+// Page-locked host memory for copies from the device, grown to the largest asked.
+struct PinnedBuf {
+    uint8_t *p = nullptr;
+    size_t n = 0;
+    PinnedBuf() {}
+    PinnedBuf(const PinnedBuf &) = delete;
+    PinnedBuf &operator=(const PinnedBuf &) = delete;
+    ~PinnedBuf() {
+        if (p) (void)hipHostFree(p);
+    }
+    hipError_t alloc(size_t bytes) {
+        if (bytes <= n) return hipSuccess;
+        if (p) (void)hipHostFree(p);
+        p = nullptr; n = 0;
+        hipError_t e = hipHostMalloc((void **)&p, bytes, hipHostMallocDefault);
+        if (e == hipSuccess) n = bytes; else p = nullptr;
+        return e;
+    }
+};
 
 // Device buffer with RAII release.
 template <typename T>

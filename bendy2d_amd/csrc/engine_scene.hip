@@ -2785,6 +2785,14 @@ int build_scene_image(const HostScene &s, const Plan &p, SceneImage &img, std::s
     return BD_OK;
 }
 
+int import_scene_chunk(bd_solver *out, const SceneDesc &d, const uint8_t *chunk, uint64_t updates, std::string &err) {
+    if (!d.P && !d.Ng)
+        return solver_import_bodies(out, d.Np, d.Nc, chunk + d.pos_off, chunk + d.prev_off, updates, err);
+    HostScene h;
+    scene_chunk_to_host(d, chunk, h);
+    return solver_import_state(out, h, updates, err);
+}
+
 void scene_chunk_to_host(const SceneDesc &d, const uint8_t *chunk, HostScene &h) {
     const float2 *pos = (const float2 *)(chunk + d.pos_off);
     const float2 *prev = (const float2 *)(chunk + d.prev_off);

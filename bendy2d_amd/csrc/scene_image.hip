@@ -242,10 +242,8 @@ int32_t bd_scene_image_read(bd_solver *s, const void *host_image, uint64_t bytes
     std::memcpy(&st, b + kImgState, sizeof(st));
     if (w.version != kImgVersion) return fail(BD_ERR_ARG, "not a scene image");
     if (bytes < kImgChunk + (uint64_t)d.ws_off) return fail(BD_ERR_ARG, "image truncated");
-    HostScene h;
-    scene_chunk_to_host(d, b + kImgChunk, h);
     std::string err;
-    int rc = solver_import_state(s, h, w.ran, err);
+    int rc = import_scene_chunk(s, d, b + kImgChunk, w.ran, err);
     if (rc) return fail(rc, err);
     if (st.err == kErrWorkspace) return fail(BD_ERR_CAPACITY, "an update was given a workspace smaller than the image needs");
     if (st.err) return fail(BD_ERR_COLLISION, "circle pair schedule failed for this scene");

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -33,6 +34,13 @@ int build_scene_image(const HostScene &s, const Plan &p, SceneImage &img, std::s
 // gravity and substeps the scene runs with (for the acc that static polygon
 // points accumulate).
 void scene_chunk_to_host(const SceneDesc &d, const uint8_t *chunk, HostScene &h);
+// What reading a scene back needs of its chunk: the bodies, which come first, and
+// with polygons all of the first init_bytes (centres and acc lie among them).
+inline uint64_t scene_read_bytes(const SceneDesc &d, uint64_t init_bytes) {
+    return d.P || d.Ng ? init_bytes : std::max<uint64_t>(d.pos_off, d.prev_off) + 8ull * d.N;
+}
+// Sets a solver to the scene in a host copy of those bytes.
+int import_scene_chunk(bd_solver *out, const SceneDesc &d, const uint8_t *chunk, uint64_t updates, std::string &err);
 void set_scene_params(SceneDesc &d, const StepParams &sp, uint32_t steps, bool acc_pending);
 
 // Kernel variants by workgroup size.  A scene of N points keeps pos and prev

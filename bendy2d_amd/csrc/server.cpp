@@ -120,6 +120,7 @@ struct bd_server {
     double tick_s = 1e-8;                // seconds per device wall-clock tick
     Arena arena;
     DevBuf<SceneState> slots;
+    PinnedBuf staging;                   // bd_server_read_scene, under launch_mu
     std::vector<uint32_t> free_slots;
     std::chrono::steady_clock::time_point t0;
 
@@ -567,20 +568,21 @@ int32_t bd_server_read_scene(bd_server *S, int64_t scene_id, bd_solver *out) {
         lg.lock();
     }
     const SceneDesc &d = sc->desc;
-    std::vector<uint8_t> buf(sc->init_bytes);
     SceneState st = sc->saved;
+    const uint8_t *chunk = sc->host.data();
     if (sc->resident) {
-        if (hipMemcpyAsync(buf.data(), S->arena.base + sc->off, sc->init_bytes, hipMemcpyDeviceToHost, S->core.stream) != hipSuccess ||
-            hipMemcpyAsync(&st, S->slots.p + sc->slot, sizeof(st), hipMemcpyDeviceToHost, S->core.stream) != hipSuccess ||
+        const uint64_t bytes = scene_read_bytes(d, sc->init_bytes);
+        const size_t at = (bytes + 255) & ~(size_t)255;
+        if (S->staging.alloc(at + sizeof(st)) != hipSuccess) return fail(BD_ERR_NOMEM, "scene readback buffer");
+        if (hipMemcpyAsync(S->staging.p, S->arena.base + sc->off, bytes, hipMemcpyDeviceToHost, S->core.stream) != hipSuccess ||
+            hipMemcpyAsync(S->staging.p + at, S->slots.p + sc->slot, sizeof(st), hipMemcpyDeviceToHost, S->core.stream) != hipSuccess ||
             hipStreamSynchronize(S->core.stream) != hipSuccess)
             return fail(BD_ERR_DEVICE, "scene readback failed");
-    } else {
-        buf = sc->host;
+        std::memcpy(&st, S->staging.p + at, sizeof(st));
+        chunk = S->staging.p;
     }
-    HostScene h;
-    scene_chunk_to_host(d, buf.data(), h);
     std::string err;
-    int rc = solver_import_state(out, h, sc->updates_run, err);
+    int rc = import_scene_chunk(out, d, chunk, sc->updates_run, err);
     if (rc) return fail(rc, err);
     if (st.err) return fail(BD_ERR_COLLISION, "circle pair schedule failed for this scene");
     return BD_OK;

@@ -199,6 +199,29 @@ int solver_import_state(bd_solver *s, const HostScene &src, uint64_t updates, st
     return BD_OK;
 }
 
+int solver_import_bodies(bd_solver *s, uint64_t np, uint64_t nc, const void *pos_, const void *prev_, uint64_t updates,
+                         std::string &err) {
+    int rc = ensure_host(s);
+    if (rc) { err = bd_last_error_str(); return rc; }
+    HostScene &h = s->host;
+    if (h.p_pos.size() != np || h.c_pos.size() != nc || !h.g_pos.empty() || !h.polys.empty()) {
+        err = "scene shape differs from the batch scene";
+        return BD_ERR_ARG;
+    }
+    const V2 *pos = (const V2 *)pos_, *prev = (const V2 *)prev_;
+    std::copy(pos, pos + np, h.p_pos.begin());
+    std::copy(prev, prev + np, h.p_prev.begin());
+    std::copy(pos + np, pos + np + nc, h.c_pos.begin());
+    std::copy(prev + np, prev + np + nc, h.c_prev.begin());
+    if (updates) {
+        std::fill(h.c_acc.begin(), h.c_acc.end(), V2{0.0f, 0.0f});
+        s->acc_pending = false;
+    }
+    s->plan_valid = false;  // device copy (if any) is stale now
+    s->dev_newer = false;
+    return BD_OK;
+}
+
 const HostScene &solver_host(const bd_solver *s) { return s->host; }
 
 }  // namespace bd
