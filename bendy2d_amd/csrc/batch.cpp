@@ -181,27 +181,20 @@ int BatchCore::enqueue_launch(uint32_t steps, std::string &err) {
     uint32_t *q = (uint32_t *)d_queue.p;
     BD_HIP(hipEventRecord(ev_fork, stream));
     BD_HIP(hipStreamWaitEvent(side, ev_fork, 0));
-    if (n_tiny) {
-        BD_HIP(hipStreamWaitEvent(side2, ev_fork, 0));
-        uint32_t blocks = std::min<uint32_t>(n_tiny, (uint32_t)(num_cu * scene_blocks_per_cu(vt, tiny.lds)));
-        int rc = launch_scene_variant(vt, std::max<uint32_t>(blocks, 1), tiny.lds, side2, dd, states_dev(), od,
-                                      n_tiny, q + 2, steps, err);
-        if (rc) return rc;
-        BD_HIP(hipEventRecord(ev_join2, side2));
-    }
-    od += n_tiny;
-    if (n_large) {
-        uint32_t blocks = std::min<uint32_t>(n_large, (uint32_t)(num_cu * scene_blocks_per_cu(vl, large.lds)));
-        int rc = launch_scene_variant(vl, std::max<uint32_t>(blocks, 1), large.lds, side, dd, states_dev(), od + n_small,
-                                      n_large, q + 1, steps, err);
-        if (rc) return rc;
-    }
-    if (n_small) {
-        uint32_t blocks = std::min<uint32_t>(n_small, (uint32_t)(num_cu * scene_blocks_per_cu(vs, small.lds)));
-        int rc = launch_scene_variant(vs, std::max<uint32_t>(blocks, 1), small.lds, stream, dd, states_dev(), od,
-                                      n_small, q, steps, err);
-        if (rc) return rc;
-    }
+    if (n_tiny) BD_HIP(hipStreamWaitEvent(side2, ev_fork, 0));
+    auto launch = [&](int v, const Shape &shape, hipStream_t st, uint32_t first, uint32_t n, uint32_t *queue) {
+        const uint32_t blocks = std::min<uint32_t>(n, (uint32_t)(num_cu * scene_blocks_per_cu(v, shape.lds)));
+        return launch_scene_variant(v, std::max<uint32_t>(blocks, 1), shape.lds, st, dd, states_dev(), od + first, n,
+                                    queue, steps, err);
+    };
+    // the largest first: a large scene takes nearly all of a CU's LDS, and finds no
+    // place on one that holds smaller scenes already
+    int rc = BD_OK;
+    if (n_large) rc = launch(vl, large, side, n_tiny + n_small, n_large, q + 1);
+    if (!rc && n_small) rc = launch(vs, small, stream, n_tiny, n_small, q);
+    if (!rc && n_tiny) rc = launch(vt, tiny, side2, 0, n_tiny, q + 2);
+    if (rc) return rc;
+    if (n_tiny) BD_HIP(hipEventRecord(ev_join2, side2));
     BD_HIP(hipEventRecord(ev_join, side));
     BD_HIP(hipStreamWaitEvent(stream, ev_join, 0));
     if (n_tiny) BD_HIP(hipStreamWaitEvent(stream, ev_join2, 0));
