@@ -4,7 +4,10 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
+#include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/bendy2d.h"
@@ -33,6 +36,25 @@ struct StepParams {
 
 StepParams make_params(const HostScene &s, float dt, bool acc_pending);
 
+// An engine's state as up to four arrays of 8-byte words in device memory, which
+// follow each other in a copy.  With an index, word i of the copy is src[index[i]].
+struct StateParts {
+    struct Part {
+        const void *src;
+        const uint32_t *index;
+        uint32_t words;
+    } part[4] = {};
+    int n = 0;
+    void add(const void *src, size_t words, const uint32_t *index = nullptr) {
+        if (words) part[n++] = Part{src, index, (uint32_t)words};
+    }
+};
+
+// Queues the copy of the parts into dst, in device or page-locked host memory.
+hipError_t gather_state(const StateParts &parts, void *dst, hipStream_t stream);
+
+struct PinnedPool;
+
 class Engine {
 public:
     virtual ~Engine() {}
@@ -40,23 +62,17 @@ public:
     virtual int upload(const HostScene &s, const Plan &p, std::string &err) = 0;
     // Run one update (all substeps).
     virtual int update(const StepParams &sp, Stats &st, std::string &err) = 0;
-    // Copy positions back into the host scene (and static polygon centres).
-    virtual int download(HostScene &s, std::string &err) {
-        std::vector<float2> buf(state_count());
-        int rc = copy_state(buf.data(), hipMemcpyDeviceToHost, stream(), err);
-        if (rc) return rc;
-        if (hipStreamSynchronize(stream()) != hipSuccess) {
-            err = "hipStreamSynchronize failed";
-            return BD_ERR_DEVICE;
-        }
-        return unpack(buf.data(), s, err);
-    }
+    // Copy positions back into the host scene (and static polygon centres):
+    // the state gathered into page-locked memory, one launch and one wait (a
+    // copy per array into pageable memory cost about 12 us each, and a large
+    // scene the page faults of a fresh buffer).
+    int download(HostScene &s, PinnedPool &pool, std::string &err);
     // What a download reads, as state_count() float2: pos[N], prev[N], then
     // the engine's extra words (polygon centres, the circle-pair state);
-    // copy_state queues its copy into dst (device or host memory, by kind) on
-    // stream, unpack fills the host scene from a host copy of it.
+    // state_parts describes where it lies (see gather_state), unpack fills the
+    // host scene from a host copy of it.
     virtual size_t state_count() const = 0;
-    virtual int copy_state(void *dst, hipMemcpyKind kind, hipStream_t stream, std::string &err) = 0;
+    virtual StateParts state_parts() = 0;
     virtual int unpack(const float2 *src, HostScene &s, std::string &err) = 0;
     virtual hipStream_t stream() const = 0;
     virtual int sync(std::string &err) = 0;
@@ -109,6 +125,12 @@ struct PinnedBuf {
     PinnedBuf() {}
     PinnedBuf(const PinnedBuf &) = delete;
     PinnedBuf &operator=(const PinnedBuf &) = delete;
+    PinnedBuf(PinnedBuf &&o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+    PinnedBuf &operator=(PinnedBuf &&o) noexcept {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+        return *this;
+    }
     ~PinnedBuf() {
         if (p) (void)hipHostFree(p);
     }
@@ -116,10 +138,27 @@ struct PinnedBuf {
         if (bytes <= n) return hipSuccess;
         if (p) (void)hipHostFree(p);
         p = nullptr; n = 0;
-        hipError_t e = hipHostMalloc((void **)&p, bytes, hipHostMallocDefault);
+        hipError_t e = hipHostMalloc((void **)&p, bytes, hipHostMallocPortable);
         if (e == hipSuccess) n = bytes; else p = nullptr;
         return e;
     }
+};
+
+// Page-locked buffers that downloads borrow: allocating one takes longer than the
+// download of a small scene.  At most kKept buffers of together kKeptBytes wait
+// here for the next download; all solvers of the process share them, and they are
+// freed with the last solver.
+struct PinnedPool {
+    static constexpr int kKept = 4;
+    static constexpr size_t kKeptBytes = 64u << 20, kLeast = 64u << 10;
+    // a buffer of at least `bytes` (p null when there is no memory)
+    PinnedBuf take(size_t bytes);
+    void give(PinnedBuf &&b);
+    static std::shared_ptr<PinnedPool> shared();
+
+private:
+    std::mutex m_;
+    PinnedBuf kept_[kKept];
 };
 
 // Device buffer with RAII release.

@@ -1392,14 +1392,12 @@ public:
     size_t state_count() const override { return 2ull * N_ + P_; }
     hipStream_t stream() const override { return stream_; }
 
-    int copy_state(void *dst, hipMemcpyKind kind, hipStream_t st, std::string &err) override {
-        float2 *d = (float2 *)dst;
-        if (N_) {
-            BD_HIP(hipMemcpyAsync(d, pos_.p, N_ * sizeof(float2), kind, st));
-            BD_HIP(hipMemcpyAsync(d + N_, prev_.p, N_ * sizeof(float2), kind, st));
-        }
-        if (P_) BD_HIP(hipMemcpyAsync(d + 2 * N_, centers_.p, P_ * sizeof(float2), kind, st));
-        return BD_OK;
+    StateParts state_parts() override {
+        StateParts s;
+        s.add(pos_.p, N_);
+        s.add(prev_.p, N_);
+        s.add(centers_.p, P_);
+        return s;
     }
 
     int unpack(const float2 *src, HostScene &s, std::string &err) override {

@@ -2560,8 +2560,8 @@ __global__ void __launch_bounds__(WG, WG == 1024 ? 4 : 3) k_scenes(const SceneDe
     __shared__ CCShared s_cc;
     __shared__ __align__(16) uint32_t s_wl[2 * WG];  // also float4 scratch of the list builds
     __shared__ uint32_t s_next;
-    for (;;) {
-        if (threadIdx.x == 0) s_next = atomicAdd(queue, 1u);
+    for (uint32_t turn = blockIdx.x;; turn += gridDim.x) {
+        if (threadIdx.x == 0) s_next = queue ? atomicAdd(queue, 1u) : turn;
         __syncthreads();
         const uint32_t k = uni(s_next);
         __syncthreads();
@@ -2853,6 +2853,7 @@ public:
         desc_ = img.desc;
         desc_.base = (uint64_t)(uintptr_t)chunk_;
         acc_pending_ = img.acc_pending;
+        sent_ = false;
         if (!dev_) BD_HIP(hipMalloc((void **)&dev_, 512));
         SceneState st{};
         st.skin = img.skin0;
@@ -2868,13 +2869,17 @@ public:
     int update(const StepParams &sp, Stats &st, std::string &err) override {
         set_scene_params(desc_, sp, 1, acc_pending_ && sp.first_acc);
         acc_pending_ = false;
-        // descriptor, order and queue live in one small buffer (one copy per update)
-        std::memcpy(host_blob_, &desc_, sizeof(desc_));
-        uint32_t zero_order[2] = {0u, 0u};
-        std::memcpy(host_blob_ + 256, zero_order, 8);
-        BD_HIP(hipMemcpyAsync(dev_, host_blob_, 264, hipMemcpyHostToDevice, stream_));
+        // the descriptor goes to the device when the update's parameters changed
+        // (each copy held up a frame by about 8 us)
+        if (!sent_ || std::memcmp(host_blob_, &desc_, sizeof(desc_)) != 0) {
+            sent_ = false;
+            std::memset(host_blob_, 0, sizeof(host_blob_));
+            std::memcpy(host_blob_, &desc_, sizeof(desc_));
+            BD_HIP(hipMemcpyAsync(dev_, host_blob_, sizeof(host_blob_), hipMemcpyHostToDevice, stream_));
+            sent_ = true;
+        }
         int rc = launch_scene_variant(variant_, 1, lds_bytes_, stream_, (const SceneDesc *)dev_, state_ptr(),
-                                      (const uint32_t *)(dev_ + 256), 1, (uint32_t *)(dev_ + 260), 1u, err);
+                                      (const uint32_t *)(dev_ + 256), 1, nullptr, 1u, err);
         if (rc) return rc;
         st.launches++;
         st.substeps += sp.sub_steps;
@@ -2886,15 +2891,13 @@ public:
     size_t state_count() const override { return 2ull * N_ + kStateWords + P_; }
     hipStream_t stream() const override { return stream_; }
 
-    int copy_state(void *dst, hipMemcpyKind kind, hipStream_t st, std::string &err) override {
-        float2 *d = (float2 *)dst;
-        if (N_) {
-            BD_HIP(hipMemcpyAsync(d, chunk_ + desc_.pos_off, 8ull * N_, kind, st));
-            BD_HIP(hipMemcpyAsync(d + N_, chunk_ + desc_.prev_off, 8ull * N_, kind, st));
-        }
-        BD_HIP(hipMemcpyAsync(d + 2 * N_, state_ptr(), sizeof(SceneState), kind, st));
-        if (P_) BD_HIP(hipMemcpyAsync(d + 2 * N_ + kStateWords, chunk_ + desc_.ctr_off, 8ull * P_, kind, st));
-        return BD_OK;
+    StateParts state_parts() override {
+        StateParts s;
+        s.add(chunk_ + desc_.pos_off, N_);
+        s.add(chunk_ + desc_.prev_off, N_);
+        s.add(state_ptr(), kStateWords);
+        s.add(chunk_ + desc_.ctr_off, P_);
+        return s;
     }
 
     int unpack(const float2 *src, HostScene &s, std::string &err) override {
@@ -2931,8 +2934,9 @@ private:
     SceneState *state_ptr() { return (SceneState *)(dev_ + 384); }
     hipStream_t stream_;
     uint8_t *chunk_ = nullptr;
-    uint8_t *dev_ = nullptr;  // [0,256) desc, [256,260) order, [260,264) queue, [384,512) state
-    uint8_t host_blob_[264];
+    uint8_t *dev_ = nullptr;  // [0,256) desc, [256,260) order, [384,512) state
+    uint8_t host_blob_[260] = {};  // what dev_ begins with, when sent_
+    bool sent_ = false;
     SceneDesc desc_{};
     bool acc_pending_ = false;
     int variant_ = 0;

@@ -177,7 +177,7 @@ public:
         int rc = build_tile_plan(s, p, points, region_cap, tp, err);
         if (rc) return rc;
         N_ = p.N;
-        perm_ = tp.perm;
+        const std::vector<uint32_t> &perm = tp.perm;
         passes_.clear();
         passes_.resize(tp.passes.size());
         for (size_t i = 0; i < tp.passes.size(); i++) {
@@ -199,24 +199,28 @@ public:
             BD_HIP(hipStreamSynchronize(stream_));  // host plan vectors are freed at return
         }
         std::vector<float2> pos(N_), prev(N_);
+        std::vector<uint32_t> rank(N_);  // each point's place in the device order
         for (uint32_t i = 0; i < N_; i++) {
-            const V2 &a = s.p_pos[perm_[i]], &b = s.p_prev[perm_[i]];
+            const V2 &a = s.p_pos[perm[i]], &b = s.p_prev[perm[i]];
             pos[i] = make_float2(a.x, a.y);
             prev[i] = make_float2(b.x, b.y);
+            rank[perm[i]] = i;
         }
+        BD_HIP(rank_.alloc(std::max<uint32_t>(N_, 1)));
         BD_HIP(pos_[0].alloc(std::max<uint32_t>(N_, 1)));
         BD_HIP(pos_[1].alloc(std::max<uint32_t>(N_, 1)));
         BD_HIP(prev_.alloc(std::max<uint32_t>(N_, 1)));
         if (N_) {
             BD_HIP(hipMemcpyAsync(pos_[0].p, pos.data(), N_ * sizeof(float2), hipMemcpyHostToDevice, stream_));
             BD_HIP(hipMemcpyAsync(prev_.p, prev.data(), N_ * sizeof(float2), hipMemcpyHostToDevice, stream_));
+            BD_HIP(hipMemcpyAsync(rank_.p, rank.data(), N_ * sizeof(uint32_t), hipMemcpyHostToDevice, stream_));
         }
         cur_ = 0;
         has_pins_ = s.any_pinned();
         if (has_pins_) {
             std::vector<uint32_t> mask((N_ + 31) / 32, 0u);
             for (uint32_t i = 0; i < N_; i++)
-                if (s.p_pin[perm_[i]]) mask[i >> 5] |= 1u << (i & 31);
+                if (s.p_pin[perm[i]]) mask[i >> 5] |= 1u << (i & 31);
             BD_HIP(pinmask_.alloc(mask.size()));
             BD_HIP(hipMemcpyAsync(pinmask_.p, mask.data(), mask.size() * 4, hipMemcpyHostToDevice, stream_));
         }
@@ -295,22 +299,20 @@ public:
     size_t state_count() const override { return 2ull * N_; }
     hipStream_t stream() const override { return stream_; }
 
-    int copy_state(void *dst, hipMemcpyKind kind, hipStream_t st, std::string &err) override {
-        float2 *d = (float2 *)dst;
-        if (N_) {
-            BD_HIP(hipMemcpyAsync(d, pos_[cur_].p, N_ * sizeof(float2), kind, st));
-            BD_HIP(hipMemcpyAsync(d + N_, prev_.p, N_ * sizeof(float2), kind, st));
-        }
-        return BD_OK;
+    // in the scene's order: the device reads its own order by index faster than
+    // the host writes by index (1,048,576 points: 3.1 ms on the host)
+    StateParts state_parts() override {
+        StateParts s;
+        s.add(pos_[cur_].p, N_, rank_.p);
+        s.add(prev_.p, N_, rank_.p);
+        return s;
     }
 
     int unpack(const float2 *src, HostScene &s, std::string &err) override {
         if (!host_shape_matches(s, N_, 0, 0, err)) return BD_ERR_STATE;
-        const float2 *pos = src, *prev = src + N_;
-        for (uint32_t i = 0; i < N_; i++) {
-            s.p_pos[perm_[i]] = V2{pos[i].x, pos[i].y};
-            s.p_prev[perm_[i]] = V2{prev[i].x, prev[i].y};
-        }
+        const V2 *pos = (const V2 *)src, *prev = pos + N_;
+        std::copy(pos, pos + N_, s.p_pos.begin());
+        std::copy(prev, prev + N_, s.p_prev.begin());
         return BD_OK;
     }
 
@@ -328,10 +330,9 @@ private:
     uint32_t N_ = 0, ncol_ = 0, nplanes_ = 0;
     int cur_ = 0;
     bool has_pins_ = false;
-    std::vector<uint32_t> perm_;
     std::vector<DevPass> passes_;
     DevBuf<float2> pos_[2], prev_;
-    DevBuf<uint32_t> pinmask_;
+    DevBuf<uint32_t> pinmask_, rank_;
     DevBuf<int4> colhdr_;
     DevBuf<float4> colgeo_, planes_;
 };

@@ -61,6 +61,7 @@ struct bd_solver {
     // 1024x1024 cloth (measured fastest of 1,024..8,192 points x 256..1,024 lanes)
     uint32_t tile_points = 0, tile_wg = 1024;  // (0: the engine chooses)
     hipStream_t stream = nullptr;
+    std::shared_ptr<PinnedPool> pool = PinnedPool::shared();
     int device = -1;
     Stats stats;
     // Readback (bd_ext_set_readback): after each update, a device-side copy of
@@ -117,7 +118,7 @@ static int ensure_host(const bd_solver *cs) {
         if (hipEventSynchronize(s->rb.done[k]) != hipSuccess) return fail(BD_ERR_DEVICE, "readback copy failed");
         rc = s->eng->unpack(s->rb.host[k], s->host, err);
     } else {
-        rc = s->eng->download(s->host, err);
+        rc = s->eng->download(s->host, *s->pool, err);
     }
     if (rc) return fail(rc, err);
     for (size_t p = 0; p < s->host.polys.size(); p++)
@@ -685,9 +686,8 @@ static int readback_begin(bd_solver *s) {
         rb.host_cap[k] = n;
     }
     std::string err;
-    int rc = s->eng->copy_state(rb.dev[k].p, hipMemcpyDeviceToDevice, s->stream, err);
-    if (rc) return fail(rc, err);
-    if (!hip_ok(hipEventRecord(rb.snap[k], s->stream)) || !hip_ok(hipStreamWaitEvent(rb.copy, rb.snap[k], 0)) ||
+    if (!hip_ok(gather_state(s->eng->state_parts(), rb.dev[k].p, s->stream)) ||
+        !hip_ok(hipEventRecord(rb.snap[k], s->stream)) || !hip_ok(hipStreamWaitEvent(rb.copy, rb.snap[k], 0)) ||
         (n && !hip_ok(hipMemcpyAsync(rb.host[k], rb.dev[k].p, n * sizeof(float2), hipMemcpyDeviceToHost, rb.copy))) ||
         !hip_ok(hipEventRecord(rb.done[k], rb.copy)))
         return fail(BD_ERR_DEVICE, "readback copy");
