@@ -184,7 +184,7 @@ __global__ void k_zero_acc0(float2 *acc0, uint32_t n) {
 // atomics on one word take about 30 us (k_cg_check 34 -> 11 us).
 
 constexpr int kLevels = 12;
-constexpr uint32_t kSlotG = 8;  // candidates kept by the counting scan
+constexpr uint32_t kSlotG = 16;  // candidates kept by the counting scan
 constexpr uint32_t kLvlShift = 26;  // bucket record .w: circle | level << 26
 constexpr uint32_t kIdxMaskG = (1u << kLvlShift) - 1u;
 constexpr uint32_t kLater = 0x80000000u;   // list entry: the partner's number is larger
@@ -201,6 +201,10 @@ constexpr int64_t kMaxScanCells = 1024, kOwnScanCells = 32;
 constexpr int kPieceCells = 4;
 constexpr uint32_t kNoneG = 0xffffffffu;
 constexpr int kCompWG = 256;
+// Lanes that share a slot's edges in k_cg_union: an edge is a chain of a dozen
+// dependent loads, and jammed circles have a dozen edges (one lane a slot 17.5 us
+// with 20,011 circles and 25.0 with 262,144, four 8.9 and 19.1).
+constexpr uint32_t kEdgeLanes = 4;
 constexpr uint32_t kCheckPer = 4;  // slots a thread of k_cg_ranges and k_cg_check
 
 // Per-sweep grid of every level, in device memory.
@@ -370,36 +374,6 @@ __device__ __forceinline__ void cswap(T &a, T &b) {
     a = lo; b = hi;
 }
 
-// Ascending sort of a list in global memory: insertion for short lists,
-// heapsort for long ones.
-__device__ __noinline__ void sort_list(uint64_t *a, uint32_t n) {
-    if (n <= 32u) {
-        for (uint32_t x = 1; x < n; x++) {
-            const uint64_t v = a[x];
-            uint32_t y = x;
-            while (y > 0 && a[y - 1] > v) { a[y] = a[y - 1]; y--; }
-            a[y] = v;
-        }
-        return;
-    }
-    auto sift = [&](uint32_t root, uint32_t end) {
-        for (;;) {
-            uint32_t child = 2u * root + 1u;
-            if (child >= end) return;
-            if (child + 1u < end && a[child] < a[child + 1u]) child++;
-            const uint64_t vr = a[root], vc = a[child];
-            if (!(vr < vc)) return;
-            a[root] = vc; a[child] = vr;
-            root = child;
-        }
-    };
-    for (uint32_t s = n / 2u; s-- > 0;) sift(s, n);
-    for (uint32_t e = n - 1u; e > 0; e--) {
-        const uint64_t t = a[0]; a[0] = a[e]; a[e] = t;
-        sift(0, e);
-    }
-}
-
 // Exclusive place of each thread's v among the workgroup's 256 threads; total is
 // the sum (64-bit: lists can be as long as the scene).  s_sum: 4 words of LDS.
 __device__ __forceinline__ uint64_t block_place(uint32_t v, uint64_t *s_sum, uint64_t &total) {
@@ -556,24 +530,50 @@ __global__ void __launch_bounds__(256) k_cg_cand(Buckets bk, const CGrid *__rest
         keys[s_o[st] + k] = key;
     });
     __syncthreads();
+    // lists from a second scan: a wavefront each, a key to a lane at a time, ranked
+    // against all keys (loads of one address for all lanes that wait for nothing,
+    // where a lane's own sort in memory was a chain of them; with 16 instead of 8
+    // entries kept in LDS, which spares most lists the second scan, this kernel
+    // took 20.0 us instead of 34.9 with 20,011 circles and 34.0 instead of 51.6
+    // with 262,144)
+    const uint32_t number = __float_as_uint(r.w) & kIdxMaskG;
+    uint32_t low = s;
+    for (uint64_t todo = __ballot(n > kSlotG); todo; todo &= todo - 1ull) {
+        const int src = __ffsll((unsigned long long)todo) - 1;
+        const uint32_t ln = (uint32_t)__shfl((int)n, src), lo0 = (uint32_t)__shfl((int)o0, src);
+        const uint32_t li = (uint32_t)__shfl((int)number, src), self = s - lane + (uint32_t)src;
+        const uint64_t *const k = keys + lo0;
+        uint32_t least = self;
+        for (uint32_t x = lane; x < ln; x += 64u) least = min(least, (uint32_t)k[x]);
+        for (int o = 32; o > 0; o >>= 1) least = min(least, (uint32_t)__shfl_xor((int)least, o));
+        for (uint32_t x = lane; x < ln; x += 64u) {
+            const uint64_t key = k[x];
+            uint32_t rank = 0;
+#pragma unroll 8
+            for (uint32_t y = 0; y < ln; y++) rank += k[y] < key ? 1u : 0u;
+            cand[lo0 + rank] = (uint32_t)key | ((uint32_t)(key >> 32) > li ? kLater : 0u) |
+                               ((uint32_t)key == least ? kParent : 0u);
+        }
+        if ((int)lane == src) low = least;
+    }
     if (s >= bk.nc) return;
     cnt[s] = n;
     off[s] = o0;
-    const uint32_t i = __float_as_uint(r.w) & kIdxMaskG;
-    uint32_t low = s;
     auto entry = [&](uint64_t key) {
-        return (uint32_t)key | ((uint32_t)(key >> 32) > i ? kLater : 0u) | ((uint32_t)key == low ? kParent : 0u);
+        return (uint32_t)key | ((uint32_t)(key >> 32) > number ? kLater : 0u) | ((uint32_t)key == low ? kParent : 0u);
     };
-    if (n <= kSlotG) {
-        uint64_t v[kSlotG];
+    // the kept ones by a sorting network of the size that the wavefront needs
+    auto put = [&](auto size) {
+        constexpr uint32_t K = decltype(size)::value;
+        uint64_t v[K];
 #pragma unroll
-        for (uint32_t k = 0; k < kSlotG; k++) v[k] = k < n ? s_keep[k][tid] : ~0ull;
+        for (uint32_t k = 0; k < K; k++) v[k] = k < n ? s_keep[k][tid] : ~0ull;
 #pragma unroll
-        for (uint32_t k = 2; k <= kSlotG; k <<= 1)
+        for (uint32_t k = 2; k <= K; k <<= 1)
 #pragma unroll
             for (uint32_t j = k >> 1; j > 0; j >>= 1)
 #pragma unroll
-                for (uint32_t x = 0; x < kSlotG; x++) {
+                for (uint32_t x = 0; x < K; x++) {
                     const uint32_t l = x ^ j;
                     if (l > x) {
                         if ((x & k) == 0u) cswap(v[x], v[l]);
@@ -581,15 +581,16 @@ __global__ void __launch_bounds__(256) k_cg_cand(Buckets bk, const CGrid *__rest
                     }
                 }
 #pragma unroll
-        for (uint32_t k = 0; k < kSlotG; k++)
+        for (uint32_t k = 0; k < K; k++)
             if (k < n) low = min(low, (uint32_t)v[k]);
 #pragma unroll
-        for (uint32_t k = 0; k < kSlotG; k++)
+        for (uint32_t k = 0; k < K; k++)
             if (k < n) cand[o0 + k] = entry(v[k]);
-    } else {
-        sort_list(keys + o0, n);
-        for (uint32_t k = 0; k < n; k++) low = min(low, (uint32_t)keys[o0 + k]);
-        for (uint32_t k = 0; k < n; k++) cand[o0 + k] = entry(keys[o0 + k]);
+    };
+    if (n <= kSlotG) {
+        if (__ballot(n > 4u) == 0ull) put(std::integral_constant<uint32_t, 4>{});
+        else if (__ballot(n > 8u) == 0ull) put(std::integral_constant<uint32_t, 8>{});
+        else put(std::integral_constant<uint32_t, kSlotG>{});
     }
     par[s] = low;
 }
@@ -618,10 +619,10 @@ __device__ uint32_t uf_find(uint32_t *par, uint32_t x) {
 __global__ void __launch_bounds__(256) k_cg_union(const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
                                                   const uint32_t *__restrict__ cand, uint32_t nc, uint32_t *par,
                                                   const uint32_t *__restrict__ ctl) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t / kEdgeLanes;
     if (i >= nc || ctl[kCtlFull]) return;
     const uint32_t s0 = off[i], n = cnt[i];
-    for (uint32_t s = 0; s < n; s++) {
+    for (uint32_t s = t % kEdgeLanes; s < n; s += kEdgeLanes) {
         const uint32_t e = cand[s0 + s];
         uint32_t a = e & kIdxMaskG, b = i;
         if (a >= i || (e & kParent)) continue;  // each edge once, from its larger end
@@ -1460,7 +1461,7 @@ private:
             hipLaunchKernelGGL(k_cg_cand, dim3(nb), dim3(256), 0, stream_, bk, ws_.grid, (uint32_t)cand_cap_, ws_.cnt,
                                ws_.off, cc_cand_.p, (uint64_t *)cg_traj_.p, ws_.par, ws_.csize, ws_.spos,
                                ws_.exc, cg_order_.p, ws_.aux, cg_need_.p, ctl);
-            hipLaunchKernelGGL(k_cg_union, dim3(nb), dim3(256), 0, stream_, ws_.cnt, ws_.off, cc_cand_.p, nc,
+            hipLaunchKernelGGL(k_cg_union, dim3((unsigned)(((uint64_t)nc * kEdgeLanes + 255u) / 256u)), dim3(256), 0, stream_, ws_.cnt, ws_.off, cc_cand_.p, nc,
                                ws_.par, ctl);
             hipLaunchKernelGGL(k_cg_comp, dim3(nb), dim3(256), 0, stream_, ws_.cnt, nc, ws_.par, ws_.root,
                                ws_.place, ws_.csize, ctl);
@@ -1486,7 +1487,7 @@ private:
             hipLaunchKernelGGL(k_cg_check, dim3((nb + kCheckPer - 1) / kCheckPer), dim3(256), 0, stream_, ws_.exc,
                                ws_.aux, ws_.rec, ws_.spos, ws_.cnt, cg_need_.p, s0_, nc, pos_.p, Np_,
                                ws_.overq, ctl);
-            hipLaunchKernelGGL(k_cg_verify, dim3(std::min<uint32_t>(nb, kVerifyGrid)), dim3(256), 0, stream_, bk,
+            hipLaunchKernelGGL(k_cg_verify, dim3(std::min<uint32_t>((nc + 3) / 4, kVerifyGrid)), dim3(256), 0, stream_, bk,
                                ws_.aux, ws_.exc, ws_.grid, ws_.cnt, ws_.off, cc_cand_.p, ws_.overq,
                                cg_traj_.p, ctl);
             st.launches += 11;

@@ -54,6 +54,17 @@ def test_clumps(n):
     check(at(xy.astype(np.float32), 1.0), 3, 1000.0)
 
 
+@pytest.mark.parametrize("n", [4, 5, 6, 16, 17, 18, 65, 66, 130])
+def test_kept_lists(n):
+    # a few hundred circles in clumps of n: lists of n - 1 entries around what a
+    # lane sorts (4, 8, 16) and what a wavefront ranks at once (64), many of them
+    # in each wavefront
+    rng = np.random.default_rng(100 + n)
+    clumps = -(-400 // n)
+    xy = rng.uniform(-0.25, 0.25, (clumps, n, 2)) + np.array([(12.0 * k, 5.0 * (k % 3)) for k in range(clumps)])[:, None]
+    check(at(xy.reshape(-1, 2)[rng.permutation(clumps * n)].astype(np.float32), 1.0), 2, 9000.0)
+
+
 @pytest.mark.parametrize("n", [2, 3, 7, 16, 17, 257, 4097])
 @pytest.mark.parametrize("mixed", [False, True])
 def test_levels(n, mixed):
