@@ -77,10 +77,6 @@ __global__ void __launch_bounds__(256) k_poly_pairs(float2 *pos, const uint2 *__
 }
 
 // Fused per-body phase: EXT4 static colliders -> bounds -> Verlet.
-constexpr int kMaxStagedColliders = 256;
-constexpr int kMaxStagedPlanes = 1024;
-
-template <bool STAGED>
 __global__ void __launch_bounds__(256) k_bodies(float2 *__restrict__ pos, float2 *__restrict__ prev,
                                                 const uint32_t *__restrict__ pinmask,
                                                 const float *__restrict__ crad,
@@ -89,18 +85,6 @@ __global__ void __launch_bounds__(256) k_bodies(float2 *__restrict__ pos, float2
                                                 const int4 *__restrict__ colhdr,
                                                 const float4 *__restrict__ colgeo,
                                                 const float4 *__restrict__ planes, BodyParams P) {
-    __shared__ int4 s_hdr[STAGED ? kMaxStagedColliders : 1];
-    __shared__ float4 s_geo[STAGED ? kMaxStagedColliders : 1];
-    __shared__ float4 s_pl[STAGED ? kMaxStagedPlanes : 1];
-    const int4 *hdr = colhdr;
-    const float4 *geo = colgeo;
-    const float4 *pl = planes;
-    if (STAGED) {
-        for (uint32_t k = threadIdx.x; k < P.ncol; k += blockDim.x) { s_hdr[k] = colhdr[k]; s_geo[k] = colgeo[k]; }
-        for (uint32_t k = threadIdx.x; k < P.nplanes; k += blockDim.x) s_pl[k] = planes[k];
-        __syncthreads();
-        hdr = s_hdr; geo = s_geo; pl = s_pl;
-    }
     for (uint32_t u = blockIdx.x * blockDim.x + threadIdx.x; u < P.N; u += gridDim.x * blockDim.x) {
         float r = 0.0f;
         float ax = P.gex, ay = P.gey;
@@ -116,7 +100,7 @@ __global__ void __launch_bounds__(256) k_bodies(float2 *__restrict__ pos, float2
             if (P.first_acc && integrate) { float2 a = acc0[u - P.Np]; ax = a.x + P.gx; ay = a.y + P.gy; }
         }
         float2 p = pos[u], q = prev[u];
-        static_colliders(p, r, P.ncol, hdr, geo, pl);
+        static_colliders(p, r, P.ncol, colhdr, colgeo, planes);
         if (circle) {
             circle_bounds_axis(p.x, q.x, P.lox, P.hix, r);
             circle_bounds_axis(p.y, q.y, P.loy, P.hiy, r);
@@ -1340,7 +1324,7 @@ public:
         bp.dt = sp.delta; bp.gex = sp.gex; bp.gey = sp.gey; bp.gx = sp.gx; bp.gy = sp.gy;
         bp.lox = sp.lox; bp.loy = sp.loy; bp.hix = sp.hix; bp.hiy = sp.hiy;
         bp.N = N_; bp.Np = Np_; bp.Nc = Nc_;
-        bp.ncol = ncol_; bp.nplanes = nplanes_;
+        bp.ncol = ncol_;
         for (uint32_t step = 0; step < sp.sub_steps; step++) {
             // links, k sweeps; polygon centres before the last sweep
             for (uint32_t it = 0; it < sp.link_iters; it++) {
@@ -1369,14 +1353,9 @@ public:
             bp.first_acc = (sp.first_acc && step == 0 && acc0_.p) ? 1u : 0u;
             if (N_) {
                 uint32_t blocks = std::min<uint32_t>((N_ + 255) / 256, 65535u * 4);
-                if (ncol_ <= (uint32_t)kMaxStagedColliders && nplanes_ <= (uint32_t)kMaxStagedPlanes)
-                    hipLaunchKernelGGL(k_bodies<true>, dim3(blocks), dim3(256), 0, stream_, pos_.p, prev_.p,
-                                       has_pins_ ? pinmask_.p : nullptr, crad_.p, acc0_.p, gflags_.p, colhdr_.p,
-                                       colgeo_.p, planes_.p, bp);
-                else
-                    hipLaunchKernelGGL(k_bodies<false>, dim3(blocks), dim3(256), 0, stream_, pos_.p, prev_.p,
-                                       has_pins_ ? pinmask_.p : nullptr, crad_.p, acc0_.p, gflags_.p, colhdr_.p,
-                                       colgeo_.p, planes_.p, bp);
+                hipLaunchKernelGGL(k_bodies, dim3(blocks), dim3(256), 0, stream_, pos_.p, prev_.p,
+                                   has_pins_ ? pinmask_.p : nullptr, crad_.p, acc0_.p, gflags_.p, colhdr_.p, colgeo_.p,
+                                   planes_.p, bp);
                 st.launches++;
             }
             st.substeps++;

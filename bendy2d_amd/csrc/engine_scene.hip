@@ -36,11 +36,6 @@
 
 namespace bd {
 
-// A value every lane of the workgroup holds alike, moved to a scalar register
-// (the compiler cannot see that values read back from LDS are uniform).
-__device__ __forceinline__ uint32_t uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ float uni(float v) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v))); }
-
 // Orders one wavefront's memory operations between its lanes: a wavefront's
 // LDS and vector memory instructions execute in order, so keeping the
 // compiler from moving them across this point is all that is needed.
@@ -48,31 +43,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// A uniform pointer into global memory, typed as such, with its base read
-// from the first lane: loads through it take a 32-bit offset beside a scalar
-// base instead of a 64-bit flat address.
-#define BD_GLOBAL __attribute__((address_space(1)))
-template <typename T>
-__device__ __forceinline__ BD_GLOBAL T *to_global(T *p) {
-    const uint64_t a = (uint64_t)p;
-    // each half through uni(), which returns it unsigned: the builtin's int,
-    // widened directly, would carry bit 31 of the low half into the high one
-    const uint64_t lo = uni((uint32_t)a);
-    const uint64_t hi = uni((uint32_t)(a >> 32));
-    return (BD_GLOBAL T *)((hi << 32) | lo);
-}
-
-// The same for read-only data read at uniform indices: typed as constant, it
-// is read by scalar loads into scalar registers.
-#define BD_CONST __attribute__((address_space(4)))
-template <typename T>
-__device__ __forceinline__ BD_CONST const T *to_const(const T *p) {
-    const uint64_t a = (uint64_t)p;
-    const uint64_t lo = uni((uint32_t)a);
-    const uint64_t hi = uni((uint32_t)(a >> 32));
-    return (BD_CONST const T *)((hi << 32) | lo);
 }
 
 // A pointer into LDS, typed as such: the low 32 bits of a generic LDS address
@@ -2263,20 +2233,11 @@ __device__ __noinline__ void link_phase(const SceneDesc *dp, float2 *P_, const L
     }
 }
 
-// Bodies: static colliders -> bounds -> Verlet.  Collider records are uniform
-// and come through the scalar cache into scalar registers; a plane's scan ends
-// once no lane's body is still inside all planes so far (640 flying bodies: the
-// phase 20 % shorter than with records staged in LDS).  acc: the initial acc
-// of circles and polygon points is pending (the first substep).
+// Bodies: static colliders -> bounds -> Verlet.  acc: the initial acc of circles
+// and polygon points is pending (the first substep).
 template <int WG, uint32_t KIND, typename PP, typename QP>
 __device__ __forceinline__ void step_bodies(const SceneDesc &d, PP P, QP Q, bool acc) {
     const char *base = (const char *)d.base;
-    typedef int I4 __attribute__((ext_vector_type(4)));
-    typedef float F4 __attribute__((ext_vector_type(4)));
-    BD_CONST const I4 *const hdr = to_const((const I4 *)(base + d.hdr_off));
-    BD_CONST const F4 *const geo = to_const((const F4 *)(base + d.geo_off));
-    BD_CONST const F4 *const pl = to_const((const F4 *)(base + d.pl_off));
-    BD_GLOBAL const F4 *const gpl = to_global((const F4 *)(base + d.pl_off));
     BD_GLOBAL const float *const crad = to_global((const float *)(base + d.crad_off));
     BD_GLOBAL const uint32_t *const pinmask = to_global((const uint32_t *)(base + d.pin_off));
     BD_GLOBAL const uint32_t *const gstatic = to_global((const uint32_t *)(base + d.gst_off));
@@ -2295,17 +2256,7 @@ __device__ __forceinline__ void step_bodies(const SceneDesc &d, PP P, QP Q, bool
         float r = 0.0f;
         if (KIND == kBodiesCircles) r = runi;
         else if (KIND == kBodiesMixed && circle) r = uni_r ? runi : crad[j - Np];
-#pragma unroll 1
-        for (uint32_t k = 0; k < ncol; k++) {
-            const I4 h = hdr[k];
-            if (h.x == 0) {
-                const F4 g = geo[k];
-                static_circle(p.x, p.y, r, g.x, g.y, g.z);
-            } else {
-                static_planes(p, r, (uint32_t)h.z, [&](uint32_t e) -> F4 { return pl[h.y + e]; },
-                              [&](uint32_t e) -> F4 { return gpl[h.y + e]; });
-            }
-        }
+        static_colliders(p, r, ncol, base + d.hdr_off, base + d.geo_off, base + d.pl_off);
         float ax = gex, ay = gey;
         if (KIND == kBodiesCircles || circle) {
             circle_bounds_axis(p.x, q.x, lox, hix, r);

@@ -258,7 +258,7 @@ public:
         BodyParams bp{};
         bp.dt = sp.delta; bp.gex = sp.gex; bp.gey = sp.gey; bp.gx = sp.gx; bp.gy = sp.gy;
         bp.lox = sp.lox; bp.loy = sp.loy; bp.hix = sp.hix; bp.hiy = sp.hiy;
-        bp.N = N_; bp.Np = N_; bp.Nc = 0; bp.first_acc = 0; bp.ncol = ncol_; bp.nplanes = nplanes_;
+        bp.N = N_; bp.Np = N_; bp.Nc = 0; bp.first_acc = 0; bp.ncol = ncol_;
         const uint32_t *pin = has_pins_ ? pinmask_.p : nullptr;
         for (uint32_t step = 0; step < sp.sub_steps; step++) {
             if (passes_.empty()) {
