@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -76,7 +77,33 @@ __global__ void __launch_bounds__(256) k_poly_pairs(float2 *pos, const uint2 *__
     poly_pair_loop<256>((uint64_t *)pos, ptab, centers, P, s_slot);
 }
 
-// Fused per-body phase: EXT4 static colliders -> bounds -> Verlet.
+constexpr int kLevels = 12;  // of the circle-pair grid
+// component queues: for 4, 16 and 64 lanes, a workgroup in LDS, one in memory
+constexpr uint32_t kQueues = 5, kQueueLds = 3, kQueueBig = 4;
+// Control words of a sweep (zeroed with the bucket counters, which follow them;
+// the two at kCtlTotal are one 64-bit counter).
+enum : uint32_t {
+    kCtlTotal = 0, kCtlMask = 2, kCtlOver, kCtlBad, kCtlRounds, kCtlInf, kCtlMissed, kCtlQuiet, kCtlMembers, kCtlFull,
+    kCtlQueue = 12, kCtlEmax = kCtlQueue + kQueues, kCtlWords = 32
+};
+static_assert(kCtlEmax + kLevels <= (int)kCtlWords, "control words");
+
+// The sweep whose control words these are was carried out and missed no pair.
+__device__ __forceinline__ bool sweep_stands(const uint32_t *ctl) {
+    return !(ctl[kCtlFull] | ctl[kCtlBad] | ctl[kCtlInf] | ctl[kCtlMissed]);
+}
+
+// The control words to the host: 32 words over PCIe and then their number, which
+// the host waits for.
+__global__ void __launch_bounds__(64) k_cg_verdict(const uint32_t *__restrict__ ctl, uint32_t *host, uint32_t number) {
+    if (threadIdx.x < kCtlWords) host[threadIdx.x] = ctl[threadIdx.x];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0u) __hip_atomic_store(host + kCtlWords, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Fused per-body phase: EXT4 static colliders -> bounds -> Verlet.  With a verdict
+// nothing happens unless that sweep stands.
 __global__ void __launch_bounds__(256) k_bodies(float2 *__restrict__ pos, float2 *__restrict__ prev,
                                                 const uint32_t *__restrict__ pinmask,
                                                 const float *__restrict__ crad,
@@ -84,7 +111,9 @@ __global__ void __launch_bounds__(256) k_bodies(float2 *__restrict__ pos, float2
                                                 const uint8_t *__restrict__ gflags,
                                                 const int4 *__restrict__ colhdr,
                                                 const float4 *__restrict__ colgeo,
-                                                const float4 *__restrict__ planes, BodyParams P) {
+                                                const float4 *__restrict__ planes, BodyParams P,
+                                                const uint32_t *__restrict__ verdict) {
+    if (verdict && !sweep_stands(verdict)) return;  // uniform
     for (uint32_t u = blockIdx.x * blockDim.x + threadIdx.x; u < P.N; u += gridDim.x * blockDim.x) {
         float r = 0.0f;
         float ax = P.gex, ay = P.gey;
@@ -160,14 +189,17 @@ __global__ void k_zero_acc0(float2 *acc0, uint32_t n) {
 // of a wavefront, a circle to a lane; larger ones in a workgroup, in LDS or, above
 // kLdsMembers circles, in global memory.
 //
-// The host waits once a sweep, for its verdict: lists are handed their space by
+// The host waits once a sweep, for its verdict, and the device meanwhile runs what
+// follows: the bodies, which look at the verdict themselves, and the zeroes of the
+// next sweep's counters (a copy, a wait for the stream and then those two launches
+// left the device idle: 20,011 circles, 8 updates with clone and readback 5.2 -> 4.2
+// ms, 262,144 11.5 -> 10.8).  Lists are handed their space by
 // one atomic per workgroup, out of what earlier sweeps needed (a sweep whose
 // lists do not fit changes nothing and runs again with more), components
 // likewise, and the check of overruns takes their number from device memory.
 // Counters that many wavefronts add to are added to once a workgroup: 4,096
 // atomics on one word take about 30 us (k_cg_check 34 -> 11 us).
 
-constexpr int kLevels = 12;
 constexpr uint32_t kSlotG = 16;  // candidates kept by the counting scan
 constexpr uint32_t kLvlShift = 26;  // bucket record .w: circle | level << 26
 constexpr uint32_t kIdxMaskG = (1u << kLvlShift) - 1u;
@@ -175,8 +207,6 @@ constexpr uint32_t kLater = 0x80000000u;   // list entry: the partner's number i
 constexpr uint32_t kParent = 0x40000000u;  // list entry: the parent that the circle starts with (k_cg_union)
 constexpr uint32_t kLaneList = 32;  // list entries of a circle that a lane holds
 constexpr uint32_t kLdsMembers = 1024, kLdsEntries = 8192;
-// component queues: for 4, 16 and 64 lanes, a workgroup in LDS, one in memory
-constexpr uint32_t kQueues = 5, kQueueLds = 3, kQueueBig = 4;
 // A reach over more cells than kMaxScanCells in one level scans every circle.  One
 // over more than kOwnScanCells (a circle above level 0; level 0 takes up to 3 x 3)
 // is scanned by 16 lanes, kPieceCells cells of a row to each at a time: left to
@@ -197,14 +227,6 @@ struct CGrid {
     float lim[kLevels];        // largest margin of level L: lim_0 * 4^L
     float reach_max[kLevels];  // largest reach of level L: rmax + lim
 };
-
-// Control words of a sweep (zeroed with the bucket counters, which follow them;
-// the two at kCtlTotal are one 64-bit counter).
-enum : uint32_t {
-    kCtlTotal = 0, kCtlMask = 2, kCtlOver, kCtlBad, kCtlRounds, kCtlInf, kCtlMissed, kCtlQuiet, kCtlMembers, kCtlFull,
-    kCtlQueue = 12, kCtlEmax = kCtlQueue + kQueues, kCtlWords = 32
-};
-static_assert(kCtlEmax + kLevels <= (int)kCtlWords, "control words");
 
 __device__ __forceinline__ int cell_coord_d(double x, double inv_h) {
     double c = floor(x * inv_h);
@@ -1299,6 +1321,8 @@ public:
             BD_HIP(hipMemcpyAsync(planes_.p, pl.data(), pl.size() * sizeof(float4), hipMemcpyHostToDevice, stream_));
         }
         if (!host_ctl_) BD_HIP(hipHostMalloc((void **)&host_ctl_, 64 * sizeof(uint32_t), hipHostMallocDefault));
+        host_ctl_[kCtlWords] = verdict_ = 0u;
+        zeroed_[0] = zeroed_[1] = false;
         rmax_ = 0.0f;
         for (float r : s.c_r) rmax_ = std::max(rmax_, r);
         if (Nc_ > kIdxMaskG) {
@@ -1326,6 +1350,7 @@ public:
         bp.N = N_; bp.Np = Np_; bp.Nc = Nc_;
         bp.ncol = ncol_;
         for (uint32_t step = 0; step < sp.sub_steps; step++) {
+            bp.first_acc = (sp.first_acc && step == 0 && acc0_.p) ? 1u : 0u;
             // links, k sweeps; polygon centres before the last sweep
             for (uint32_t it = 0; it < sp.link_iters; it++) {
                 if (P_ && it + 1 == sp.link_iters) {
@@ -1343,21 +1368,18 @@ public:
                 st.launches++;
             }
             if (Nc_ >= 2) {
-                int rc = circles(st, err);
+                int rc = circles(st, err, P_ < 2 ? &bp : nullptr);
                 if (rc) return rc;
+                if (P_ < 2) {  // the bodies came with the sweep
+                    st.substeps++;
+                    continue;
+                }
             }
             if (P_ >= 2) {
                 hipLaunchKernelGGL(k_poly_pairs, dim3(1), dim3(256), 0, stream_, pos_.p, ptab_.p, P_, centers_.p);
                 st.launches++;
             }
-            bp.first_acc = (sp.first_acc && step == 0 && acc0_.p) ? 1u : 0u;
-            if (N_) {
-                uint32_t blocks = std::min<uint32_t>((N_ + 255) / 256, 65535u * 4);
-                hipLaunchKernelGGL(k_bodies, dim3(blocks), dim3(256), 0, stream_, pos_.p, prev_.p,
-                                   has_pins_ ? pinmask_.p : nullptr, crad_.p, acc0_.p, gflags_.p, colhdr_.p, colgeo_.p,
-                                   planes_.p, bp);
-                st.launches++;
-            }
+            if (N_) launch_bodies(bp, nullptr, st);
             st.substeps++;
         }
         if (sp.first_acc && acc0_.p) {
@@ -1406,7 +1428,8 @@ private:
     // from per-circle margins on the level grid, components, then the lane and
     // workgroup replays.  A sweep in which some circle went further than 0.9 of
     // its margin is undone and run again with the needs it showed.
-    int circles(Stats &st, std::string &err) {
+    // With bodies, the per-body phase follows in the attempt that stands.
+    int circles(Stats &st, std::string &err, const BodyParams *bodies) {
         const uint32_t nc = Nc_;
         const uint32_t nb = (nc + 255) / 256;
         uint32_t T = 1;
@@ -1417,9 +1440,10 @@ private:
         const size_t zn = kCtlWords + (size_t)T + 1;
         const int rw = place_workspace(nc, T, zn, err);
         if (rw) return rw;
-        uint32_t *const ctl = ws_.zero, *const count = ctl + kCtlWords;
         if (!cand_cap_) cand_cap_ = std::max<uint64_t>(4ull * nc, 1024);
         for (int attempt = 0; attempt < 12; attempt++) {
+            const uint32_t turn = turn_;
+            uint32_t *const ctl = ws_.zero[turn], *const count = ctl + kCtlWords;
             BD_HIP(cc_cand_.alloc(cand_cap_));
             BD_HIP(cg_traj_.alloc(cand_cap_));
             // Level 0 takes margins up to 1.5 r_max, also while the base margin is
@@ -1427,7 +1451,8 @@ private:
             // 1 each scans 5x5 cells of level 0 (limit s0 17.4 ms, 0.5 r_max 16.9, 1.0
             // to 2.0 16.4 for 262,144 circles).
             const float lim0 = std::max(s0_, 1.5f * rmax_);
-            fill_u32(ws_.zero, zn, 0u, st);
+            if (!zeroed_[turn]) fill_u32(ctl, zn, 0u, st);
+            zeroed_[turn] = false;
             hipLaunchKernelGGL(k_cg_prep, dim3(nb), dim3(256), 0, stream_, pos_.p, Np_, cg_need_.p, cg_order_.p, s0_,
                                lim0, rmax_, nc,
                                tmask, stride, ws_.grid, ws_.key, count, ctl);
@@ -1469,9 +1494,15 @@ private:
             hipLaunchKernelGGL(k_cg_verify, dim3(std::min<uint32_t>((nc + 3) / 4, kVerifyGrid)), dim3(256), 0, stream_, bk,
                                ws_.aux, ws_.exc, ws_.grid, ws_.cnt, ws_.off, cc_cand_.p, ws_.overq,
                                cg_traj_.p, ctl);
-            st.launches += 11;
-            BD_HIP(hipMemcpyAsync(host_ctl_, ctl, kCtlWords * sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
-            BD_HIP(hipStreamSynchronize(stream_));
+            hipLaunchKernelGGL(k_cg_verdict, dim3(1), dim3(64), 0, stream_, ctl, host_ctl_, ++verdict_);
+            st.launches += 12;
+            if (bodies) launch_bodies(*bodies, ctl, st);
+            turn_ ^= 1u;
+            fill_u32(ws_.zero[turn_], zn, 0u, st);
+            BD_HIP(hipGetLastError());
+            zeroed_[turn_] = true;
+            rc = await_verdict(err);
+            if (rc) return rc;
             uint64_t total;
             std::memcpy(&total, host_ctl_ + kCtlTotal, sizeof total);
             if (host_ctl_[kCtlFull]) {
@@ -1515,10 +1546,33 @@ private:
         return BD_ERR_COLLISION;
     }
 
+    void launch_bodies(const BodyParams &bp, const uint32_t *verdict, Stats &st) {
+        const uint32_t blocks = std::min<uint32_t>((N_ + 255) / 256, 65535u * 4);
+        hipLaunchKernelGGL(k_bodies, dim3(blocks), dim3(256), 0, stream_, pos_.p, prev_.p,
+                           has_pins_ ? pinmask_.p : nullptr, crad_.p, acc0_.p, gflags_.p, colhdr_.p, colgeo_.p,
+                           planes_.p, bp, verdict);
+        st.launches++;
+    }
+
+    // Waits for the last verdict: for its number at first, where a sweep takes some
+    // hundred microseconds, then for the stream.
+    int await_verdict(std::string &err) {
+        auto here = [&]() { return __atomic_load_n(host_ctl_ + kCtlWords, __ATOMIC_ACQUIRE) == verdict_; };
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+        while (!here()) {
+            if (std::chrono::steady_clock::now() < until) continue;
+            BD_HIP(hipStreamSynchronize(stream_));
+            if (here()) break;
+            err = "circle pair sweep gave no verdict";
+            return BD_ERR_DEVICE;
+        }
+        return BD_OK;
+    }
+
     // The sweep's workspace, one allocation: 22 of them, and as many releases, took
     // 1.5 to 4 ms of a scene's life (a clone rolled out for 32 sweeps: 16 ms).
     struct Workspace {
-        uint32_t *zero, *start, *cnt, *off, *par, *root, *place, *csize, *cstart, *members, *queues, *overq, *head, *nxp,
+        uint32_t *zero[2], *start, *cnt, *off, *par, *root, *place, *csize, *cstart, *members, *queues, *overq, *head, *nxp,
             *stamp;
         float *exc;
         float2 *spos;
@@ -1536,7 +1590,7 @@ private:
         };
         auto all = [&]() {
             at = 0;
-            take(ws_.zero, zn);
+            take(ws_.zero[0], zn); take(ws_.zero[1], zn);
             take(ws_.grid, 1);
             take(ws_.key, nc); take(ws_.start, (size_t)T + 1); take(ws_.rec, nc); take(ws_.aux, nc);
             take(ws_.spos, nc); take(ws_.exc, nc); take(ws_.cnt, nc); take(ws_.off, nc);
@@ -1584,7 +1638,11 @@ private:
     DevBuf<float> cg_need_;
     uint64_t cand_cap_ = 0;  // list entries there is room for
     ScanTemp scan_tmp_;
-    uint32_t *host_ctl_ = nullptr;
+    // page-locked: the last verdict's words and its number
+    uint32_t *host_ctl_ = nullptr, verdict_ = 0;
+    // the counters alternate between sweeps; those of the next one are zeroed ahead
+    uint32_t turn_ = 0;
+    bool zeroed_[2] = {false, false};
 };
 
 Engine *make_global_engine(hipStream_t stream) { return new GlobalEngine(stream); }

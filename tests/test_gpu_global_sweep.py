@@ -78,3 +78,27 @@ def test_levels(n, mixed):
     c[:, 2:4] -= (speed * rng.standard_normal((n, 2)) * DT / 2).astype(np.float32)
     c[0, 0:4] += 3000.0
     check(c, 3, 5000.0)
+
+
+@pytest.mark.parametrize("polygons", [0, 1, 2, 3])
+def test_bodies_after_a_sweep_run_again(polygons):
+    # fast circles bring sweeps that run again; the bodies move once, also where
+    # they are queued with the sweep (no two polygons), with initial acc pending
+    rng = np.random.default_rng(polygons)
+    s = Solver()
+    s.set_engine(BD_ENGINE_GLOBAL)
+    s.gravity, s.bounds = (0.0, -9.0), ((-10.0, -10.0), (90.0, 90.0))
+    s.set_sub_steps(3)
+    c = at(rng.uniform(0.0, 60.0, (1500, 2)).astype(np.float32), rng.uniform(0.2, 0.9, 1500))
+    c[:, 2:4] -= (25.0 * rng.standard_normal((1500, 2)) * DT / 3).astype(np.float32)
+    c[:, 4:6] = rng.uniform(-5.0, 5.0, (1500, 2))
+    s.add_circles(c)
+    s.add_particle((5.0, 5.0))
+    for k in range(polygons):
+        s.add_polygon_circle(5.0, (20.0 + 8.0 * k, 70.0), 8, k == 2)
+    o = to_oracle(s, 32)
+    for _ in range(4):
+        s.update(DT)
+        assert o.update(DT) == 0
+        assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
+    assert s.stats()["cc_redos"] > 0
