@@ -82,8 +82,9 @@ typedef float F4 __attribute__((ext_vector_type(4)));
 // particles and polygon points).  hdr: (kind, plane offset, planes, -);
 // geo: circle (cx, cy, R, -); pl: polygon edge planes (nx, ny, c, -).  The
 // records are uniform and come through the scalar cache into scalar registers
-// (staged in LDS every wavefront read two records a collider: 262,144 circles
-// over 68 colliders @B -> @A us; 640 flying bodies: their phase 20 % shorter).
+// (262,144 circles over 68 colliders: staged in LDS, two reads a collider for
+// every wavefront, 19.9 us; from the scalar cache one by one, two dependent loads
+// each, 21.6; four at a time 14.2.  48 flying bodies: a pass 5 % shorter).
 // kU: how many at a time.  The tiled pass takes one: four held 87 scalar registers
 // instead of 63 there, two of its workgroups no longer shared a CU, and a pass over
 // 1,048,576 points took 18.2 us instead of 15.2.
