@@ -53,10 +53,9 @@ __global__ void __launch_bounds__(WG) k_tiled_pass(const float2 *__restrict__ sr
     auto bound = [&](uint32_t L) { return L < 64u ? (uint32_t)__builtin_amdgcn_readlane(held, L) : lo[L]; };
     // A thread's first two records of the next layer load while it solves the
     // current one (and stay in flight across the barrier): nothing is left
-    // behind a barrier but LDS and arithmetic.  Loads past a layer's end read
-    // its tile's first record instead, unused.  (1024 x 1024 cloth: 0.515 ->
+    // behind a barrier but LDS and arithmetic.  (1024 x 1024 cloth: 0.515 ->
     // 0.475 ms an update.)
-    auto load = [&](uint32_t l, uint32_t e) { return lk[l < e ? l : 0u]; };
+    auto load = [&](uint32_t l, uint32_t e) { return lk[tile_record(l, e)]; };
     uint32_t b0 = bound(0), b1 = bound(1);
     LinkS n0 = load(b0 + tid, b1), n1 = load(b0 + WG + tid, b1);
     for (uint32_t r = tid; r < ti.int_count; r += WG) s_reg[region_slot(r)] = src[ti.int_start + r];

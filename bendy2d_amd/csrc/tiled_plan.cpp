@@ -128,6 +128,7 @@ bool build_pass(const Plan &p, const TilePlan &tp, const Incidence &inc, const s
                 cnt += (uint32_t)v.size();
             }
             out.loff.push_back(cnt);
+            if (cnt == 0) ti.link_off = 0;  // (its layers have links elsewhere: record 0 is there)
             out.link_count += cnt;
             out.max_region = std::max<uint32_t>(out.max_region, (uint32_t)((R.size() + 15) & ~size_t(15)));
             out.tiles.push_back(ti);
@@ -210,9 +211,14 @@ uint64_t tile_plan_selfcheck(const HostScene &s, const Plan &p, const TilePlan &
         solve_particle_link(A.x, A.y, B.x, B.y, l.t, (l.a & kPinBit) != 0, (l.b & kPinBit) != 0);
     }
     std::vector<V2> reg;
+    uint64_t bad = 0;
     for (const TilePass &ps : tp.passes) {
         const uint32_t nl = ps.L1 - ps.L0;
         for (const TileInfo &ti : ps.tiles) {
+            for (uint32_t d = 0; d < nl; d++) {
+                const uint32_t b = ps.loff[ti.loff_off + d], e = ps.loff[ti.loff_off + d + 1];
+                for (uint32_t l = b; l <= e; l++) bad += (uint64_t)ti.link_off + tile_record(l, e) >= ps.links.size();
+            }
             reg.assign((ti.int_count + ti.halo_count + 15) & ~15u, V2{0.0f, 0.0f});
             for (uint32_t r = 0; r < ti.int_count; r++) reg[region_slot(r)] = cur[ti.int_start + r];
             for (uint32_t h = 0; h < ti.halo_count; h++)
@@ -227,7 +233,6 @@ uint64_t tile_plan_selfcheck(const HostScene &s, const Plan &p, const TilePlan &
         }
         std::swap(cur, nxt);
     }
-    uint64_t bad = 0;
     for (uint32_t i = 0; i < N; i++)
         bad += (std::memcmp(&cur[i].x, &seq[i].x, 4) != 0) + (std::memcmp(&cur[i].y, &seq[i].y, 4) != 0);
     return bad;

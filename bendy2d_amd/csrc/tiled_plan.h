@@ -32,6 +32,11 @@ namespace bd {
 // so a region of n points needs ceil(n / 16) * 16 slots.
 BD_HD uint32_t region_slot(uint32_t m) { return m ^ ((m >> 4) & 15u); }
 
+// The record of its tile that a lane loads ahead as the l-th of a layer that ends
+// at record e: past the end the tile's first one, unused.  A tile without links
+// has no record of its own, so its link_off has to name one all the same.
+BD_HD uint32_t tile_record(uint32_t l, uint32_t e) { return l < e ? l : 0u; }
+
 struct TileInfo {
     uint32_t int_start, int_count;   // interior: internal points [int_start, int_start + int_count)
     uint32_t halo_off, halo_count;   // halo: internal indices halo[halo_off ...]
@@ -66,7 +71,9 @@ int build_tile_plan(const HostScene &s, const Plan &p, uint32_t tile_points, uin
 
 // Runs one sweep of the plan on the host with the engine's link arithmetic
 // and compares it with the sequential sweep over the same positions.
-// Returns the number of differing f32 values (0: the schedule is exact).
+// Returns the number of differing f32 values (0: the schedule is exact), plus
+// the number of records that a pass of the engine would load from outside the
+// plan's.
 uint64_t tile_plan_selfcheck(const HostScene &s, const Plan &p, const TilePlan &tp);
 
 }  // namespace bd

@@ -44,3 +44,20 @@ def test_tiled_schedule_random_graph():
     s.set_pinned_range(0, (rng.random(n) < 0.05).astype(np.uint8))
     bad, passes = s.tiled_selfcheck(256, 2048)
     assert bad == 0 and passes >= 1
+
+
+@pytest.mark.parametrize("n,linked,chain,cap", [
+    (20480, 513, 1, 16384),    # 512 records, a whole page, and 38 of 40 tiles without links
+    (20480, 513, 1, 544),
+    (5000, 65, 3, 16384),
+    (1025, 2, 1, 1100),        # one link; the last tile is one free particle
+])
+def test_tiles_without_links_load_inside_the_records(n, linked, chain, cap):
+    s = Solver()
+    i = np.arange(n)
+    s.add_particles(np.stack([i % 128, i // 128], 1).astype(np.float32))
+    a = np.arange(0, linked - 1)
+    for d in range(chain):
+        s.add_particle_links(a[: linked - 1 - d], a[: linked - 1 - d] + 1 + d, np.full(linked - 1 - d, 0.9, np.float32))
+    bad, passes = s.tiled_selfcheck(512, cap)
+    assert bad == 0 and passes >= 1
