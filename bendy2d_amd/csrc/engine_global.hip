@@ -720,10 +720,11 @@ __device__ __forceinline__ void note_rounds(uint32_t *ctl, uint32_t rounds) {
 // rounds but the trajectory.  (20,011 circles 28 -> 11 us, 262,144 72 -> 45 us
 // against a wavefront with the state in LDS and a worklist for each component, and
 // a serial replay by one lane for those of up to 4.)  The lists, as places in the component, are
-// staged in LDS.  A component with a longer list than kLaneList joins the queue of
-// the LDS workgroups.
+// staged in LDS, each with a bit for a partner of larger number: such a pair's first
+// end is the circle itself (the order shows in the sign of a zero).  A component with
+// a longer list than kLaneList joins the queue of the LDS workgroups.
 template <uint32_t W>
-__device__ __forceinline__ void replay_lanes(uint32_t first, uint32_t step, const uint32_t *__restrict__ queue,
+__device__ __forceinline__ void replay_lanes(uint32_t from, uint32_t step, const uint32_t *__restrict__ queue,
                                              uint32_t nq, float2 *__restrict__ P, const float4 *__restrict__ aux,
                                              const float4 *__restrict__ rec, float *__restrict__ exc,
                                              const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ off,
@@ -732,10 +733,10 @@ __device__ __forceinline__ void replay_lanes(uint32_t first, uint32_t step, cons
                                              const uint32_t *__restrict__ place, uint32_t *__restrict__ lds_queue,
                                              float2 *__restrict__ traj, uint32_t *__restrict__ ctl,
                                              uint8_t (*s_list)[kLaneList + 4]) {
-    constexpr uint32_t kNone8 = 0xffu;
+    constexpr uint32_t kNone8 = 0xffu, kLater8 = 0x40u;
     const uint32_t lane = threadIdx.x & 63u, k = lane & (W - 1u), base = lane & ~(W - 1u);
     uint32_t most = 0;
-    for (uint32_t q0 = first; q0 < nq; q0 += step) {  // uniform per wavefront
+    for (uint32_t q0 = from; q0 < nq; q0 += step) {  // uniform per wavefront
         const uint32_t q = q0 + lane / W;
         uint32_t c = 0, m = 0, o = 0, r = 0;
         float2 p = make_float2(0.0f, 0.0f), p0 = p;
@@ -765,9 +766,9 @@ __device__ __forceinline__ void replay_lanes(uint32_t first, uint32_t step, cons
         for (uint32_t t0 = 0; t0 < m; t0 += kU) {
             uint32_t v[kU];
 #pragma unroll
-            for (uint32_t u = 0; u < kU; u++) v[u] = cand[o + min(t0 + u, m - 1u)] & kIdxMaskG;
+            for (uint32_t u = 0; u < kU; u++) v[u] = cand[o + min(t0 + u, m - 1u)];
 #pragma unroll
-            for (uint32_t u = 0; u < kU; u++) v[u] = place[v[u]];
+            for (uint32_t u = 0; u < kU; u++) v[u] = place[v[u] & kIdxMaskG] | (v[u] & kLater ? kLater8 : 0u);
 #pragma unroll
             for (uint32_t u = 0; u < kU; u++) s_list[lane][t0 + u] = (uint8_t)v[u];  // (kU - 1 past the end at most)
         }
@@ -778,14 +779,16 @@ __device__ __forceinline__ void replay_lanes(uint32_t first, uint32_t step, cons
             const uint32_t theirs = (uint32_t)__shfl((int)next, src);
             const float2 pj = make_float2(__shfl(p.x, src), __shfl(p.y, src));
             const float rj = __shfl(rad, src);
-            const bool ready = next != kNone8 && theirs == k;
+            const bool first = (next & kLater8) != 0u;
+            // (my partner's entry for me has the other bit; kNone8 is neither)
+            const bool ready = next != kNone8 && theirs == (first ? k : k | kLater8);
             if (!__ballot(ready)) break;
             if (ready) {
                 const uint32_t after = s_list[lane][head + 1u];
-                float2 a = k < next ? p : pj, b = k < next ? pj : p;
+                float2 a = first ? p : pj, b = first ? pj : p;
                 float qi = 0.0f, qj = 0.0f;
-                if (solve_circle_pair(a.x, a.y, b.x, b.y, k < next ? rad : rj, k < next ? rj : rad, qi, qj)) {
-                    p = k < next ? a : b;
+                if (solve_circle_pair(a.x, a.y, b.x, b.y, first ? rad : rj, first ? rj : rad, qi, qj)) {
+                    p = first ? a : b;
                     e = excursion(e, p.x, p.y, p0.x, p0.y);
                 }
                 traj[o + head] = p;
@@ -836,8 +839,9 @@ __global__ void __launch_bounds__(64) k_cg_lanes(float2 *__restrict__ P, const f
 // Components of 65 .. kLdsMembers circles, and smaller ones with long lists: a
 // workgroup each, with the round protocol in LDS.  The members' positions, start
 // positions, radii and excursions are staged into LDS and the lists remapped to
-// local indices (a circle's place among the members); the lists keep their
-// order, which is all the protocol depends on.  Positions after each pair go to
+// local indices (a circle's place among the members, with kLater16 for a partner of
+// larger number: the pair's first end is then the circle itself); the lists keep
+// their order, which is all the protocol depends on.  Positions after each pair go to
 // traj in global memory as in the other replays.  A component whose lists do
 // not fit joins the queue of the global-memory workgroups.
 __global__ void __launch_bounds__(256) k_cg_lds(float2 *__restrict__ P, const float4 *__restrict__ aux,
@@ -857,8 +861,17 @@ __global__ void __launch_bounds__(256) k_cg_lds(float2 *__restrict__ P, const fl
     __shared__ uint32_t s_wl[2][kLdsMembers / 2 + 1];
     __shared__ uint32_t s_n[3], s_bad;
     __shared__ uint64_t s_sum[4];
-    constexpr uint16_t kNone16 = 0xffffu;
+    constexpr uint16_t kNone16 = 0xffffu, kLater16 = 0x8000u;
+    static_assert(kLdsMembers <= 0x7fffu, "a place and its flag in 16 bits");
     const uint32_t tid = threadIdx.x;
+    // the pair that x's next entry y makes, its first end in the low half, once x is
+    // the next partner of y too; 0 when it is not (no pair is: the ends differ)
+    auto pair_of = [&](uint32_t x, uint32_t y) -> uint32_t {
+        if (y == kNone16) return 0u;
+        const uint32_t o = y & 0x7fffu;
+        if (y & kLater16) return s_nxp[o] == x ? x | (o << 16) : 0u;
+        return s_nxp[o] == (x | kLater16) ? o | (x << 16) : 0u;
+    };
     if (ctl[kCtlFull]) return;  // uniform
     const uint32_t nmid = ctl[kCtlQueue + kQueueLds];
     const uint32_t *const queue = queues + (size_t)kQueueLds * nc;
@@ -903,7 +916,8 @@ __global__ void __launch_bounds__(256) k_cg_lds(float2 *__restrict__ P, const fl
         for (uint32_t k = tid; k < n; k += 256u) {
             const uint32_t *src = cand + s_off[k];
             uint16_t *dst = s_list + s_lb[k];
-            for (uint32_t e = 0, m = s_cnt[k]; e < m; e++) dst[e] = (uint16_t)place[src[e] & kIdxMaskG];
+            for (uint32_t e = 0, m = s_cnt[k]; e < m; e++)
+                dst[e] = (uint16_t)(place[src[e] & kIdxMaskG] | (src[e] & kLater ? kLater16 : 0u));
         }
         __syncthreads();
         for (uint32_t k = tid; k < n; k += 256u) {
@@ -913,8 +927,8 @@ __global__ void __launch_bounds__(256) k_cg_lds(float2 *__restrict__ P, const fl
         }
         __syncthreads();
         for (uint32_t k = tid; k < n; k += 256u) {
-            const uint32_t o = s_nxp[k];
-            if (o != kNone16 && k < o && s_nxp[o] == k) s_wl[0][atomicAdd(&s_n[0], 1u)] = k | (o << 16);
+            const uint32_t y = s_nxp[k], pr = y & kLater16 ? pair_of(k, y) : 0u;  // each from its first end
+            if (pr) s_wl[0][atomicAdd(&s_n[0], 1u)] = pr;
         }
         __syncthreads();
         uint32_t cur = s_n[0], rounds = 0;
@@ -947,10 +961,10 @@ __global__ void __launch_bounds__(256) k_cg_lds(float2 *__restrict__ P, const fl
             for (uint32_t k = tid; k < cur; k += 256u) {
                 const uint32_t pr = s_wl[cb][k];
                 for (int e = 0; e < 2; e++) {
-                    const uint32_t x = e ? pr >> 16 : pr & 0xffffu, y = s_nxp[x];
-                    if (y == kNone16 || s_nxp[y] != x) continue;
-                    if (s_stamp[y] == (uint16_t)rounds && y < x) continue;
-                    s_wl[nb][atomicAdd(&s_n[(rounds + 1u) % 3u], 1u)] = min(x, y) | (max(x, y) << 16);
+                    const uint32_t x = e ? pr >> 16 : pr & 0xffffu, y = s_nxp[x], np = pair_of(x, y);
+                    // when both ends moved this round the first one adds the pair
+                    if (np == 0u || (s_stamp[y & 0x7fffu] == (uint16_t)rounds && !(y & kLater16))) continue;
+                    s_wl[nb][atomicAdd(&s_n[(rounds + 1u) % 3u], 1u)] = np;
                 }
             }
             __syncthreads();
@@ -974,8 +988,9 @@ __global__ void __launch_bounds__(256) k_cg_lds(float2 *__restrict__ P, const fl
 // Components above kLdsMembers circles (or whose lists overflow LDS): one
 // workgroup each, taken from a queue,
 // with the round protocol.  head[c] counts c's processed partners and nxp[c]
-// is the next one (kNoneG when done), so (x, y) is ready exactly when
-// nxp[x] == y and nxp[y] == x.  Every round applies at least one pair, so the
+// is the next one (kNoneG when done; with kLater when its number is larger, c then
+// being the pair's first end), so (x, y) is ready exactly when
+// nxp[x] is y and nxp[y] is x.  Every round applies at least one pair, so the
 // loop ends; a list left unfinished (a schedule that stalls) is reported.
 __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ P, const float4 *__restrict__ aux,
                                                       const float4 *__restrict__ rec, float *__restrict__ exc,
@@ -994,6 +1009,11 @@ __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ P, co
     if (ctl[kCtlFull]) return;  // uniform
     const uint32_t nbig = ctl[kCtlQueue + kQueueBig];
     const uint32_t *const bigq = queues + (size_t)kQueueBig * nc;
+    constexpr uint32_t kEntry = kIdxMaskG | kLater;
+    // whether x is the next partner of its own next partner y
+    auto mutual = [&](uint32_t x, uint32_t y) {
+        return y != kNoneG && nxp[y & kIdxMaskG] == (y & kLater ? x : x | kLater);
+    };
     for (uint32_t q = blockIdx.x; q < nbig; q += gridDim.x) {  // uniform per workgroup
         const uint32_t r = bigq[q], base = cstart[r], n = csize[r];
         const uint32_t *M = members + base;
@@ -1001,14 +1021,14 @@ __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ P, co
         for (uint32_t k = tid; k < n; k += kCompWG) {
             const uint32_t c = M[k];
             head[c] = 0u;
-            nxp[c] = cnt[c] ? cand[off[c]] & kIdxMaskG : kNoneG;
+            nxp[c] = cnt[c] ? cand[off[c]] & kEntry : kNoneG;
             stamp[c] = kNoneG;
         }
         if (tid == 0) { s_n[0] = 0u; s_n[1] = 0u; s_n[2] = 0u; s_bad = 0u; }
         __syncthreads();
         for (uint32_t k = tid; k < n; k += kCompWG) {
-            const uint32_t c = M[k], o = nxp[c];
-            if (o != kNoneG && c < o && nxp[o] == c) W[0][atomicAdd(&s_n[0], 1u)] = make_uint2(c, o);
+            const uint32_t c = M[k], y = nxp[c];
+            if ((y & kLater) && mutual(c, y)) W[0][atomicAdd(&s_n[0], 1u)] = make_uint2(c, y & kIdxMaskG);
         }
         __syncthreads();
         uint32_t cur = s_n[0], rounds = 0;
@@ -1020,8 +1040,8 @@ __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ P, co
                 float2 pi = P[c], pj = P[o];
                 const uint32_t hc = head[c], ho = head[o];
                 const uint32_t oc = off[c], oo = off[o];
-                const uint32_t xc = hc + 1u < cnt[c] ? cand[oc + hc + 1u] & kIdxMaskG : kNoneG;
-                const uint32_t xo = ho + 1u < cnt[o] ? cand[oo + ho + 1u] & kIdxMaskG : kNoneG;
+                const uint32_t xc = hc + 1u < cnt[c] ? cand[oc + hc + 1u] & kEntry : kNoneG;
+                const uint32_t xo = ho + 1u < cnt[o] ? cand[oo + ho + 1u] & kEntry : kNoneG;
                 float qi = 0.0f, qj = 0.0f;
                 if (solve_circle_pair(pi.x, pi.y, pj.x, pj.y, aux[c].x, aux[o].x, qi, qj)) {
                     P[c] = pi;
@@ -1042,14 +1062,14 @@ __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ P, co
             if (tid == 0) s_n[(rounds + 2u) % 3u] = 0u;  // read two barriers ago
             __syncthreads();
             // pairs completed by a moved head; when both ends moved this round
-            // the smaller one adds the pair
+            // the first one adds the pair
             for (uint32_t k = tid; k < cur; k += kCompWG) {
                 const uint2 pr = W[cb][k];
                 for (int e = 0; e < 2; e++) {
-                    const uint32_t x = e ? pr.y : pr.x, y = nxp[x];
-                    if (y == kNoneG || nxp[y] != x) continue;
-                    if (stamp[y] == rounds && y < x) continue;
-                    W[nb][atomicAdd(&s_n[(rounds + 1u) % 3u], 1u)] = make_uint2(min(x, y), max(x, y));
+                    const uint32_t x = e ? pr.y : pr.x, y = nxp[x], o = y & kIdxMaskG;
+                    const bool first = (y & kLater) != 0u;
+                    if (!mutual(x, y) || (stamp[o] == rounds && !first)) continue;
+                    W[nb][atomicAdd(&s_n[(rounds + 1u) % 3u], 1u)] = first ? make_uint2(x, o) : make_uint2(o, x);
                 }
             }
             __syncthreads();

@@ -102,3 +102,29 @@ def test_bodies_after_a_sweep_run_again(polygons):
         assert o.update(DT) == 0
         assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
     assert s.stats()["cc_redos"] > 0
+
+
+@pytest.mark.parametrize("size", [2, 4, 5, 16, 17, 64, 65, 1024, 1025])
+@pytest.mark.parametrize("clump", [False, True])
+def test_pairs_are_taken_by_circle_number(size, clump):
+    # every circle at x = -0: a pair's push leaves +0 at its first circle (the one
+    # with the smaller number) and -0 at its second, so the signs in the previous
+    # positions after one substep tell which end a replay took first.  Columns of
+    # `size` circles, each overlapping the next; with clump one more in each place,
+    # numbered far from it.
+    rows = max(2, 130 // size)
+    y = np.array([1.05 * size * r + 0.9 * k for r in range(rows) for k in range(size)])
+    if clump:
+        y = np.concatenate([y, y + 0.3])
+    xy = np.stack([np.full(len(y), -0.0), y], 1).astype(np.float32)
+    rng = np.random.default_rng(size)
+    s = Solver()
+    s.set_engine(BD_ENGINE_GLOBAL)
+    s.gravity, s.bounds = (0.0, 0.0), ((-9000.0, -9000.0), (18000.0, 18000.0))
+    s.add_circles(at(xy[rng.permutation(len(xy))], 0.5))
+    o = to_oracle(s, 32)
+    s.update(DT)
+    assert o.update(DT) == 0
+    a, b = state(s), state(o)
+    assert np.signbit(b[2::4]).any() and not np.signbit(b[2::4]).all()
+    assert bits_equal(a, b), first_diff(a, b)
