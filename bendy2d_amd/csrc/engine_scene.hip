@@ -1193,9 +1193,16 @@ __device__ __forceinline__ void fallback_sweep(float2 *P, uint32_t Np, uint32_t 
 // margins raises the scene's level by two, kLevelClean sweeps without one lower it: a
 // settling pile stays at level 0 (its rounds grow with the margins), a hot gas,
 // whose first contacts push circles by most of a radius, at the top (its rounds
-// are few: 16,000 circles ran every sweep twice at level 0).
+// are few: 16,000 circles ran every sweep twice at level 0).  Level and count are
+// kept between launches: counted anew in each, a launch of fewer than kLevelClean
+// sweeps could only raise the level (4,096 soft bodies piled up, 8 sweeps a launch:
+// 6.0e6 rounds and 26.2 ms an update, 3.4e6 and 23.1 with the count kept).  A level
+// given up too soon costs a second run of the sweep, one kept too long longer rounds
+// (those bodies, and a dozen batches of piles from their first contact on: 16 sweeps
+// 23.4 ms and 16.8 on average, 32 23.1 and 16.3, 64 23.8 and 16.7).
 constexpr float kActiveBase = 0.05f;
-constexpr uint32_t kLevels = 4u, kLevelClean = 16u;
+constexpr uint32_t kLevels = 4u, kLevelClean = 32u;
+static_assert(kLevels < 128u && kLevelClean <= 128u, "kept between launches in 7 bits each");
 constexpr uint32_t kCurMask = 0x00ffffffu;
 constexpr uint32_t kStamp8 = 0xffu;
 static_assert(kCandCap * 65536ull <= kCurMask + 1ull, "a list cursor must fit 24 bits");
@@ -2375,7 +2382,7 @@ __device__ __forceinline__ void run_scene(const SceneDesc *__restrict__ dp, uint
     uint32_t err = uni(st->err);
     if (tid == 0) {
         s_cc->cs = CCShared::Steer{st->skin, (uint32_t)st->list_valid & 1u, st->pairs, st->since_build, st->s_cell, st->smin,
-                                   (uint32_t)st->list_valid >> 1, 0u};
+                                   (uint32_t)st->list_valid >> 1, (uint32_t)st->ws_ready >> 1};
         s_cc->fb_streak = 0u;
         CCShared::Counts &k = s_cc->cnt;
         k = CCShared::Counts{};
@@ -2480,7 +2487,7 @@ __device__ __forceinline__ void run_scene(const SceneDesc *__restrict__ dp, uint
         st->redos += k.redos;
         st->rebuilds += k.rebuilds;
         st->pairs = cs.pairs;
-        if (Nc >= 2) st->ws_ready = 1u;
+        if (Nc >= 2) st->ws_ready = (uint8_t)(1u | (cs.clean << 1));
         st->t_links += k.t_links;
         st->t_build += k.t_build;
         st->t_sweep += k.t_sweep - k.t_build;

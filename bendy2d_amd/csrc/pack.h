@@ -68,7 +68,8 @@ struct SceneState {
     float skin;          // base candidate margin of the circle-pair schedule
     uint8_t list_valid;  // bit 0: candidate list built and still usable; above: level of the
                          // active margins
-    uint8_t ws_ready;    // per-circle skin state initialised
+    uint8_t ws_ready;    // bit 0: per-circle skin state initialised; above: sweeps since a margin
+                         // was too small
     uint16_t sub_phase;  // substeps of the current update already run (a launch's time budget
                          // stopped the scene inside an update)
     uint32_t err;        // nonzero: the circle-pair schedule failed

@@ -97,3 +97,26 @@ def test_grid_edges(n, span, lds):
         assert o.update(DT) == 0
     b.read_scene(0, s)
     assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
+
+
+@pytest.mark.parametrize("n", [65, 300])
+@pytest.mark.parametrize("speed", [20.0, 60.0])
+def test_the_launches_do_not_change_the_schedule(n, speed):
+    # what a scene has learnt (margins, and the sweeps since one was too small) is
+    # kept between launches: the same rounds, sweeps run again and lists, a launch
+    # for each update (4 sweeps) or for 16 of them
+    def run(per_launch):
+        b = Batch()
+        s = pile(n, n, False, speed)
+        b.add_scene(s)
+        b.config = dict(steps_per_launch=per_launch)
+        b.update(DT, 48)
+        b.sync()
+        st = b.scene_status(0)
+        b.read_scene(0, s)
+        assert b.cc_stats()["fallbacks"] == 0  # (a run of those ends with the launch)
+        return state(s), st
+
+    a, b = run(1), run(16)
+    assert a[1]["redos"] > 0
+    assert bits_equal(a[0], b[0]) and a[1] == b[1]
