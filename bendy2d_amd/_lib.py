@@ -185,6 +185,7 @@ _SIGS = [
     ("bd_batch_set_config", c_int32, [_S, POINTER(BatchConfig)]),
     ("bd_batch_get_config", c_int32, [_S, POINTER(BatchConfig)]),
     ("bd_batch_autotune", c_int32, [_S, c_float, c_uint32]),
+    ("bd_batch_get_shapes", c_int32, [_S, POINTER(c_uint32), POINTER(c_uint32)]),
     ("bd_batch_last_timing", c_int32, [_S, POINTER(c_float), POINTER(c_uint32)]),
     ("bd_batch_cc_stats", c_int32, [_S, POINTER(c_uint64), POINTER(c_uint64), POINTER(c_uint64), POINTER(c_uint64)]),
     ("bd_batch_cc_fallbacks", c_int32, [_S, POINTER(c_uint64), POINTER(c_uint64)]),

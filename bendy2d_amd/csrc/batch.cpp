@@ -9,6 +9,7 @@
 #include <memory>
 #include <numeric>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/bendy2d.h"
@@ -484,8 +485,9 @@ int32_t bd_batch_read_scene(bd_batch *b, int64_t id, bd_solver *out) {
     return BD_OK;
 }
 
-int32_t bd_batch_set_config(bd_batch *b, const bd_batch_config *cfg) {
-    if (!b || !cfg) return BD_ERR_ARG;
+// Sets the configuration; adapt: whether the classes may take wider shapes than it
+// says (see choose_shapes).
+static int apply_config(bd_batch *b, const bd_batch_config *cfg, bool adapt) {
     if (variant_for_wg((int)cfg->wg_small) < 0 || variant_for_wg((int)cfg->wg_large) < 0 ||
         (cfg->split_tiny && variant_for_wg((int)cfg->wg_tiny) < 0))
         return fail(BD_ERR_ARG, "workgroup sizes must be 64, 128, 256, 512 or 1024");
@@ -499,13 +501,30 @@ int32_t bd_batch_set_config(bd_batch *b, const bd_batch_config *cfg) {
     if (b->core.cfg.lds_tiny > scene_max_lds()) b->core.cfg.lds_tiny = (uint32_t)scene_max_lds();
     if (b->core.cfg.steps_per_launch < 1) b->core.cfg.steps_per_launch = 1;
     b->core.invalidate_graph();
-    b->core.adapt = false;  // as asked from now on
+    b->core.adapt = adapt;
     b->core.choose_shapes();
     if (reorder && b->uploaded) {
         std::vector<uint32_t> all(b->images.size());
         std::iota(all.begin(), all.end(), 0u);
         b->core.build_order(all);
     }
+    return BD_OK;
+}
+
+int32_t bd_batch_set_config(bd_batch *b, const bd_batch_config *cfg) {
+    if (!b || !cfg) return BD_ERR_ARG;
+    // the classes run as asked once their shape has been asked for
+    auto shapes = [](const bd_batch_config &c) {
+        return std::make_tuple(c.wg_small, c.wg_large, c.split_points, c.lds_small, c.lds_large, c.split_tiny,
+                               c.wg_tiny, c.lds_tiny);
+    };
+    return apply_config(b, cfg, b->core.adapt && shapes(*cfg) == shapes(b->core.cfg));
+}
+
+int32_t bd_batch_get_shapes(const bd_batch *b, uint32_t *wg, uint32_t *lds) {
+    if (!b || !wg || !lds) return BD_ERR_ARG;
+    const BatchCore::Shape *const s[3] = {&b->core.tiny, &b->core.small, &b->core.large};
+    for (int c = 0; c < 3; c++) { wg[c] = s[c]->wg; lds[c] = s[c]->lds; }
     return BD_OK;
 }
 
@@ -641,10 +660,11 @@ int32_t bd_batch_autotune(bd_batch *b, float dt, uint32_t steps) {
     std::vector<uint8_t> acc_save = b->acc_pending;
     std::vector<uint64_t> upd_save = b->updates_run;
     bd_batch_config best = c.cfg;
+    bool best_adapt = c.adapt;
     float best_ms = INFINITY;
     int tried = 0;
-    auto trial = [&](const bd_batch_config &cf) -> float {
-        if (bd_batch_set_config(b, &cf)) return INFINITY;
+    auto trial = [&](const bd_batch_config &cf, bool adapt) -> float {
+        if (apply_config(b, &cf, adapt)) return INFINITY;
         restore();
         b->acc_pending = acc_save;
         float total = 0.0f;
@@ -666,6 +686,13 @@ int32_t bd_batch_autotune(bd_batch *b, float dt, uint32_t steps) {
     };
     const uint32_t wgs[] = {64, 128, 256, 512, 1024};
     const uint32_t splits[] = {512, 1024, 2048, 4096, 8192};
+    // what an untuned batch runs on, where that is wider than its configuration
+    if (c.adapt && c.widened()) {
+        bd_batch_config cf = best;
+        cf.steps_per_launch = 1;
+        best_ms = trial(cf, true);
+        if (best_ms < INFINITY) best = cf;
+    }
     // 1) workgroup sizes and the class split
     for (uint32_t split : splits)
         for (uint32_t ws : wgs)
@@ -674,12 +701,12 @@ int32_t bd_batch_autotune(bd_batch *b, float dt, uint32_t steps) {
                 bd_batch_config cf = best;
                 cf.split_points = split; cf.wg_small = ws; cf.wg_large = wl;
                 cf.steps_per_launch = 1;
-                float ms = trial(cf);
+                float ms = trial(cf, false);
                 // a larger class split has to win by more than 1 %: it puts more
                 // mid-size scenes on the small workgroups, which fall behind once
                 // the scenes come into dense contact
                 const float margin = cf.split_points > best.split_points ? 0.99f : 1.0f;
-                if (ms < best_ms * margin) { best_ms = ms; best = cf; }
+                if (ms < best_ms * margin) { best_ms = ms; best = cf; best_adapt = false; }
             }
     // the class of the smallest scenes keeps its configured shape (by default
     // 400 bodies, 64 lanes, 8 KiB): two-update trials do not rank it the way
@@ -691,18 +718,18 @@ int32_t bd_batch_autotune(bd_batch *b, float dt, uint32_t steps) {
             if (ll < 64 * 1024) continue;
             bd_batch_config cf = best;
             cf.lds_small = ls; cf.lds_large = ll;
-            float ms = trial(cf);
-            if (ms < best_ms) { best_ms = ms; best = cf; }
+            float ms = trial(cf, false);
+            if (ms < best_ms) { best_ms = ms; best = cf; best_adapt = false; }
         }
     // 3) updates per launch
     for (uint32_t spl : {1u, 2u, 4u, 8u}) {
         if (spl > steps) break;
         bd_batch_config cf = best;
         cf.steps_per_launch = spl;
-        float ms = trial(cf);
+        float ms = trial(cf, best_adapt);
         if (ms < best_ms * 0.98f) { best_ms = ms; best = cf; }
     }
-    bd_batch_set_config(b, &best);
+    apply_config(b, &best, best_adapt);
     restore();
     b->acc_pending = acc_save;
     b->updates_run = upd_save;

@@ -23,7 +23,7 @@ struct BatchCore {
     std::vector<uint64_t> order_ticks;   // per scene slot: its device ticks at the last ordering
     std::vector<uint32_t> order_rounds;  // per scene slot: its pair rounds at the last ordering
     uint32_t n_tiny = 0, n_small = 0, n_large = 0;
-    // the configuration is the default one: launches that leave CUs idle take
+    // no shape has been asked for: launches that leave CUs idle take
     // wider workgroups and more LDS than it says (see choose_shapes)
     bool adapt = false;
     struct Shape { uint32_t wg = 0, lds = 0; };
@@ -48,6 +48,10 @@ struct BatchCore {
     void invalidate_graph();
     void build_order(const std::vector<uint32_t> &active);
     void choose_shapes();
+    bool widened() const {
+        return tiny.wg != cfg.wg_tiny || tiny.lds != cfg.lds_tiny || small.wg != cfg.wg_small ||
+               small.lds != cfg.lds_small || large.wg != cfg.wg_large || large.lds != cfg.lds_large;
+    }
     // the same classes, each ordered by cost[slot] (largest first, ties by
     // bodies plus links); the launch graph stays valid
     void order_by(const std::vector<uint64_t> &cost);

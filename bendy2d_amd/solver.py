@@ -355,6 +355,11 @@ class Batch:
             setattr(c, k, int(v))
         check(lib().bd_batch_set_config(self._h, ctypes.byref(c)), "batch_set_config")
 
+    def shapes(self):
+        wg, lds = (ctypes.c_uint32 * 3)(), (ctypes.c_uint32 * 3)()
+        check(lib().bd_batch_get_shapes(self._h, wg, lds), "batch_get_shapes")
+        return list(zip(wg, lds))
+
     def autotune(self, dt, steps=2):
         return check(lib().bd_batch_autotune(self._h, float(dt), int(steps)), "batch_autotune")
 

@@ -303,10 +303,10 @@ typedef struct bd_batch bd_batch;
  * steps_per_launch updates run per kernel launch; use_graph replays the launch
  * sequence as a captured hipGraph.  A third class takes the smallest scenes:
  * those of at most split_tiny bodies run on workgroups of wg_tiny threads with
- * lds_tiny bytes of LDS (split_tiny = 0: no third class).  Until a
- * configuration is set (bd_batch_set_config, bd_batch_autotune, a server's
- * launch), launches whose scenes leave CUs idle take wider workgroups and more
- * LDS than the default one says. */
+ * lds_tiny bytes of LDS (split_tiny = 0: no third class).  Until a shape is set
+ * (wg_*, lds_* or split_* changed by bd_batch_set_config, chosen by
+ * bd_batch_autotune, or given in a server's launch), launches whose scenes leave
+ * CUs idle take wider workgroups and more LDS than the default one says. */
 typedef struct bd_batch_config {
     uint32_t wg_small, wg_large;
     uint32_t split_points;
@@ -332,10 +332,14 @@ int32_t bd_batch_sync(bd_batch *b);
 int32_t bd_batch_read_scene(bd_batch *b, int64_t id, bd_solver *out);
 int32_t bd_batch_set_config(bd_batch *b, const bd_batch_config *cfg);
 int32_t bd_batch_get_config(const bd_batch *b, bd_batch_config *cfg);
+/* What the classes run on (tiny, small, large; known after the first update):
+ * the configured workgroups and LDS, or the wider ones taken instead. */
+int32_t bd_batch_get_shapes(const bd_batch *b, uint32_t wg[3], uint32_t lds[3]);
 /* Time candidate configurations on this batch (each for `steps` updates of
  * dt on a scratch copy of the state, which is restored afterwards, after the
- * same updates once untimed) and keep the fastest: workgroup sizes, the
- * small/large split, LDS budgets, updates per launch.  The smallest class
+ * same updates once untimed) and keep the fastest: the wider shapes that an
+ * untuned batch would take, workgroup sizes, the small/large split, LDS budgets,
+ * updates per launch.  The smallest class
  * keeps its configured shape.  Returns the number of configurations tried. */
 int32_t bd_batch_autotune(bd_batch *b, float dt, uint32_t steps);
 /* Device time of the last bd_batch_update in milliseconds (HIP events on the

@@ -253,3 +253,46 @@ def test_default_shapes_match_oracle(count):
         out = kinds[k % 5][0].clone()
         b.read_scene(k, out)
         assert bits_equal(state(out), kinds[k % 5][1]), f"scene {k}: {first_diff(state(out), kinds[k % 5][1])}"
+
+
+def small_batch(sides):
+    b = Batch()
+    for k, side in enumerate(sides):
+        s = Solver()
+        workloads.softbody(s, 7000 + k, max_side=side)
+        b.add_scene(s)
+    b.update(DT, 2)
+    b.sync()
+    return b
+
+
+@pytest.mark.parametrize("change", [{}, {"steps_per_launch": 4}, {"use_graph": 0}])
+def test_other_settings_keep_the_default_shapes(change):
+    # four scenes leave the device idle: they run wider than the configuration
+    # says, also after a setting that is no shape, or none at all, was written back
+    b = small_batch((2, 19, 33, 47))
+    before, cfg = b.shapes(), b.config
+    assert before[1][0] > cfg["wg_small"]
+    b.config = change
+    assert b.config == {**cfg, **change} and b.shapes() == before
+    b.config = {"wg_small": 256}
+    assert [w for w, _ in b.shapes()] == [cfg["wg_tiny"], 256, cfg["wg_large"]]
+    b.config = {"wg_small": cfg["wg_small"]}  # asked for by now
+    assert [w for w, _ in b.shapes()] == [cfg["wg_tiny"], cfg["wg_small"], cfg["wg_large"]]
+
+
+def test_autotune_tries_the_default_shapes():
+    # its first trial is what the batch ran on, so a tuned batch takes no longer than
+    # an untuned one (1.36 times as long when it was no candidate)
+    b, t = small_batch([40] * 48), small_batch([40] * 48)
+    assert t.autotune(DT, 2) > 0
+
+    def ms(x):
+        best = np.inf
+        for _ in range(8):
+            x.update(DT, 4)
+            x.sync()
+            best = min(best, x.last_timing()[0] / 4)
+        return best
+
+    assert ms(t) < 1.2 * ms(b)
