@@ -242,8 +242,9 @@ extern "C" __device__ float __ockl_wfred_add_f32(float);
 // that nobody drifted far, and is asked every substep of a body in flight: the
 // box takes four lane reductions (minima of the bounds and the negated bounds)
 // and one barrier (640 flying bodies: the sweep phase 2.1 times shorter than
-// with nine values through LDS-routed shuffles).  The slots are free again by
-// the next call: barriers lie between.
+// with nine values through LDS-routed shuffles).  Barriers lie between two calls of
+// one form, after which its slots are free again; circle_sweep may ask with MEAN
+// right after quiet_sweep has asked without, so that one takes the worklists' space.
 struct Drift {
     float ux, uy, box;
 };
@@ -2078,9 +2079,9 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
 // far that there could be one.  This is every sweep of bodies in flight, so it
 // is asked before circle_sweep is called (a call saves and restores registers).
 template <int WG>
-__device__ __forceinline__ bool quiet_sweep(const float2 *P, uint32_t Np, uint32_t Nc, CCShared *sh) {
+__device__ __forceinline__ bool quiet_sweep(const float2 *P, uint32_t Np, uint32_t Nc, CCShared *sh, uint32_t *s_wl) {
     if (uni(sh->cs.list_valid) == 0u || uni(sh->cs.pairs) != 0u || uni(sh->fb_streak) != 0u) return false;
-    const Drift dr = drift_box<WG, false>(P, Np, Nc, sh->work.ref, sh->red4);
+    const Drift dr = drift_box<WG, false>(P, Np, Nc, sh->work.ref, (float4 *)s_wl);
     if (!(drift_share(dr.box, uni(sh->cs.smin)) <= kDriftRebuild)) return false;
     if (threadIdx.x == 0) sh->cs.since_build++;
     return true;
@@ -2431,7 +2432,7 @@ __device__ __forceinline__ void run_scene(const SceneDesc *__restrict__ dp, uint
                 const uint64_t t0 = wall_clock64();
                 if constexpr (SEQ)
                     fallback_sweep<WG>(P, Np, Nc, crad, uni_r, runi, d.rmax, d.T, w, s_cc);
-                else if (!quiet_sweep<WG>(P, Np, Nc, s_cc))
+                else if (!quiet_sweep<WG>(P, Np, Nc, s_cc, s_wl))
                     err = uni(circle_sweep<WG>(P, Np, Nc, crad, uni_r, runi, d.rmax, d.T, s_cc, s_red, s_u32, s_wl));
                 if (tid == 0) s_cc->cnt.t_sweep += wall_clock64() - t0;
             }

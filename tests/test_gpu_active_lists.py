@@ -120,3 +120,25 @@ def test_the_launches_do_not_change_the_schedule(n, speed):
     a, b = run(1), run(16)
     assert a[1]["redos"] > 0
     assert bits_equal(a[0], b[0]) and a[1] == b[1]
+
+
+@pytest.mark.parametrize("n", [2, 100, 200, 400, 900, 2500])
+def test_flight_that_outruns_its_lists(n):
+    # circles far from each other, without a candidate pair, fast enough to leave
+    # their skins every few sweeps: the sweep that has nothing to do and the one that
+    # builds a new list follow each other, in workgroups of every size
+    rng = np.random.default_rng(n)
+    k = np.arange(n)
+    c = np.zeros((n, 7), np.float32)
+    c[:, 0:2] = 6.0 * np.stack([k % 50, k // 50], 1) + rng.uniform(-1.0, 1.0, (n, 2))
+    c[:, 2:4] = c[:, 0:2] - 3.0 * rng.standard_normal((n, 2)) * (DT / 8)
+    c[:, 6] = 0.35
+    s = Solver()
+    s.gravity, s.bounds = (0.0, 0.0), ((-50.0, -50.0), (500.0, 500.0))
+    s.set_sub_steps(8)
+    s.add_circles(c)
+    o = to_oracle(s, 32, candidate_mode=True)
+    for _ in range(12):
+        s.update(DT)
+        assert o.update(DT) == 0
+    assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
