@@ -1177,22 +1177,20 @@ __global__ void __launch_bounds__(256) k_cg_verify(Buckets bk, const float4 *__r
         const uint32_t ni = __float_as_uint(p.w) & kIdxMaskG;
         // a record's own reach covers r + e of a circle within its margin, the
         // level's largest r + e that of an overrun
-        auto near_at = [&](float emax) {
-            return [=](const float4 &q) {
-                const float lim = (ai + fmaxf(q.z, emax)) * (1.0f + 0x1p-15f);
-                const float dx = p.x - q.x, dy = p.y - q.y;
-                return dx * dx + dy * dy < lim * lim;
-            };
+        auto near = [&](const float4 &q, float emax) {
+            const float lim = (ai + fmaxf(q.z, emax)) * (1.0f + 0x1p-15f);
+            const float dx = p.x - q.x, dy = p.y - q.y;
+            return dx * dx + dy * dy < lim * lim;
         };
         auto test = [&](uint32_t j, const float4 &q) {
             if (j == i) return;
             const float lim = (ai + (aux[j].x + exc[j])) * (1.0f + 0x1p-16f);
             const float dx = p.x - q.x, dy = p.y - q.y;
-            if (!(dx * dx + dy * dy < lim * lim)) return;
+            const float d2 = dx * dx + dy * dy, reach = p.z + q.z;
+            // within both reaches: listed (by this very test), and replayed in order
+            if (!(d2 < lim * lim) || d2 < reach * reach) return;
             const uint32_t nj = __float_as_uint(q.w) & kIdxMaskG;
-            const uint32_t ri = rank(i, nj);
-            if (ri < cnt[i] && (cand[off[i] + ri] & kIdxMaskG) == j) return;  // listed: replayed in order
-            const uint32_t rj = rank(j, ni);
+            const uint32_t ri = rank(i, nj), rj = rank(j, ni);
             const float2 pi = ri ? traj[off[i] + ri - 1u] : make_float2(p.x, p.y);
             const float2 pj = rj ? traj[off[j] + rj - 1u] : make_float2(q.x, q.y);
             const bool first = ni < nj;
@@ -1210,7 +1208,7 @@ __global__ void __launch_bounds__(256) k_cg_verify(Buckets bk, const float4 *__r
             const double R = reach_at(L), ih = g->inv_h[L];
             const int64_t nx = (int64_t)cell_coord_d((double)p.x + R, ih) - cell_coord_d((double)p.x - R, ih) + 1;
             const int64_t ny = (int64_t)cell_coord_d((double)p.y + R, ih) - cell_coord_d((double)p.y - R, ih) + 1;
-            if (nx * ny > kMaxScanCells) brute = true;
+            if (nx * ny > kMaxScanCells || nx * ny > (int64_t)bk.tmask) brute = true;
         }
         if (brute) {
             for (uint32_t j = lane; j < bk.nc; j += 64u) test(j, bk.rec[j]);
@@ -1219,15 +1217,40 @@ __global__ void __launch_bounds__(256) k_cg_verify(Buckets bk, const float4 *__r
         for (uint32_t m = mask; m; m &= m - 1u) {
             const uint32_t L = (uint32_t)__ffs(m) - 1u;
             const double R = reach_at(L), ih = g->inv_h[L];
-            const auto near = near_at(__uint_as_float(ctl[kCtlEmax + L]));
+            const float emax = __uint_as_float(ctl[kCtlEmax + L]);
             const int x0 = cell_coord_d((double)p.x - R, ih), x1 = cell_coord_d((double)p.x + R, ih);
             const int y0 = cell_coord_d((double)p.y - R, ih), y1 = cell_coord_d((double)p.y + R, ih);
-            // rows over the lanes, each cut into pieces of 4 cells
-            const uint32_t pieces = (uint32_t)(x1 - x0 + 4) >> 2, items = pieces * (uint32_t)(y1 - y0 + 1);
-            for (uint32_t c = lane; c < items; c += 64u) {
-                const int cx = x0 + (int)(c % pieces) * 4;
-                const int cy = y0 + (int)(c / pieces);
-                scan_rows(bk, L, cx, min(cx + 3, x1), cy, cy, 1, ih, near, test);
+            const uint32_t cells = (uint32_t)(x1 - x0) + 1u, T = bk.tmask + 1u;
+            // a lane looks up a row's run of records; the records of up to 64 rows are
+            // then spread over the lanes (a row, or a piece of one, to a lane left most
+            // of them idle where a few cells hold thousands of records)
+            for (int r0 = y0; r0 <= y1; r0 += 64) {
+                uint32_t s0 = 0, len = 0;
+                if (r0 + (int)lane <= y1) {
+                    const uint32_t at = bucket_of(bk.tmask, bk.stride, L, x0, r0 + (int)lane), e = at + cells;
+                    s0 = bk.start[at];
+                    const uint32_t s1 = bk.start[e > T ? e - T : e];
+                    len = e > T ? bk.nc - s0 + s1 : s1 - s0;
+                }
+                uint32_t end = len;
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t v = (uint32_t)__shfl_up((int)end, o);
+                    if ((int)lane >= o) end += v;
+                }
+                const uint32_t total = (uint32_t)__shfl((int)end, 63);
+                for (uint32_t t0 = 0; t0 < total; t0 += 64u) {
+                    const uint32_t t = min(t0 + lane, total - 1u);
+                    uint32_t row = 0;  // the rows that end at t or before
+                    for (uint32_t o = 32u; o > 0u; o >>= 1)
+                        if ((uint32_t)__shfl((int)end, (int)(row + o - 1u)) <= t) row += o;
+                    uint32_t s = (uint32_t)__shfl((int)s0, (int)row) + (t - (uint32_t)__shfl((int)(end - len), (int)row));
+                    if (s >= bk.nc) s -= bk.nc;
+                    const float4 q = bk.rec[s];
+                    if (t0 + lane >= total || !near(q, emax)) continue;
+                    if ((__float_as_uint(q.w) >> kLvlShift) != L || cell_coord(q.y, ih) != r0 + (int)row) continue;
+                    const int cx = cell_coord(q.x, ih);
+                    if (cx >= x0 && cx <= x1) test(s, q);
+                }
             }
         }
     }

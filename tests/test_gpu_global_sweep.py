@@ -128,3 +128,28 @@ def test_pairs_are_taken_by_circle_number(size, clump):
     a, b = state(s), state(o)
     assert np.signbit(b[2::4]).any() and not np.signbit(b[2::4]).all()
     assert bits_equal(a, b), first_diff(a, b)
+
+
+@pytest.mark.parametrize("n", [300, 1500, 4000])
+@pytest.mark.parametrize("big", [3.0, 15.0])
+def test_overruns_in_crowded_cells(n, big):
+    # a few large circles make the cells so large that many records share one; fast
+    # circles leave their margins, so their cells are searched for pairs that no list
+    # holds, in rows of far more records than lanes; the component is replayed in memory
+    rng = np.random.default_rng(n + int(big))
+    span = 1.6 * np.sqrt(n)
+    r = np.where(np.arange(n) % 300 == 7, big, rng.uniform(0.1, 0.4, n))
+    c = at(rng.uniform(0.0, span, (n, 2)).astype(np.float32), r)
+    speed = np.where(rng.uniform(size=n) < 0.2, 60.0, 1.0)[:, None]
+    c[:, 2:4] -= (speed * rng.standard_normal((n, 2)) * DT / 2).astype(np.float32)
+    s = Solver()
+    s.set_engine(BD_ENGINE_GLOBAL)
+    s.gravity, s.bounds = (0.0, 0.0), ((-9000.0, -9000.0), (18000.0, 18000.0))
+    s.set_sub_steps(2)
+    s.add_circles(c)
+    o = to_oracle(s, 32, candidate_mode=True)
+    for _ in range(4):
+        s.update(DT)
+        assert o.update(DT) == 0
+        assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
+    assert s.stats()["cc_redos"] > 0
