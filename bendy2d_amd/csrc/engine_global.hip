@@ -985,13 +985,26 @@ __global__ void __launch_bounds__(256) k_cg_lds(float2 *__restrict__ P, const fl
     }
 }
 
+// A circle of a component that is replayed in memory: all that a pair reads and
+// writes of it in half a cache line.  (Such a component's circles are met in no
+// order of memory: as nine arrays, 150,000 circles of which 1 % are 8 times as large
+// missed L2 530 million times in 16 sweeps of 124 ms; like this they take 86.)
+struct __align__(64) CompCircle {
+    float2 p, from;
+    float rad, exc;
+    uint32_t off, cnt, head, nxp, stamp;
+};
+
 // Components above kLdsMembers circles (or whose lists overflow LDS): one
 // workgroup each, taken from a queue,
-// with the round protocol.  head[c] counts c's processed partners and nxp[c]
-// is the next one (kNoneG when done; with kLater when its number is larger, c then
-// being the pair's first end), so (x, y) is ready exactly when
-// nxp[x] is y and nxp[y] is x.  Every round applies at least one pair, so the
+// with the round protocol.  head counts a circle's processed partners and nxp
+// is the next one (kNoneG when done; with kLater when its number is larger, the
+// circle then being the pair's first end), so (x, y) is ready exactly when
+// x's nxp is y and y's is x.  Every round applies at least one pair, so the
 // loop ends; a list left unfinished (a schedule that stalls) is reported.
+// comp: a record a circle, or null until a scene has such a component; its sweep
+// then changes nothing and runs again with them (a gas never does, and allocating
+// them for a clone of 262,144 circles took 0.3 ms of its 11).
 __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ P, const float4 *__restrict__ aux,
                                                       const float4 *__restrict__ rec, float *__restrict__ exc,
                                                       const uint32_t *__restrict__ cnt,
@@ -1001,82 +1014,82 @@ __global__ void __launch_bounds__(kCompWG) k_cg_comps(float2 *__restrict__ P, co
                                                       const uint32_t *__restrict__ cstart,
                                                       const uint32_t *__restrict__ members,
                                                       const uint32_t *__restrict__ queues, uint32_t nc,
-                                                      uint32_t *__restrict__ head, uint32_t *__restrict__ nxp,
-                                                      uint32_t *__restrict__ stamp, uint2 *__restrict__ wl,
+                                                      CompCircle *__restrict__ comp, uint2 *__restrict__ wl,
                                                       float2 *__restrict__ traj, uint32_t *__restrict__ ctl) {
     __shared__ uint32_t s_n[3], s_bad;
     const uint32_t tid = threadIdx.x;
     if (ctl[kCtlFull]) return;  // uniform
     const uint32_t nbig = ctl[kCtlQueue + kQueueBig];
+    if (nbig != 0u && !comp) {  // uniform
+        if (tid == 0u) ctl[kCtlFull] = 1u;
+        return;
+    }
     const uint32_t *const bigq = queues + (size_t)kQueueBig * nc;
     constexpr uint32_t kEntry = kIdxMaskG | kLater;
     // whether x is the next partner of its own next partner y
     auto mutual = [&](uint32_t x, uint32_t y) {
-        return y != kNoneG && nxp[y & kIdxMaskG] == (y & kLater ? x : x | kLater);
+        return y != kNoneG && comp[y & kIdxMaskG].nxp == (y & kLater ? x : x | kLater);
     };
     for (uint32_t q = blockIdx.x; q < nbig; q += gridDim.x) {  // uniform per workgroup
         const uint32_t r = bigq[q], base = cstart[r], n = csize[r];
         const uint32_t *M = members + base;
         uint2 *const W[2] = {wl + base, wl + nc + base};
         for (uint32_t k = tid; k < n; k += kCompWG) {
-            const uint32_t c = M[k];
-            head[c] = 0u;
-            nxp[c] = cnt[c] ? cand[off[c]] & kEntry : kNoneG;
-            stamp[c] = kNoneG;
+            const uint32_t c = M[k], m = cnt[c], o = off[c];
+            const float4 v = rec[c];
+            const float2 p = make_float2(v.x, v.y);
+            comp[c] = CompCircle{p, p, aux[c].x, 0.0f, o, m, 0u, m ? cand[o] & kEntry : kNoneG, kNoneG};
         }
         if (tid == 0) { s_n[0] = 0u; s_n[1] = 0u; s_n[2] = 0u; s_bad = 0u; }
         __syncthreads();
         for (uint32_t k = tid; k < n; k += kCompWG) {
-            const uint32_t c = M[k], y = nxp[c];
+            const uint32_t c = M[k], y = comp[c].nxp;
             if ((y & kLater) && mutual(c, y)) W[0][atomicAdd(&s_n[0], 1u)] = make_uint2(c, y & kIdxMaskG);
         }
         __syncthreads();
         uint32_t cur = s_n[0], rounds = 0;
         for (; cur > 0; rounds++) {
-            const uint32_t cb = rounds & 1u, nb = cb ^ 1u;
+            const uint32_t now = rounds & 1u, nb = now ^ 1u;
             for (uint32_t k = tid; k < cur; k += kCompWG) {
-                const uint2 pr = W[cb][k];
-                const uint32_t c = pr.x, o = pr.y;
-                float2 pi = P[c], pj = P[o];
-                const uint32_t hc = head[c], ho = head[o];
-                const uint32_t oc = off[c], oo = off[o];
-                const uint32_t xc = hc + 1u < cnt[c] ? cand[oc + hc + 1u] & kEntry : kNoneG;
-                const uint32_t xo = ho + 1u < cnt[o] ? cand[oo + ho + 1u] & kEntry : kNoneG;
+                const uint2 pr = W[now][k];
+                // (whole records: storing only what changed took 7 % longer)
+                CompCircle a = comp[pr.x], b = comp[pr.y];
+                const uint32_t ua = a.off + a.head++, ub = b.off + b.head++;
+                a.nxp = a.head < a.cnt ? cand[ua + 1u] & kEntry : kNoneG;
+                b.nxp = b.head < b.cnt ? cand[ub + 1u] & kEntry : kNoneG;
+                a.stamp = b.stamp = rounds;
                 float qi = 0.0f, qj = 0.0f;
-                if (solve_circle_pair(pi.x, pi.y, pj.x, pj.y, aux[c].x, aux[o].x, qi, qj)) {
-                    P[c] = pi;
-                    P[o] = pj;
-                    const float4 sc = rec[c], so = rec[o];
-                    exc[c] = excursion(exc[c], pi.x, pi.y, sc.x, sc.y);
-                    exc[o] = excursion(exc[o], pj.x, pj.y, so.x, so.y);
+                if (solve_circle_pair(a.p.x, a.p.y, b.p.x, b.p.y, a.rad, b.rad, qi, qj)) {
+                    a.exc = excursion(a.exc, a.p.x, a.p.y, a.from.x, a.from.y);
+                    b.exc = excursion(b.exc, b.p.x, b.p.y, b.from.x, b.from.y);
                 }
-                traj[oc + hc] = pi;
-                traj[oo + ho] = pj;
-                head[c] = hc + 1u;
-                head[o] = ho + 1u;
-                nxp[c] = xc;
-                nxp[o] = xo;
-                stamp[c] = rounds;
-                stamp[o] = rounds;
+                traj[ua] = a.p;
+                traj[ub] = b.p;
+                comp[pr.x] = a;
+                comp[pr.y] = b;
             }
             if (tid == 0) s_n[(rounds + 2u) % 3u] = 0u;  // read two barriers ago
             __syncthreads();
             // pairs completed by a moved head; when both ends moved this round
             // the first one adds the pair
             for (uint32_t k = tid; k < cur; k += kCompWG) {
-                const uint2 pr = W[cb][k];
+                const uint2 pr = W[now][k];
                 for (int e = 0; e < 2; e++) {
-                    const uint32_t x = e ? pr.y : pr.x, y = nxp[x], o = y & kIdxMaskG;
+                    const uint32_t x = e ? pr.y : pr.x, y = comp[x].nxp, o = y & kIdxMaskG;
                     const bool first = (y & kLater) != 0u;
-                    if (!mutual(x, y) || (stamp[o] == rounds && !first)) continue;
+                    if (!mutual(x, y) || (comp[o].stamp == rounds && !first)) continue;
                     W[nb][atomicAdd(&s_n[(rounds + 1u) % 3u], 1u)] = first ? make_uint2(x, o) : make_uint2(o, x);
                 }
             }
             __syncthreads();
             cur = s_n[(rounds + 1u) % 3u];
         }
-        for (uint32_t k = tid; k < n; k += kCompWG)
-            if (head[M[k]] != cnt[M[k]]) s_bad = 1u;
+        for (uint32_t k = tid; k < n; k += kCompWG) {
+            const uint32_t c = M[k];
+            P[c] = comp[c].p;
+            exc[c] = comp[c].exc;
+            if (comp[c].head != comp[c].cnt) s_bad = 1u;
+        }
         __syncthreads();
         if (tid == 0) {
             if (s_bad) atomicOr(&ctl[kCtlBad], 1u);
@@ -1529,8 +1542,8 @@ private:
                                ws_.csize, ws_.cstart, ws_.members, ws_.place, ws_.queues, nc, cg_traj_.p, ctl);
             hipLaunchKernelGGL(k_cg_comps, dim3(kCompGrid), dim3(kCompWG), 0, stream_, ws_.spos, ws_.aux, ws_.rec,
                                ws_.exc, ws_.cnt, ws_.off, cc_cand_.p, ws_.csize, ws_.cstart,
-                               ws_.members, ws_.queues, nc, ws_.head, ws_.nxp, ws_.stamp, ws_.wl,
-                               cg_traj_.p, ctl);
+                               ws_.members, ws_.queues, nc, cg_comp_.n >= nc ? cg_comp_.p : nullptr,
+                               ws_.wl, cg_traj_.p, ctl);
             hipLaunchKernelGGL(k_cg_check, dim3((nb + kCheckPer - 1) / kCheckPer), dim3(256), 0, stream_, ws_.exc,
                                ws_.aux, ws_.rec, ws_.spos, ws_.cnt, cg_need_.p, s0_, nc, pos_.p, Np_,
                                ws_.overq, ctl);
@@ -1550,11 +1563,15 @@ private:
             std::memcpy(&total, host_ctl_ + kCtlTotal, sizeof total);
             if (host_ctl_[kCtlFull]) {
                 // nothing was replayed: the same attempt again, with room
-                if (total + total / 4 > 0xffffffffull) {
-                    err = "too many candidate circle pairs";
-                    return BD_ERR_CAPACITY;
+                if (total > cand_cap_) {
+                    if (total + total / 4 > 0xffffffffull) {
+                        err = "too many candidate circle pairs";
+                        return BD_ERR_CAPACITY;
+                    }
+                    cand_cap_ = total + total / 4;
+                } else {
+                    BD_HIP(cg_comp_.alloc(nc));
                 }
-                cand_cap_ = total + total / 4;
                 attempt--;
                 continue;
             }
@@ -1615,8 +1632,7 @@ private:
     // The sweep's workspace, one allocation: 22 of them, and as many releases, took
     // 1.5 to 4 ms of a scene's life (a clone rolled out for 32 sweeps: 16 ms).
     struct Workspace {
-        uint32_t *zero[2], *start, *cnt, *off, *par, *root, *place, *csize, *cstart, *members, *queues, *overq, *head, *nxp,
-            *stamp;
+        uint32_t *zero[2], *start, *cnt, *off, *par, *root, *place, *csize, *cstart, *members, *queues, *overq;
         float *exc;
         float2 *spos;
         float4 *rec, *aux;
@@ -1639,7 +1655,7 @@ private:
             take(ws_.spos, nc); take(ws_.exc, nc); take(ws_.cnt, nc); take(ws_.off, nc);
             take(ws_.par, nc); take(ws_.root, nc); take(ws_.place, nc); take(ws_.csize, nc);
             take(ws_.cstart, nc); take(ws_.members, nc); take(ws_.queues, kQueues * (size_t)nc);
-            take(ws_.overq, nc); take(ws_.head, nc); take(ws_.nxp, nc); take(ws_.stamp, nc);
+            take(ws_.overq, nc);
             take(ws_.wl, 2 * (size_t)nc);
         };
         all();
@@ -1675,6 +1691,7 @@ private:
     DevBuf<uint8_t> cg_arena_;
     Workspace ws_;
     DevBuf<uint32_t> cc_cand_;
+    DevBuf<CompCircle> cg_comp_;  // (from the first component that is replayed in memory on)
     DevBuf<float2> cg_traj_;
     // by slot of the last sweep: the circles (by number after an upload), their needs
     DevBuf<uint32_t> cg_order_;
