@@ -536,13 +536,44 @@ __global__ void __launch_bounds__(256) k_cg_cand(Buckets bk, const CGrid *__rest
         keys[s_o[st] + k] = key;
     });
     __syncthreads();
-    // lists from a second scan: a wavefront each, a key to a lane at a time, ranked
-    // against all keys (loads of one address for all lanes that wait for nothing,
-    // where a lane's own sort in memory was a chain of them; with 16 instead of 8
-    // entries kept in LDS, which spares most lists the second scan, this kernel
-    // took 20.0 us instead of 34.9 with 20,011 circles and 34.0 instead of 51.6
-    // with 262,144)
+    // lists from a second scan: a wavefront each, U keys to a lane at a time, ranked
+    // by number against all keys, 64 of them in a register that every lane's
+    // comparison reads a lane of (a lane's own sort in memory was a chain of loads;
+    // with 16 instead of 8 entries kept in LDS, which spares most lists the second
+    // scan, this kernel took 20.0 us instead of 34.9 with 20,011 circles and 34.0
+    // instead of 51.6 with 262,144).  The comparisons grow with the square of the
+    // length: with 20,000 lists of 2,000 entries and one of 20,000 the scans and sorts
+    // took 104 ms with a heap sort in a lane, 236 with a load for each key and list,
+    // 113 like this; what the pairs of longer lists take grows as fast and is more.
     const uint32_t number = __float_as_uint(r.w) & kIdxMaskG;
+    auto rank_list = [&](const uint64_t *k, uint32_t *to, uint32_t ln, uint32_t li, uint32_t least, auto per) {
+        constexpr uint32_t U = decltype(per)::value;
+        for (uint32_t x0 = 0; x0 < ln; x0 += 64u * U) {
+            uint64_t key[U];
+            uint32_t rank[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                key[u] = k[min(x0 + 64u * u + lane, ln - 1u)];
+                rank[u] = 0u;
+            }
+            for (uint32_t y0 = 0; y0 < ln; y0 += 64u) {
+                const uint32_t m = min(ln - y0, 64u);
+                const uint32_t theirs = lane < m ? (uint32_t)(k[y0 + lane] >> 32) : kNoneG;
+                for (uint32_t y = 0; y < m; y += 8u)
+#pragma unroll
+                    for (uint32_t v = 0; v < 8u; v++) {
+                        const uint32_t one = __builtin_amdgcn_readlane(theirs, y + v);
+#pragma unroll
+                        for (uint32_t u = 0; u < U; u++) rank[u] += one < (uint32_t)(key[u] >> 32) ? 1u : 0u;
+                    }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++)
+                if (x0 + 64u * u + lane < ln)
+                    to[rank[u]] = (uint32_t)key[u] | ((uint32_t)(key[u] >> 32) > li ? kLater : 0u) |
+                                  ((uint32_t)key[u] == least ? kParent : 0u);
+        }
+    };
     uint32_t low = s;
     for (uint64_t todo = __ballot(n > kSlotG); todo; todo &= todo - 1ull) {
         const int src = __ffsll((unsigned long long)todo) - 1;
@@ -552,14 +583,8 @@ __global__ void __launch_bounds__(256) k_cg_cand(Buckets bk, const CGrid *__rest
         uint32_t least = self;
         for (uint32_t x = lane; x < ln; x += 64u) least = min(least, (uint32_t)k[x]);
         for (int o = 32; o > 0; o >>= 1) least = min(least, (uint32_t)__shfl_xor((int)least, o));
-        for (uint32_t x = lane; x < ln; x += 64u) {
-            const uint64_t key = k[x];
-            uint32_t rank = 0;
-#pragma unroll 8
-            for (uint32_t y = 0; y < ln; y++) rank += k[y] < key ? 1u : 0u;
-            cand[lo0 + rank] = (uint32_t)key | ((uint32_t)(key >> 32) > li ? kLater : 0u) |
-                               ((uint32_t)key == least ? kParent : 0u);
-        }
+        if (ln <= 64u) rank_list(k, cand + lo0, ln, li, least, std::integral_constant<uint32_t, 1>{});
+        else rank_list(k, cand + lo0, ln, li, least, std::integral_constant<uint32_t, 4>{});
         if ((int)lane == src) low = least;
     }
     if (s >= bk.nc) return;

@@ -130,6 +130,17 @@ def test_pairs_are_taken_by_circle_number(size, clump):
     assert bits_equal(a, b), first_diff(a, b)
 
 
+@pytest.mark.parametrize("n", [17, 18, 64, 65, 66, 72, 73, 256, 257, 258, 700])
+def test_ranked_lists(n):
+    # clumps with lists of n - 1 entries, numbered in no order of place: the first
+    # lengths that are not kept (above 16), those ranked by one key or four to a lane
+    # (64), by blocks of 8 and 64 keys, and in more than one go (256)
+    rng = np.random.default_rng(200 + n)
+    clumps = max(2, 150 // n)
+    xy = rng.uniform(-0.2, 0.2, (clumps, n, 2)) + np.array([(9.0 * k, 4.0 * (k % 2)) for k in range(clumps)])[:, None]
+    check(at(xy.reshape(-1, 2)[rng.permutation(clumps * n)].astype(np.float32), 1.0), 2, 9000.0)
+
+
 @pytest.mark.parametrize("n", [300, 1500, 4000])
 @pytest.mark.parametrize("big", [3.0, 15.0])
 def test_overruns_in_crowded_cells(n, big):
