@@ -147,11 +147,14 @@ struct PinnedBuf {
 // Page-locked buffers that downloads borrow: allocating one takes longer than the
 // download of a small scene.  At most kKept buffers of together kKeptBytes wait
 // here for the next download; all solvers of the process share them, and they are
-// freed with the last solver.
+// freed with the last solver.  A state of more than kKeptBytes gets none: page-locking
+// a buffer that is not kept takes longer than a copy into pageable memory (6 and 12
+// million bodies: 40 and 78 ms a download, 27 and 54 pageable).  The first download
+// pays for its buffer (a million bodies 6.8 ms, then 0.9; pageable 1.7 each time).
 struct PinnedPool {
     static constexpr int kKept = 4;
     static constexpr size_t kKeptBytes = 64u << 20, kLeast = 64u << 10;
-    // a buffer of at least `bytes` (p null when there is no memory)
+    // a buffer of at least `bytes` (p null when there is no memory, or not so much is kept)
     PinnedBuf take(size_t bytes);
     void give(PinnedBuf &&b);
     static std::shared_ptr<PinnedPool> shared();

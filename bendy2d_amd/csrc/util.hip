@@ -67,12 +67,23 @@ int Engine::download(HostScene &s, PinnedPool &pool, std::string &err) {
         pool.give(std::move(host));
         return rc;
     }
-    // no page-locked memory left
+    // more than the pool holds, or no page-locked memory left: into pageable memory,
+    // a part at a time where none is read by index
     DevBuf<float2> dev;
     std::vector<float2> plain(std::max<size_t>(words, 1));
-    BD_HIP(dev.alloc(plain.size()));
-    BD_HIP(gather_state(parts, dev.p, stream()));
-    BD_HIP(hipMemcpyAsync(plain.data(), dev.p, words * sizeof(float2), hipMemcpyDeviceToHost, stream()));
+    bool by_index = false;
+    for (const StateParts::Part &p : parts.part) by_index |= p.index != nullptr;
+    if (by_index) {
+        BD_HIP(dev.alloc(plain.size()));
+        BD_HIP(gather_state(parts, dev.p, stream()));
+        BD_HIP(hipMemcpyAsync(plain.data(), dev.p, words * sizeof(float2), hipMemcpyDeviceToHost, stream()));
+    } else {
+        float2 *to = plain.data();
+        for (const StateParts::Part &p : parts.part) {
+            if (p.words) BD_HIP(hipMemcpyAsync(to, p.src, p.words * sizeof(float2), hipMemcpyDeviceToHost, stream()));
+            to += p.words;
+        }
+    }
     BD_HIP(hipStreamSynchronize(stream()));
     return unpack(plain.data(), s, err);
 }
@@ -95,9 +106,10 @@ PinnedBuf PinnedPool::take(size_t bytes) {
             if (kept_[k].p && kept_[k].n >= bytes && (best < 0 || kept_[k].n < kept_[best].n)) best = k;
         if (best >= 0) b = std::move(kept_[best]);
     }
-    if (!b.p) {
-        // a half more, so that a growing scene does not ask anew each time
-        hipError_t e = b.alloc(std::max(kLeast, bytes + bytes / 2));
+    if (!b.p && bytes <= kKeptBytes) {
+        // a half more, so that a growing scene does not ask anew each time, as long
+        // as the buffer can be kept
+        hipError_t e = b.alloc(std::max(kLeast, std::min(bytes + bytes / 2, kKeptBytes)));
         if (e != hipSuccess) e = b.alloc(std::max<size_t>(bytes, 16));
         if (e != hipSuccess) (void)hipGetLastError();
     }

@@ -41,6 +41,28 @@ def test_sizes(n, engine):
     assert s.engine_used == engine
 
 
+# 64 MiB of state, the most that goes through page-locked memory, and more, whole
+# arrays or read by index
+@pytest.mark.parametrize("n,engine", [(4194304, BD_ENGINE_GLOBAL), (4194305, BD_ENGINE_GLOBAL),
+                                      (4194305, BD_ENGINE_TILED)])
+def test_large_sizes(n, engine):
+    s = Solver()
+    s.set_engine(engine)
+    s.gravity, s.bounds = (0.0, -9.81), ((-1e6, -1e6), (2e6, 2e6))
+    i = np.arange(n)
+    p = np.stack([i % 2048, i // 2048], -1).astype(np.float32)
+    s.add_particles(p, p - np.float32(0.25))
+    a = np.arange(0, 2000, 2, dtype=np.uint32)
+    s.add_particle_links(a, a + 1, np.full(len(a), 0.75, np.float32))
+    o = to_oracle(s, 32)
+    for _ in range(2):
+        s.update(1.0 / 60.0)
+        assert o.update(1.0 / 60.0) == 0
+        x, w = s.get_particles()[:, :4], o.get_particles()[:, :4]
+        assert bits_equal(x, w), first_diff(x.ravel(), np.asarray(w).ravel())
+    assert s.engine_used == engine
+
+
 def test_parameters_change_between_updates():
     s = Solver()
     workloads.cloth_pinned(s, n=12, sub_steps=2, link_iters=2)
