@@ -219,6 +219,7 @@ struct CCShared {
         float s_cell, smin;
         uint32_t level;   // of the active margins' base (see kActiveBase)
         uint32_t clean;   // sweeps since a margin was too small
+        uint32_t heat;    // second runs of late (see kHeatMiss)
     } cs;
     // statistics of the scene during a launch, written by lane 0 only (in LDS
     // rather than in every lane's registers)
@@ -1190,20 +1191,27 @@ __device__ __forceinline__ void fallback_sweep(float2 *P, uint32_t Np, uint32_t 
 // Returns the slots used; with more than cap of them nothing past cap is
 // written, and the caller chooses another place.
 // The base margin, in units of the largest radius, at level 0; each level
-// doubles it.  A sweep that had to run again because a pair touched beyond the
-// margins raises the scene's level by two, kLevelClean sweeps without one lower it: a
+// doubles it.  A sweep that had to run again because a circle within its skin met a
+// pair beyond its margin raises the scene's level by two, kLevelClean sweeps without
+// one lower it: a
 // settling pile stays at level 0 (its rounds grow with the margins), a hot gas,
 // whose first contacts push circles by most of a radius, at the top (its rounds
-// are few: 16,000 circles ran every sweep twice at level 0).  Level and count are
+// are few: 16,000 circles ran every sweep twice at level 0).  Circles beyond their
+// skins meet such pairs too, a few in a pile that is being hit, where a second run of
+// the sweep costs less than the level, but every third sweep in a gas that falls into
+// a heap: they raise it once the second runs come closer together than the sweeps
+// that heat takes to cool (16,000 circles falling, 320 sweeps: 111 second runs and
+// 4.02 ms an update without, 12 and 3.56 with).  All of it is
 // kept between launches: counted anew in each, a launch of fewer than kLevelClean
 // sweeps could only raise the level (4,096 soft bodies piled up, 8 sweeps a launch:
-// 6.0e6 rounds and 26.2 ms an update, 3.4e6 and 23.1 with the count kept).  A level
+// 6.0e6 rounds and 26.2 ms an update, 3.5e6 and 23.6 with the count kept).  A level
 // given up too soon costs a second run of the sweep, one kept too long longer rounds
 // (those bodies, and a dozen batches of piles from their first contact on: 16 sweeps
 // 23.4 ms and 16.8 on average, 32 23.1 and 16.3, 64 23.8 and 16.7).
 constexpr float kActiveBase = 0.05f;
 constexpr uint32_t kLevels = 4u, kLevelClean = 32u;
-static_assert(kLevels < 128u && kLevelClean <= 128u, "kept between launches in 7 bits each");
+constexpr uint32_t kHeatMiss = 7u, kHeatRaise = 13u;  // one off a clean sweep
+static_assert(kLevels < 8u && kLevelClean <= 128u && kHeatRaise <= 16u, "kept between launches in 3, 7 and 4 bits");
 constexpr uint32_t kCurMask = 0x00ffffffu;
 constexpr uint32_t kStamp8 = 0xffu;
 static_assert(kCandCap * 65536ull <= kCurMask + 1ull, "a list cursor must fit 24 bits");
@@ -1867,7 +1875,7 @@ __device__ __noinline__ uint32_t build_lists(const float2 *P, uint32_t Np_, uint
     else if (since_build > 32) sbase = fmaxf(0.8f * sbase, 0.05f * fmaxf(rmax, 1e-3f));
     const uint64_t tb3 = wall_clock64();
     if (tid == 0) {
-        sh->cs = CCShared::Steer{sbase, 1u, total / 2, 0u, s_cell, smin, sh->cs.level, sh->cs.clean};
+        sh->cs = CCShared::Steer{sbase, 1u, total / 2, 0u, s_cell, smin, sh->cs.level, sh->cs.clean, sh->cs.heat};
         sh->cnt.n_out = n_out;
         sh->cnt.n_far = n_far;
         sh->cnt.smax = smax;
@@ -2049,9 +2057,12 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
             if (tid == 0) {
                 cs.since_build++;
                 if (n_over) sh->cnt.kept++;
-                if (widen == 0u && ++cs.clean >= kLevelClean) {
-                    cs.clean = 0u;
-                    if (cs.level) cs.level--;
+                if (widen == 0u) {
+                    if (cs.heat) cs.heat--;
+                    if (++cs.clean >= kLevelClean) {
+                        cs.clean = 0u;
+                        if (cs.level) cs.level--;
+                    }
                 }
             }
             return 0u;
@@ -2064,8 +2075,9 @@ __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t 
         if (tid == 0) {
             sh->cnt.redos++;
             if (!same_list) cs.list_valid = 0u;
-            if (missed_near) {
-                cs.clean = 0u;
+            if (check == 1 && !missed_near && widen == 0u) cs.heat += kHeatMiss;
+            if (missed_near || cs.heat >= kHeatRaise) {
+                cs.clean = cs.heat = 0u;
                 if (widen == 0u) cs.level = min(cs.level + 2u, kLevels);
             }
         }
@@ -2383,7 +2395,8 @@ __device__ __forceinline__ void run_scene(const SceneDesc *__restrict__ dp, uint
     uint32_t err = uni(st->err);
     if (tid == 0) {
         s_cc->cs = CCShared::Steer{st->skin, (uint32_t)st->list_valid & 1u, st->pairs, st->since_build, st->s_cell, st->smin,
-                                   (uint32_t)st->list_valid >> 1, (uint32_t)st->ws_ready >> 1};
+                                   (uint32_t)st->list_valid >> 1 & 7u, (uint32_t)st->ws_ready >> 1,
+                                   (uint32_t)st->list_valid >> 4};
         s_cc->fb_streak = 0u;
         CCShared::Counts &k = s_cc->cnt;
         k = CCShared::Counts{};
@@ -2481,7 +2494,7 @@ __device__ __forceinline__ void run_scene(const SceneDesc *__restrict__ dp, uint
     if (tid == 0) {
         const CCShared::Steer &cs = s_cc->cs;
         st->skin = cs.skin;
-        st->list_valid = (uint8_t)((cs.list_valid ? 1u : 0u) | (cs.level << 1));
+        st->list_valid = (uint8_t)((cs.list_valid ? 1u : 0u) | cs.level << 1 | cs.heat << 4);
         st->err = err;
         const CCShared::Counts &k = s_cc->cnt;
         st->rounds += k.rounds;

@@ -66,8 +66,8 @@ constexpr uint32_t kFlagSequential = 16u; // every circle-pair sweep by the sequ
 // Per-scene state that persists between launches (written by the kernel).
 struct SceneState {
     float skin;          // base candidate margin of the circle-pair schedule
-    uint8_t list_valid;  // bit 0: candidate list built and still usable; above: level of the
-                         // active margins
+    uint8_t list_valid;  // bit 0: candidate list built and still usable; bits 1-3: level of the
+                         // active margins; above: second runs of late
     uint8_t ws_ready;    // bit 0: per-circle skin state initialised; above: sweeps since a margin
                          // was too small
     uint16_t sub_phase;  // substeps of the current update already run (a launch's time budget

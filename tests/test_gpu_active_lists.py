@@ -142,3 +142,26 @@ def test_flight_that_outruns_its_lists(n):
         s.update(DT)
         assert o.update(DT) == 0
     assert bits_equal(state(s), state(o)), first_diff(state(s), state(o))
+
+
+@pytest.mark.parametrize("n", [1000, 4000])
+def test_few_sweeps_run_twice(n):
+    # a gas that falls into a heap, one update (4 sweeps) a launch: margins that are
+    # too small again and again grow, and sweeps seldom have to run a second time
+    rng = np.random.default_rng(n)
+    box = np.sqrt(n * np.pi * 0.25 / 0.5)
+    c = np.zeros((n, 7), np.float32)
+    c[:, 0:2] = rng.uniform(0.5, box - 0.5, (n, 2))
+    c[:, 2:4] = c[:, 0:2] - rng.standard_normal((n, 2)) * (DT / 4)
+    c[:, 6] = 0.5
+    s = Solver()
+    s.gravity, s.bounds = (0.0, -20.0), ((0.0, 0.0), (box, box))
+    s.set_sub_steps(4)
+    s.add_circles(c)
+    b = Batch()
+    b.add_scene(s)
+    for _ in range(60):
+        b.update(DT, 1)
+    b.sync()
+    st = b.scene_status(0)
+    assert st["err"] == 0 and st["redos"] <= 60 * 4 // 16
