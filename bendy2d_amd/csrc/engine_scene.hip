@@ -2633,11 +2633,17 @@ int scene_blocks_per_cu(int v, size_t lds_bytes) {
 // Launch shape of a single scene on an otherwise idle device: about two bodies
 // per lane; positions, previous positions and, when they fit, the link records
 // in LDS, with room behind them for the circle-pair rounds' state (8 bytes a
-// circle) and active lists (2 bytes an entry, room for four a circle).
-void scene_launch_shape(const SceneDesc &d, uint32_t &wg, uint32_t &lds) {
+// circle) and active lists (2 bytes an entry).  In a batch, where LDS decides how
+// many scenes run at once, that is room for four entries a circle; a scene with
+// the device to itself takes room for kAloneEntries: lists that do not fit are written
+// a second time, into memory, and the rounds read them there (a gas of 2,000 circles
+// that falls into a heap 702 us an update with room for four, 645 with sixteen; one
+// of 1,000 with mixed radii 634 and 585).
+void scene_launch_shape(const SceneDesc &d, uint32_t &wg, uint32_t &lds, uint32_t entries) {
     wg = 64;
     while (wg < 1024 && wg * 2 < d.N) wg <<= 1;
-    const uint64_t bodies = 16ull * d.N, links = 8ull * d.L, rounds = d.Nc >= 2 ? 16ull * d.Nc : 0ull;
+    const uint64_t bodies = 16ull * d.N, links = 8ull * d.L;
+    const uint64_t rounds = d.Nc >= 2 ? (8ull + 2ull * entries) * d.Nc : 0ull;
     const uint64_t want = bodies + links <= kMaxDynLds ? bodies + links + rounds : bodies + rounds;
     lds = (uint32_t)std::min<uint64_t>(want, kMaxDynLds);
 }
@@ -2834,7 +2840,7 @@ public:
         st.skin = img.skin0;
         BD_HIP(hipMemcpyAsync(state_ptr(), &st, sizeof(st), hipMemcpyHostToDevice, stream_));
         uint32_t wg;
-        scene_launch_shape(desc_, wg, lds_bytes_);
+        scene_launch_shape(desc_, wg, lds_bytes_, kAloneEntries);
         variant_ = variant_for_wg((int)wg);
         BD_HIP(hipStreamSynchronize(stream_));
         N_ = p.N; Np_ = p.Np; Nc_ = p.Nc; P_ = desc_.P;

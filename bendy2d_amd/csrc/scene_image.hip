@@ -198,7 +198,7 @@ int32_t bd_scene_image_describe(const bd_solver *s, bd_scene_image_info *info) {
     info->workspace_bytes = img.desc.Nc >= 2 ? img.desc.ws_bytes : 0u;
     info->n_bodies = img.desc.N;
     info->n_circles = img.desc.Nc;
-    scene_launch_shape(img.desc, info->workgroup, info->lds_bytes);
+    scene_launch_shape(img.desc, info->workgroup, info->lds_bytes, kAloneEntries);
     return BD_OK;
 }
 

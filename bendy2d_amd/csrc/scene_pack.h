@@ -49,7 +49,8 @@ void set_scene_params(SceneDesc &d, const StepParams &sp, uint32_t steps, bool a
 int scene_variant_count();
 int scene_variant_wg(int v);
 int variant_for_wg(int wg);
-void scene_launch_shape(const SceneDesc &d, uint32_t &wg, uint32_t &lds);
+constexpr uint32_t kAloneEntries = 16u;  // active list entries a circle
+void scene_launch_shape(const SceneDesc &d, uint32_t &wg, uint32_t &lds, uint32_t entries = 4u);
 size_t scene_max_lds();
 // steps: updates each scene runs in this launch (at most its desc.steps).
 int launch_scene_variant(int v, uint32_t blocks, size_t lds_bytes, hipStream_t stream, const SceneDesc *d,
