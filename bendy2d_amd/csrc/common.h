@@ -127,18 +127,6 @@ BD_HD void solve_particle_link(float &ax, float &ay, float &bx, float &by, float
     }
 }
 
-// CircleLink::solve (src/link.rs:36-48) with ra*ra, rb*rb and
-// 1.0f / (ra*ra + rb*rb) computed once by the caller: the same f32 values, so
-// the same results as solve_circle_link.
-BD_HD void solve_circle_link_w(float &ax, float &ay, float &bx, float &by, float t, float ra2, float rb2,
-                               float scale) {
-    float dx = ax - bx, dy = ay - by, dist, nx, ny;
-    length_and_unit(dx, dy, dx * dx + dy * dy, dist, nx, ny);
-    float e = dist - t;
-    ax = ax - ((nx * e) * scale) * rb2; ay = ay - ((ny * e) * scale) * rb2;
-    bx = bx + ((nx * e) * scale) * ra2; by = by + ((ny * e) * scale) * ra2;
-}
-
 // CircleLink::solve (src/link.rs:36-48).
 BD_HD void solve_circle_link(float &ax, float &ay, float &bx, float &by, float t, float ra, float rb) {
     float dx = ax - bx, dy = ay - by, dist, nx, ny;

@@ -13,8 +13,8 @@
 //              a sweep whose circles left their margins is checked pair by pair
 //              at each skipped pair's turn and redone only if one met
 //   polygons   one workgroup replays the polygon-pair loop (src/solver.rs:178-187)
-//   per body   EXT4 static colliders (staged in LDS), bounds, Verlet, fused in
-//              one streaming kernel (src/solver.rs:155-165, 118-128)
+//   per body   EXT4 static colliders (records through the scalar cache), bounds,
+//              Verlet, fused in one streaming kernel (src/solver.rs:155-165, 118-128)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -159,7 +159,9 @@ __global__ void k_zero_acc0(float2 *acc0, uint32_t n) {
 // |save_i - save_j| < reach_i + reach_j.  A pair left out can only meet during
 // the sweep if e_i + e_j > m_i + m_j, e being each circle's largest distance
 // from save during the sweep (excursion), so the sweep stands when every
-// e_i <= 0.9 m_i; otherwise it is undone and run again with the larger needs.
+// e_i <= 0.9 m_i.  Otherwise the pairs that the overrunning circles left out are
+// checked at their turns (k_cg_verify), and only if one met is the sweep undone and
+// run again with the larger needs.
 //
 // Margins can differ by orders of magnitude (a jammed ring of circles around a
 // collider beside quiet gas), so the grid is hierarchical: circle i sits at
@@ -1507,8 +1509,9 @@ public:
 private:
     // Exact replay of the circle-pair sweep (see the circle-pair kernels): lists
     // from per-circle margins on the level grid, components, then the lane and
-    // workgroup replays.  A sweep in which some circle went further than 0.9 of
-    // its margin is undone and run again with the needs it showed.
+    // workgroup replays.  A sweep in which a circle that went further than 0.9 of
+    // its margin met a pair that was left out is undone and run again with the
+    // needs it showed.
     // With bodies, the per-body phase follows in the attempt that stands.
     int circles(Stats &st, std::string &err, const BodyParams *bodies) {
         const uint32_t nc = Nc_;

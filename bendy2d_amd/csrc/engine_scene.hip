@@ -1902,8 +1902,10 @@ __device__ __noinline__ uint32_t build_lists(const float2 *P, uint32_t Np_, uint
 // overruns_check look at every pair of theirs that was not run; only if one of
 // them touched is the sweep undone and rerun, first with wider active margins,
 // then with a new candidate list and larger skins for the circles that moved.
-// The list is rebuilt before a sweep when a circle drifted more than
-// kDriftRebuild of its skin since it was built.
+// The list is rebuilt before a sweep when more circles than kDriftedBase +
+// Nc / kDriftedShare (any, in scenes of fewer than kDriftedLeast) have drifted more
+// than kDriftRebuild of their skins since it was built, or one of those has come into
+// reach of a circle that it does not list.
 // Returns the new error state (0 = fine).
 template <int WG>
 __device__ __noinline__ uint32_t circle_sweep(float2 *P, uint32_t Np_, uint32_t Nc_, const float *crad, bool uni_r_,

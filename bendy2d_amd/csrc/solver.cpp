@@ -57,9 +57,10 @@ struct bd_solver {
     std::unique_ptr<Engine> eng;
     int32_t engine_pref = BD_ENGINE_AUTO;
     int32_t engine_used = 0;
-    // TILED shape: 2,048-point tiles, two workgroups of 1,024 per CU on the
-    // 1024x1024 cloth (measured fastest of 1,024..8,192 points x 256..1,024 lanes)
-    uint32_t tile_points = 0, tile_wg = 1024;  // (0: the engine chooses)
+    // TILED shape: the engine chooses the tile size (0) by the particle count, from
+    // 512 points to the 2,048 of the 1024x1024 cloth, on workgroups of 1,024
+    // (measured fastest there of 1,024..8,192 points x 256..1,024 lanes)
+    uint32_t tile_points = 0, tile_wg = 1024;
     hipStream_t stream = nullptr;
     std::shared_ptr<PinnedPool> pool = PinnedPool::shared();
     int device = -1;
