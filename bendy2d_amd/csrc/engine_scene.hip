@@ -1201,16 +1201,17 @@ __device__ __forceinline__ void fallback_sweep(float2 *P, uint32_t Np, uint32_t 
 // the sweep costs less than the level, but every third sweep in a gas that falls into
 // a heap: they raise it once the second runs come closer together than the sweeps
 // that heat takes to cool (16,000 circles falling, 320 sweeps: 111 second runs and
-// 4.02 ms an update without, 12 and 3.56 with).  All of it is
+// 4.02 ms an update without, 8 and 3.55 with).  All of it is
 // kept between launches: counted anew in each, a launch of fewer than kLevelClean
 // sweeps could only raise the level (4,096 soft bodies piled up, 8 sweeps a launch:
-// 6.0e6 rounds and 26.2 ms an update, 3.5e6 and 23.6 with the count kept).  A level
+// 6.0e6 rounds and 26.0 ms an update, 3.6e6 and 23.7 with the count kept).  A level
 // given up too soon costs a second run of the sweep, one kept too long longer rounds
-// (those bodies, and a dozen batches of piles from their first contact on: 16 sweeps
-// 23.4 ms and 16.8 on average, 32 23.1 and 16.3, 64 23.8 and 16.7).
+// (those bodies, and batches of 96 piles from their first contact, 8 updates each: 32
+// clean sweeps 23.6 and 15.10 ms, 48 24.0 and 15.06, 64 23.7 and 14.95; piles settling
+// for 30 updates 48.5, 48.8 and 49.3, 52.7 at a level that never falls).
 constexpr float kActiveBase = 0.05f;
-constexpr uint32_t kLevels = 4u, kLevelClean = 32u;
-constexpr uint32_t kHeatMiss = 7u, kHeatRaise = 13u;  // one off a clean sweep
+constexpr uint32_t kLevels = 4u, kLevelClean = 64u;
+constexpr uint32_t kHeatMiss = 5u, kHeatRaise = 13u;  // one off a clean sweep
 static_assert(kLevels < 8u && kLevelClean <= 128u && kHeatRaise <= 16u, "kept between launches in 3, 7 and 4 bits");
 constexpr uint32_t kCurMask = 0x00ffffffu;
 constexpr uint32_t kStamp8 = 0xffu;
